@@ -413,6 +413,34 @@ int ssm_decode_layers(int64_t batch, int64_t nlayers, int64_t model_dim, int64_t
 int ssm_decode_layers_status(void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * The decode step for larger batches, 1 <= batch <= 64 (the calls above take
+ * at most 8 rows): the projections as matrix-core products over all rows.
+ * ssm_decode_rows_linear computes what ssm_decode_gemv does, with the same
+ * arguments.  ssm_decode_rows_block is one whole layer's step, Block.step
+ * (modules/block.py:78-90) with norm_weight and residual set, Mamba.step
+ * (modules/mamba.py:189-243) without: out = W_out @ y (+ b_out) (+ x when
+ * residual), from the in-projection with the conv step, the x-projection, the
+ * state update and the out-projection, four launches.
+ *
+ * layer: a HOST array of SSM_LAYER_NPTR device pointers in the SSM_LAYER_*
+ * order (the biases, norm weight, dt_bias and D may be NULL); the projection
+ * weights, norm weight and state 16-byte aligned.  The conv window and the
+ * state advance in place.  x, out: (batch, model_dim), distinct.  model_dim
+ * and dim multiples of 16 bytes of elements; nstate in {4, 8, 16, 32, 64};
+ * rank >= 1; 2 <= width <= 8.  workspace: ssm_decode_rows_block_workspace
+ * bytes, 256-byte aligned, written before it is read.
+ */
+int ssm_decode_rows_linear(int64_t batch, int64_t out_dim, int64_t in_dim, int dtype,
+                           const void* weight, const void* x, const void* norm_weight,
+                           float norm_eps, const void* bias, const void* residual, void* y,
+                           void* stream);
+int64_t ssm_decode_rows_block_workspace(int64_t batch, int64_t dim, int64_t params_dim, int dtype);
+int ssm_decode_rows_block(int64_t batch, int64_t model_dim, int64_t dim, int64_t nstate,
+                          int64_t rank, int64_t width, int dtype, const void* const* layer,
+                          const void* x, void* out, float norm_eps, int residual, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
+/*
  * Greedy pick of the decode loop: token[b] = argmax_v probs[b, v] over the
  * softmax output (batch, vocab) -- the argmax of models/causal_lm.py:117-120,
  * the first maximum, NaN ranking above every number as in torch.argmax --

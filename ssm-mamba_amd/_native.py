@@ -115,6 +115,17 @@ SIGNATURES = {
         _p, _p, _p, ctypes.c_float,            # layer_table, x, out, norm_eps
         _p, _i64, _p,                          # workspace, workspace_bytes, stream
     ]),
+    "ssm_decode_rows_linear": (_i32, [
+        _i64, _i64, _i64, _i32,                # batch, out_dim, in_dim, dtype
+        _p, _p, _p, ctypes.c_float,            # weight, x, norm_weight, norm_eps
+        _p, _p, _p, _p,                        # bias, residual, y, stream
+    ]),
+    "ssm_decode_rows_block_workspace": (_i64, [_i64, _i64, _i64, _i32]),
+    "ssm_decode_rows_block": (_i32, [
+        _i64, _i64, _i64, _i64, _i64, _i64, _i32,  # batch, model_dim, dim, nstate, rank, width, dtype
+        _p, _p, _p, ctypes.c_float, _i32,      # layer (host array), x, out, norm_eps, residual
+        _p, _i64, _p,                          # workspace, workspace_bytes, stream
+    ]),
     "ssm_decode_layers_status": (_i32, [_p, _i64, _p]),
     "ssm_decode_pick_workspace": (_i64, [_i64]),
     "ssm_decode_pick": (_i32, [

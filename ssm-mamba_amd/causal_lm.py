@@ -361,6 +361,8 @@ class Mamba(nn.Module):
                                "or allocate_cache()")
         if _dec.block_step_supported(self, hidden_states, None):
             return _dec.block_step(self, hidden_states)
+        if _dec.rows_step_supported(self, hidden_states, None):
+            return _dec.rows_block_step(self, hidden_states)
         inner, rank, nstate = self.inner_dim, self.delta_rank, self.state_dim
         w_in, b_in = self.input_proj.weight, self.input_proj.bias
         xs = F.linear(hidden_states, w_in[:inner], None if b_in is None else b_in[:inner])
@@ -437,6 +439,11 @@ class Block(nn.Module):
             # norm, mixer and residual in the four fused decode kernels
             return _dec.block_step(self.ssm, hidden_states, self.norm.weight, self.norm.eps,
                                    residual=True)
+        if (_dec.plain(self.norm, RMSNorm)
+                and _dec.rows_step_supported(self.ssm, hidden_states, self.norm.weight)):
+            # the same for 9 to 64 rows, on the matrix cores
+            return _dec.rows_block_step(self.ssm, hidden_states, self.norm.weight, self.norm.eps,
+                                        residual=True)
         return hidden_states + self.ssm.step(self.norm(hidden_states))
 
 
@@ -531,6 +538,11 @@ class CausalLM(nn.Module):
         if _dec.gemv_supported(self.lm_head.weight, x, self.norm.weight):
             return _dec.gemv(self.lm_head.weight, x, norm_weight=self.norm.weight,
                              eps=self.norm.eps)
+        if (_dec.plain(self.lm_head, nn.Linear) and self.lm_head.bias is None
+                and _dec.plain(self.norm, RMSNorm)
+                and _dec.rows_supported(self.lm_head.weight, x, self.norm.weight)):
+            return _dec.rows_linear(self.lm_head.weight, x, norm_weight=self.norm.weight,
+                                    eps=self.norm.eps)
         return self.lm_head(self.norm(x))
 
     def step(self, input_ids: torch.Tensor) -> torch.Tensor:

@@ -53,6 +53,14 @@ int decode_layers_max_width();
 hipError_t launch_decode_layers(int bf16, const void* table, int nlayers, int B, int K, int dim,
                                 int width, int R, int nout, float eps, const void* x, void* out,
                                 void* ws, hipStream_t st);
+int decode_rows_max_batch();
+hipError_t launch_decode_rows_linear(int bf16, const void* W, const void* x, const void* nw,
+                                     float eps, const void* bias, const void* res, void* y, int B,
+                                     int O, int K, hipStream_t st);
+hipError_t launch_decode_rows_in_proj(int bf16, const void* W, const void* x, const void* nw,
+                                      float eps, const void* bias, void* xz, int B, int dim, int K,
+                                      int width, void* ctx, const void* cw, const void* cb, void* xc,
+                                      hipStream_t st);
 hipError_t launch_rms_norm_cm(int bf16, const void* x, const void* w, float eps, void* out, int B,
                               int C, int L, bool pair, hipStream_t st);
 hipError_t launch_causal_conv1d_fwd(int batch, int dim, int L, int K, int dtype_bf16,
@@ -772,6 +780,125 @@ int ssm_decode_layers(int64_t batch, int64_t nlayers, int64_t model_dim, int64_t
                 "decode_layers needs all %d workgroups resident at once, more than this device holds",
                 ssm::decode_layers_grid((int)batch, (int)model_dim, (int)dim));
   return hip_status(he, "decode_layers launch");
+}
+
+namespace {
+int check_decode_rows(int64_t batch, int dtype) {
+  if (dtype != SSM_F32 && dtype != SSM_BF16)
+    return fail(SSM_ERR_INVALID, "dtype must be SSM_F32 or SSM_BF16 (got %d)", dtype);
+  if (batch < 1 || batch > ssm::decode_rows_max_batch())
+    return fail(SSM_ERR_UNSUPPORTED, "decode_rows kernels take 1 <= batch <= %d (got %lld)",
+                ssm::decode_rows_max_batch(), (long long)batch);
+  return SSM_OK;
+}
+
+// workspace of ssm_decode_rows_block, in 256-byte aligned parts
+struct RowsWs {
+  size_t xz, xc, params, y, total;
+};
+RowsWs rows_ws(int64_t batch, int64_t dim, int64_t nout, int dtype) {
+  const size_t e = dtype == SSM_BF16 ? 2 : 4;
+  RowsWs w{};
+  size_t o = 0;
+  w.xz = o; o += round256((size_t)batch * 2 * dim * e);
+  w.xc = o; o += round256((size_t)batch * dim * e);
+  w.params = o; o += round256((size_t)batch * nout * e);
+  w.y = o; o += round256((size_t)batch * dim * e);
+  w.total = o;
+  return w;
+}
+}  // namespace
+
+int ssm_decode_rows_linear(int64_t batch, int64_t out_dim, int64_t in_dim, int dtype,
+                           const void* weight, const void* x, const void* norm_weight,
+                           float norm_eps, const void* bias, const void* residual, void* y,
+                           void* stream) {
+  g_err.clear();
+  if (int rc = check_decode_rows(batch, dtype)) return rc;
+  if (!weight || !x || !y) return fail(SSM_ERR_INVALID, "weight, x and y must be non-NULL");
+  const int e = elems16(dtype);
+  if (out_dim < 1 || in_dim < e || in_dim % e || out_dim > INT_MAX / 2 || in_dim > INT_MAX / 2)
+    return fail(SSM_ERR_UNSUPPORTED, "decode_rows_linear needs in_dim a positive multiple of %d (got %lld x %lld)",
+                e, (long long)out_dim, (long long)in_dim);
+  if (!aligned16(weight) || !aligned16(x) || !aligned16(norm_weight))
+    return fail(SSM_ERR_UNSUPPORTED, "decode_rows_linear needs 16-byte aligned weight, x and norm_weight");
+  return hip_status(ssm::launch_decode_rows_linear(dtype == SSM_BF16, weight, x, norm_weight,
+                                                   norm_eps, bias, residual, y, (int)batch,
+                                                   (int)out_dim, (int)in_dim,
+                                                   static_cast<hipStream_t>(stream)),
+                    "decode_rows_linear launch");
+}
+
+int64_t ssm_decode_rows_block_workspace(int64_t batch, int64_t dim, int64_t params_dim, int dtype) {
+  if (check_decode_rows(batch, dtype) != SSM_OK || dim < 1 || dim > INT_MAX / 4 || params_dim < 1 ||
+      params_dim > 16384)
+    return 0;
+  return (int64_t)rows_ws(batch, dim, params_dim, dtype).total;
+}
+
+int ssm_decode_rows_block(int64_t batch, int64_t model_dim, int64_t dim, int64_t nstate,
+                          int64_t rank, int64_t width, int dtype, const void* const* layer,
+                          const void* x, void* out, float norm_eps, int residual, void* workspace,
+                          int64_t workspace_bytes, void* stream) {
+  g_err.clear();
+  if (int rc = check_decode_rows(batch, dtype)) return rc;
+  if (!layer || !x || !out || !workspace)
+    return fail(SSM_ERR_INVALID, "layer, x, out and workspace must be non-NULL");
+  for (int i : {SSM_LAYER_IN_PROJ_W, SSM_LAYER_CONV_W, SSM_LAYER_X_PROJ_W, SSM_LAYER_DT_PROJ_W,
+                SSM_LAYER_LOG_A, SSM_LAYER_OUT_PROJ_W, SSM_LAYER_CONV_WINDOW, SSM_LAYER_STATE})
+    if (!layer[i]) return fail(SSM_ERR_INVALID, "layer pointer %d must be non-NULL", i);
+  const int e = elems16(dtype);
+  if (model_dim < e || model_dim % e || model_dim > INT_MAX / 4 || dim < e || dim % e ||
+      dim > INT_MAX / 4)
+    return fail(SSM_ERR_UNSUPPORTED, "decode_rows_block needs model_dim and dim positive multiples of %d", e);
+  if (!(nstate == 4 || nstate == 8 || nstate == 16 || nstate == 32 || nstate == 64))
+    return fail(SSM_ERR_UNSUPPORTED, "decode_rows_block supports nstate in {4, 8, 16, 32, 64} (got %lld)",
+                (long long)nstate);
+  const int64_t nout = rank + 2 * nstate;
+  if (rank < 1 || nout > 16384)
+    return fail(SSM_ERR_UNSUPPORTED, "decode_rows_block needs rank >= 1 and rank + 2 * nstate <= 16384");
+  if (width < 2 || width > ssm::conv1d_max_width())
+    return fail(SSM_ERR_UNSUPPORTED, "decode conv width must be in [2, %d] (got %lld)",
+                ssm::conv1d_max_width(), (long long)width);
+  for (int i : {SSM_LAYER_IN_PROJ_W, SSM_LAYER_NORM_W, SSM_LAYER_X_PROJ_W, SSM_LAYER_OUT_PROJ_W,
+                SSM_LAYER_STATE})
+    if (!aligned16(layer[i]))
+      return fail(SSM_ERR_UNSUPPORTED, "decode_rows_block needs layer pointer %d 16-byte aligned", i);
+  if (!aligned16(x) || (reinterpret_cast<uintptr_t>(workspace) & 255))
+    return fail(SSM_ERR_UNSUPPORTED, "decode_rows_block needs a 16-byte aligned x and a 256-byte aligned workspace");
+  const RowsWs ws = rows_ws(batch, dim, nout, dtype);
+  if (workspace_bytes < (int64_t)ws.total)
+    return fail(SSM_ERR_INVALID, "decode_rows_block workspace is %lld bytes, needs %lld",
+                (long long)workspace_bytes, (long long)ws.total);
+  char* base = static_cast<char*>(workspace);
+  void *xz = base + ws.xz, *xc = base + ws.xc, *params = base + ws.params, *y = base + ws.y;
+  const int bf16 = dtype == SSM_BF16;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (int rc = hip_status(ssm::launch_decode_rows_in_proj(
+                              bf16, layer[SSM_LAYER_IN_PROJ_W], x, layer[SSM_LAYER_NORM_W], norm_eps,
+                              layer[SSM_LAYER_IN_PROJ_B], xz, (int)batch, (int)dim, (int)model_dim,
+                              (int)width, const_cast<void*>(layer[SSM_LAYER_CONV_WINDOW]),
+                              layer[SSM_LAYER_CONV_W], layer[SSM_LAYER_CONV_B], xc, st),
+                          "decode_rows_block in-projection launch"))
+    return rc;
+  if (int rc = hip_status(ssm::launch_decode_rows_linear(bf16, layer[SSM_LAYER_X_PROJ_W], xc, nullptr,
+                                                         0.0f, nullptr, nullptr, params, (int)batch,
+                                                         (int)nout, (int)dim, st),
+                          "decode_rows_block x-projection launch"))
+    return rc;
+  const bool vecR = rank % e == 0 && rank <= 16 * e && aligned16(layer[SSM_LAYER_DT_PROJ_W]);
+  if (int rc = hip_status(ssm::launch_decode_ssm_step(
+                              bf16, params, (int)nout, 0, (int)rank, layer[SSM_LAYER_DT_PROJ_W],
+                              layer[SSM_LAYER_DT_BIAS], layer[SSM_LAYER_LOG_A], layer[SSM_LAYER_D], xc,
+                              xz, (int)(2 * dim),
+                              static_cast<float*>(const_cast<void*>(layer[SSM_LAYER_STATE])), y,
+                              (int)batch, (int)dim, (int)nstate, vecR, st),
+                          "decode_rows_block state update launch"))
+    return rc;
+  return hip_status(ssm::launch_decode_rows_linear(bf16, layer[SSM_LAYER_OUT_PROJ_W], y, nullptr, 0.0f,
+                                                   layer[SSM_LAYER_OUT_PROJ_B], residual ? x : nullptr,
+                                                   out, (int)batch, (int)model_dim, (int)dim, st),
+                    "decode_rows_block out-projection launch");
 }
 
 int64_t ssm_decode_pick_workspace(int64_t batch) {

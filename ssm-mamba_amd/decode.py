@@ -11,6 +11,7 @@ otherwise.
 """
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -18,7 +19,8 @@ import torch
 from . import _native as N
 
 _DTYPES = {torch.float32: N.SSM_F32, torch.bfloat16: N.SSM_BF16}
-MAX_BATCH = 8
+MAX_BATCH = 8        # rows of the GEMV kernels
+MAX_ROWS = 64        # rows of the matrix-core kernels (rows_linear, rows_block_step)
 _STATE_SIZES = (4, 8, 16, 32, 64)
 
 # The model harness takes the fused path whenever it qualifies; set False to
@@ -118,9 +120,20 @@ def ssm_step(params: torch.Tensor, rank: int, dt_proj_weight: torch.Tensor,
 
 
 def gemv_supported(weight: torch.Tensor, x: torch.Tensor, *others) -> bool:
+    return _linear_supported(1, MAX_BATCH, weight, x, *others)
+
+
+def rows_supported(weight: torch.Tensor, x: torch.Tensor, *others) -> bool:
+    """Whether ``rows_linear`` takes the product: the GEMV kernels' conditions,
+    for the batches past theirs (autocast keeps the op-by-op path and its
+    casts)."""
+    return not torch.is_autocast_enabled() and _linear_supported(MAX_BATCH + 1, MAX_ROWS, weight, x, *others)
+
+
+def _linear_supported(lo: int, hi: int, weight: torch.Tensor, x: torch.Tensor, *others) -> bool:
     if not ENABLED or torch.is_grad_enabled():
         return False
-    if not (x.is_cuda and x.dim() == 2 and x.dtype in _DTYPES and 1 <= x.shape[0] <= MAX_BATCH):
+    if not (x.is_cuda and x.dim() == 2 and x.dtype in _DTYPES and lo <= x.shape[0] <= hi):
         return False
     e = _elems16(x.dtype)
     k = x.shape[1]
@@ -134,6 +147,31 @@ def gemv_supported(weight: torch.Tensor, x: torch.Tensor, *others) -> bool:
 
 def block_step_supported(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tensor]) -> bool:
     """Whether the fused kernels can run Mamba ``ssm`` on the token batch x."""
+    return _step_supported(gemv_supported, ssm, x, norm_weight)
+
+
+def plain(module, cls) -> bool:
+    """Whether calling ``module`` is exactly ``cls.forward``: no subclass and no
+    hooks of its own, so a kernel may stand in for the call."""
+    return (type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks)
+
+
+def rows_step_supported(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tensor]) -> bool:
+    """Whether ``rows_block_step`` can run Mamba ``ssm`` on the token batch x:
+    block_step_supported's conditions, for the batches past its own, with a
+    projection shape the step's products take."""
+    if not _step_supported(rows_supported, ssm, x, norm_weight):
+        return False
+    nout = ssm.delta_rank + 2 * ssm.state_dim
+    return (tuple(ssm.input_proj.weight.shape) == (2 * ssm.inner_dim, x.shape[1])
+            and tuple(ssm.ssm_param_proj.weight.shape) == (nout, ssm.inner_dim)
+            and tuple(ssm.delta_proj.weight.shape) == (ssm.inner_dim, ssm.delta_rank)
+            and tuple(ssm.out_proj.weight.shape) == (x.shape[1], ssm.inner_dim)
+            and tuple(ssm.conv.weight.shape) == (ssm.inner_dim, 1, ssm.conv_kernel)
+            and tuple(ssm.log_A.shape) == (ssm.inner_dim, ssm.state_dim))
+
+
+def _step_supported(linear_supported, ssm, x, norm_weight) -> bool:
     if torch.is_grad_enabled():
         return False
     ctx, state = ssm._conv_context, ssm._ssm_hiddens
@@ -149,7 +187,7 @@ def block_step_supported(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tenso
     params = [ssm.input_proj.weight, ssm.input_proj.bias, ssm.conv.weight, ssm.conv.bias,
               ssm.ssm_param_proj.weight, ssm.delta_proj.weight, ssm.delta_proj.bias, ssm.log_A,
               ssm.D, ssm.out_proj.weight, ssm.out_proj.bias, norm_weight]
-    if not gemv_supported(ssm.input_proj.weight, x, *params):
+    if not linear_supported(ssm.input_proj.weight, x, *params):
         return False
     if tuple(ctx.shape) != (batch, inner, ssm.conv_kernel - 1) or ctx.dtype != x.dtype \
             or not ctx.is_contiguous():
@@ -178,6 +216,42 @@ def block_step(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tensor] = None,
     return gemv(ssm.out_proj.weight, y, bias=ssm.out_proj.bias, residual=x if residual else None)
 
 
+def rows_linear(weight: torch.Tensor, x: torch.Tensor, norm_weight: Optional[torch.Tensor] = None,
+                eps: float = 1e-6, bias: Optional[torch.Tensor] = None,
+                residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``gemv`` on the matrix cores, for up to MAX_ROWS rows."""
+    batch, k = x.shape
+    o = weight.shape[0]
+    y = torch.empty(batch, o, device=x.device, dtype=x.dtype)
+    with torch.cuda.device(x.device):
+        N.check(N.lib().ssm_decode_rows_linear(batch, o, k, _DTYPES[x.dtype], weight.data_ptr(),
+                                               x.data_ptr(), _ptr(norm_weight), float(eps),
+                                               _ptr(bias), _ptr(residual), y.data_ptr(),
+                                               _stream(x.device)))
+    return y
+
+
+def rows_block_step(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tensor] = None,
+                    eps: float = 1e-6, residual: bool = False) -> torch.Tensor:
+    """``block_step`` for up to MAX_ROWS rows: the four launches of one layer
+    in one library call."""
+    batch, model_dim = x.shape
+    dim, rank, nstate = ssm.inner_dim, ssm.delta_rank, ssm.state_dim
+    lib = N.lib()
+    out = torch.empty_like(x)
+    ws = torch.empty(lib.ssm_decode_rows_block_workspace(batch, dim, rank + 2 * nstate,
+                                                         _DTYPES[x.dtype]),
+                     dtype=torch.uint8, device=x.device)
+    tensors = _mixer_tensors(ssm, norm_weight)  # held until the launches are enqueued
+    ptrs = (ctypes.c_void_p * _LAYER_NPTR)(*(_ptr(t) for t in tensors))
+    with torch.cuda.device(x.device):
+        N.check(lib.ssm_decode_rows_block(batch, model_dim, dim, nstate, rank, ssm.conv_kernel,
+                                          _DTYPES[x.dtype], ctypes.cast(ptrs, ctypes.c_void_p),
+                                          x.data_ptr(), out.data_ptr(), float(eps), int(residual),
+                                          ws.data_ptr(), ws.numel(), _stream(x.device)))
+    return out
+
+
 # ---- the layer chain: every layer's step in one launch ------------------------
 
 _CHAIN_STATE = 16
@@ -185,10 +259,16 @@ _CHAIN_MAX_WIDTH = 4
 _CHAIN_MAX_BATCH = 4
 
 
+_LAYER_NPTR = 14
+
+
 def _layer_tensors(block):
     """The SSM_LAYER_* row of one Block, in the header's order."""
-    ssm = block.ssm
-    return [ssm.input_proj.weight, ssm.input_proj.bias, block.norm.weight, ssm.conv.weight,
+    return _mixer_tensors(block.ssm, block.norm.weight)
+
+
+def _mixer_tensors(ssm, norm_weight):
+    return [ssm.input_proj.weight, ssm.input_proj.bias, norm_weight, ssm.conv.weight,
             ssm.conv.bias, ssm.ssm_param_proj.weight, ssm.delta_proj.weight, ssm.delta_proj.bias,
             ssm.log_A, ssm.D, ssm.out_proj.weight, ssm.out_proj.bias, ssm._conv_context,
             ssm._ssm_hiddens]

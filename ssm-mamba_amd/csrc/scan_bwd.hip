@@ -671,9 +671,9 @@ __global__ __launch_bounds__(kThreads) void scan_bwd_kernel(
   }
 }
 
-// ---------------------------------------------------------------- backward, N <= 16
+// ---------------------------------------------------------------- backward, N <= 64
 
-// Role-split backward for up to 16 states, the counterpart of the forward's
+// Role-split backward for up to 64 states, the counterpart of the forward's
 // role split.  A workgroup of 12 waves covers one batch row b x 64 channels
 // and walks its segment's 16-step tiles from the end:
 //   consumer waves 0..7   lane = channel, wave w = states 2w and 2w+1: take
@@ -707,13 +707,24 @@ constexpr int kCacheNTb = 2;  // cache-policy bit NT (nontemporal) of a buffer a
 // whole-column accesses are permutations of 64 consecutive float4s.
 __device__ __forceinline__ constexpr int bws_swz(int q) { return 2 * q + 8 * (q & 1); }
 
-template <typename T>
+template <typename T, int kSG>
 struct BwsRows {  // one tile's raw loads of a producer lane, as loaded
   typename Raw4<T>::type u, d, dy, z, y;
-  uint32_t B, C;  // element bits
+  uint32_t B[kSG], C[kSG];  // element bits
 };
 
-template <typename T, bool kHasZ, bool kAligned>
+// kSG: state pairs of a consumer wave, for up to 16 kSG states (wave w: pairs
+// g * 8 + w, g < kSG, one after the other over a tile).  With more than one the
+// slices are single-buffered (two buffers would not fit beside the B/C of 64
+// states) behind a second barrier per tile, between the producers' finish of
+// the previous tile, which reads them, and the consumers' first write: the
+// consumers run the recompute of their first pair meanwhile.  A pair's A,
+// adjoint carry and dA then live in LDS between its turns and the pairs run
+// in a loop: held in registers over unrolled pairs, four of them spilled 155
+// registers at the 168 three waves a SIMD allow.  Measured against
+// scan_bwd_kernel at (4, 1024, 1000) x 64 states, bf16: 272 -> 197 us, its
+// segment summaries 102 -> 45 us; at (8, 2048, 512) x 32 states 206 -> 193 us.
+template <typename T, int kSG, bool kHasZ, bool kAligned>
 __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
     const ScanDims p, const T* __restrict__ u, const T* __restrict__ dl,
     const float* __restrict__ Ap, const T* __restrict__ Bp, const T* __restrict__ Cp,
@@ -731,9 +742,12 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
   static_assert(2 * 2 * kWsCons * kTileB == 2 * 64 * kWsProd, "two B/C elements per producer lane");
 
   __shared__ float4 sSt[2][3][kT4][kBlockCh];     // [parity][delta | delta*u | dout][column][row]
-  __shared__ float sBlk[2][kWsCons][kT4][16];     // [parity][pair][block][(step, state, B|C)]
-  __shared__ float4 sGB[2][kWsCons][kT4][kBlockCh];  // per-wave sum_n G B
-  __shared__ float4 sDD[2][kWsCons][kT4][kBlockCh];  // per-wave sum_n A G a h_{t-1}
+  constexpr int kSlices = kSG == 1 ? 2 : 1;  // slice buffers (by tile parity)
+  __shared__ float sBlk[2][kSG * kWsCons][kT4][16];  // [parity][pair][block][(step, state, B|C)]
+  __shared__ float4 sGB[kSlices][kWsCons][kT4][kBlockCh];  // per-wave sum_n G B
+  __shared__ float4 sDD[kSlices][kWsCons][kT4][kBlockCh];  // per-wave sum_n A G a h_{t-1}
+  // [wave][pair][state][A | carry | dA][lane] (kSG > 1)
+  __shared__ float sPair[kSG > 1 ? kWsCons : 1][kSG][2][3][kSG > 1 ? kBlockCh : 1];
 
   const int lane = threadIdx.x & 63;
   const int w = wave_id_uniform();
@@ -746,7 +760,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
   const int tile_beg = seg * (p.seg_len / kTileB);
   const int tile_end = min(ntiles_all, tile_beg + p.seg_len / kTileB);
   const int nt = tile_end - tile_beg;  // tiles of this segment, walked from the end
-  const int nbar = 1 + 4 * ((nt + 3) / 4);  // barriers of both roles
+  const int nbar = 1 + 4 * ((nt + 3) / 4);  // iterations of both roles (one barrier each, two with kSG > 1)
   const size_t srow = (size_t)seg * p.batch + b;
   const size_t rb = (size_t)b * Dm;
 
@@ -757,52 +771,81 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
     const int chc = min(ch, Dm - 1);
     const int Lp = bc_part_len(L);  // partial rows padded to whole tiles
     const size_t nBC = (size_t)p.batch * N * Lp;
-    float gam[2], dA[2], Av[2], A2[2];
+    float gam[kSG][2], dA[kSG][2], Av[kSG][2];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int n = 2 * w + s;
-      const bool ok = ch_ok && n < N;
-      dA[s] = 0.0f;
-      Av[s] = ok ? Ap[(size_t)ch * N + n] : 0.0f;
-      A2[s] = Av[s] * kLog2e;
-      // carry in from the later segments, last first:
-      // gamma <- gamma_seg + exp(A sum dt) gamma (their summaries, zero carry-in)
-      // (summary row k: sub-segment k + sub_k of seg_len / sub_k steps)
-      float q = (ok && dh_last) ? dh_last[(rb + ch) * N + n] : 0.0f;
-      if (ok)
-        q = fold_carry(q, A2[s], seg_dt, seg_g, (p.nseg - 1) * p.sub_k - 1, -1,
-                       (p.nseg - 1 - seg) * p.sub_k, p.batch, b, Dm, N, n, ch);
-      gam[s] = q;
+    for (int g = 0; g < kSG; ++g)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int n = 2 * (g * kWsCons + w) + s;
+        const bool ok = ch_ok && n < N;
+        dA[g][s] = 0.0f;
+        Av[g][s] = ok ? Ap[(size_t)ch * N + n] : 0.0f;
+        gam[g][s] = (ok && dh_last) ? dh_last[(rb + ch) * N + n] : 0.0f;
+      }
+    // carry in from the later segments, last first:
+    // gamma <- gamma_seg + exp(A sum dt) gamma (their summaries, zero carry-in)
+    // (summary row k: sub-segment k + sub_k of seg_len / sub_k steps)
+    {
+      float A2[kSG][2];
+#pragma unroll
+      for (int g = 0; g < kSG; ++g)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          A2[g][s] = Av[g][s] * kLog2e;
+          const int n = 2 * (g * kWsCons + w) + s;
+          if (kSG == 1 && ch_ok && n < N)
+            gam[g][s] = fold_carry(gam[g][s], A2[g][s], seg_dt, seg_g, (p.nseg - 1) * p.sub_k - 1, -1,
+                                   (p.nseg - 1 - seg) * p.sub_k, p.batch, b, Dm, N, n, ch);
+        }
+      if constexpr (kSG > 1)
+        fold_carry_pairs<kSG>(gam, A2, seg_dt, seg_g, (p.nseg - 1) * p.sub_k - 1, -1,
+                              (p.nseg - 1 - seg) * p.sub_k, p.batch, b, Dm, N, 2 * w, ch, ch_ok);
     }
     // The state the forward saved before tile t: h_init (or zero) before
     // tile 0, else through a buffer range over the batch row's saved rows
-    // (the launch keeps them below 2^31 bytes), the lane's state row as the
-    // vector offset and the tile as the scalar offset.
-    const int nc0 = min(2 * w, N - 1), nc1 = min(2 * w + 1, N - 1);
+    // (the launch keeps them below 2^31 bytes), the lane's channel as the
+    // vector offset, the state and the tile as the scalar offset.
     const size_t hrow = (size_t)N * p.hs * Dm;  // floats per saved slot
     const auto h_rsrc = raw_rsrc(const_cast<float*>(h_chunks) + (size_t)b * p.nchunks * hrow,
                                  (uint32_t)((size_t)p.nchunks * hrow * sizeof(float)));
+    const int nc0 = min(2 * w, N - 1), nc1 = min(2 * w + 1, N - 1);
     const uint32_t hv0 = (uint32_t)(((size_t)nc0 * p.hs * Dm + chc) * sizeof(float));
     const uint32_t hv1 = (uint32_t)(((size_t)nc1 * p.hs * Dm + chc) * sizeof(float));
-    const float hi0 = h_init ? h_init[(rb + chc) * N + nc0] : 0.0f;
-    const float hi1 = h_init ? h_init[(rb + chc) * N + nc1] : 0.0f;
-    // (the loads are unconditional, from slot 0 for tile 0, and the choice is
-    // made where the state is used: a load inside a branch is waited for at
-    // the branch's end)
+    const float hi0 = kSG == 1 && h_init ? h_init[(rb + chc) * N + nc0] : 0.0f;
+    const float hi1 = kSG == 1 && h_init ? h_init[(rb + chc) * N + nc1] : 0.0f;
+    const auto hi_rsrc =
+        raw_rsrc(kSG > 1 && h_init ? const_cast<float*>(h_init) + rb * N : const_cast<float*>(h_chunks),
+                 kSG > 1 && h_init ? (uint32_t)((size_t)Dm * N * sizeof(float)) : 0u);
+    // (the loads are unconditional and the choice of h_init is made where the
+    // state is used, or with kSG > 1 between descriptors and offsets: a load
+    // inside a branch is waited for at the branch's end)
     // (nontemporal loads: each saved state is read once, in whole 256-byte
     // runs, so it need not displace the input lines that serve several tiles)
-    auto saved_state = [&](int tile, float (&r)[2]) {
-      const int so = (int)((size_t)max(tile - 1, 0) * hrow * sizeof(float));
-      r[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(h_rsrc, (int)hv0, so, kCacheNTb));
-      r[1] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(h_rsrc, (int)hv1, so, kCacheNTb));
+    auto saved_state = [&](int tile, int g, float (&r)[2]) {
+      if constexpr (kSG == 1) {
+        const int so = (int)((size_t)max(tile - 1, 0) * hrow * sizeof(float));
+        r[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(h_rsrc, (int)hv0, so, kCacheNTb));
+        r[1] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(h_rsrc, (int)hv1, so, kCacheNTb));
+      } else {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int n = min(2 * (g * kWsCons + w) + s, N - 1);
+          const bool first = tile <= 0;
+          const int so = first ? n * 4
+                               : (int)(((size_t)(tile - 1) * hrow + (size_t)n * p.hs * Dm) * sizeof(float));
+          const int vo = first ? chc * N * 4 : chc * 4;
+          r[s] = __uint_as_float(
+              __builtin_amdgcn_raw_buffer_load_b32(first ? hi_rsrc : h_rsrc, vo, so, kCacheNTb));
+        }
+      }
     };
     float hcn[2];
-    saved_state(tile_end - 1, hcn);
+    saved_state(tile_end - 1, 0, hcn);
     // the value of lane l after the reduction of two blocks (block of the
     // pair, kind, state, step)
     const int vi = reduce32_index(lane);
     const int rsel = vi >> 4, rkind = (vi >> 3) & 1, rs = (vi >> 2) & 1, rj = vi & 3;
-    const int rn = 2 * w + rs;
+    const int rn = 2 * w + rs;  // of pair group 0; group g adds 16
     // the partials go through a buffer range over all of them (the launch
     // keeps them below 2^31 bytes): the lane's row and step as the vector
     // offset, the tile's first step as the scalar offset, the block as the
@@ -811,99 +854,162 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
     // (the offset of the pair's second block, jq - 1; the first block adds 16
     // bytes, 4 steps, so that no offset is negative)
     const uint32_t bc_off =
-        rn < N ? (uint32_t)((((size_t)rkind * p.nblk + blk) * nBC + ((size_t)b * N + rn) * Lp + rj) *
-                            sizeof(float)) + 16u * (1 - rsel)
-               : kOffDrop;
-    const bool hc_ok0 = ch_ok && 2 * w < N, hc_ok1 = ch_ok && 2 * w + 1 < N;
+        (uint32_t)((((size_t)rkind * p.nblk + blk) * nBC + ((size_t)b * N + rn) * Lp + rj) *
+                   sizeof(float)) + 16u * (1 - rsel);
 
-    // One iteration per barrier; the staging parity is a template constant
-    // (the loop runs iterations in pairs), so every LDS address is a
-    // per-lane base plus an immediate.
+    if constexpr (kSG > 1) {
+#pragma unroll
+      for (int g = 0; g < kSG; ++g)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          sPair[w][g][s][0][lane] = Av[g][s];
+          sPair[w][g][s][1][lane] = gam[g][s];
+          sPair[w][g][s][2][lane] = 0.0f;
+        }
+    }
+    // One iteration per tile.  With kSG == 1 the staging parity is a template
+    // constant (the loop runs iterations in pairs), so every LDS address is
+    // a per-lane base plus an immediate.
     auto iteration = [&](int i, auto parity) {
-      constexpr int buf = decltype(parity)::value;
+      const int buf = parity;
+      const int sl = kSG == 1 ? buf : 0;  // slice buffer
       __syncthreads();
-      if (i >= nt) return;
+      if (i >= nt) {
+        if constexpr (kSG > 1) __syncthreads();
+        return;
+      }
       const int tile = tile_end - 1 - i;
       const int t0 = tile * kTileB;
-      float hc[2];
-      hc[0] = tile > 0 ? (hc_ok0 ? hcn[0] : 0.0f) : hi0;
-      hc[1] = tile > 0 ? (hc_ok1 ? hcn[1] : 0.0f) : hi1;
-      saved_state(max(tile - 1, tile_beg), hcn);  // the next tile's (re-read at the last)
+      // the tile's work of pair g (first: pair 0, which starts the slices'
+      // sums; the others add to them)
+      auto pair = [&](const int g, auto first_tag) {
+        constexpr bool kFirst = decltype(first_tag)::value;
+        const int n0 = 2 * (g * kWsCons + w);
+        float hc[2] = {ch_ok && n0 < N ? hcn[0] : 0.0f, ch_ok && n0 + 1 < N ? hcn[1] : 0.0f};
+        if constexpr (kSG == 1) {
+          hc[0] = tile > 0 ? hc[0] : hi0;
+          hc[1] = tile > 0 ? hc[1] : hi1;
+        }
+        // the next pair's state, or the next tile's (re-read at the last)
+        if (g + 1 < kSG) saved_state(tile, g + 1, hcn);
+        else saved_state(max(tile - 1, tile_beg), 0, hcn);
+        float pA[2], pG[2], pD[2];  // the pair's A, carry and dA
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          pA[s] = kSG == 1 ? Av[0][s] : sPair[w][g][s][0][lane];
+          pG[s] = kSG == 1 ? gam[0][s] : sPair[w][g][s][1][lane];
+          pD[s] = kSG == 1 ? dA[0][s] : sPair[w][g][s][2][lane];
+        }
+        const float A2[2] = {pA[0] * kLog2e, pA[1] * kLog2e};
 
-      float a[2][kChunk], H[2][kChunk];
-      StepVals X, Y;
-      float bcg[kT4];  // block registers of the wave's pair: lane l holds value l & 15
+        float a[2][kChunk], H[2][kChunk];
+        StepVals X, Y;
+        float bcg[kT4];  // block registers of the pair: lane l holds value l & 15
 #pragma unroll
-      for (int jq = 0; jq < kT4; ++jq) bcg[jq] = sBlk[buf][w][jq][lane & 15];
-      auto put4 = [&](float4 (&slice)[kT4][kBlockCh], int q, const float (&v)[4]) {
-        slice[q][lane ^ bws_swz(q)] = make_float4(v[0], v[1], v[2], v[3]);
-      };
-      auto fwd = [&](int jq, const StepVals& sv) {
-        float y[4];  // unused here (the forward saved the output)
-        bwd_recompute_block(jq, sv, bcg[jq], A2, hc, a, H, y);
-      };
-      // the reverse of block jq; its 16 dB/dC terms go to vals[16 * half ..]
-      auto rev = [&](int jq, const StepVals& sv, float (&vals)[32], int half) {
-        float gB[4], gD[4], v16[16];
-        bwd_reverse_block(jq, sv, bcg[jq], Av, A2, hc, a, H, gam, dA, v16, gB, gD);
-        put4(sGB[buf][w], jq, gB);
-        put4(sDD[buf][w], jq, gD);
+        for (int jq = 0; jq < kT4; ++jq) bcg[jq] = sBlk[buf][g * kWsCons + w][jq][lane & 15];
+        auto put4 = [&](float4 (&slice)[kT4][kBlockCh], int q, const float (&v)[4]) {
+          float4& dst = slice[q][lane ^ bws_swz(q)];
+          if constexpr (kFirst) {
+            dst = make_float4(v[0], v[1], v[2], v[3]);
+          } else {
+            const float4 o = dst;
+            dst = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
+          }
+        };
+        auto fwd = [&](int jq, const StepVals& sv) {
+          float y[4];  // unused here (the forward saved the output)
+          bwd_recompute_block(jq, sv, bcg[jq], A2, hc, a, H, y);
+        };
+        // the reverse of block jq; its 16 dB/dC terms go to vals[16 * half ..]
+        auto rev = [&](int jq, const StepVals& sv, float (&vals)[32], int half) {
+          float gB[4], gD[4], v16[16];
+          bwd_reverse_block(jq, sv, bcg[jq], pA, A2, hc, a, H, pG, pD, v16, gB, gD);
+          put4(sGB[sl][w], jq, gB);
+          put4(sDD[sl][w], jq, gD);
 #pragma unroll
-        for (int k = 0; k < 16; ++k) vals[16 * half + k] = v16[k];
-      };
-      // sum over the 64 channels of blocks jq and jq - 1 together
-      auto reduce_store = [&](int jq, float (&vals)[32], auto old) {
-        wave_reduce32<decltype(old)::value>(vals, lane);
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(vals[0]), bc_rsrc,
-                                              (int)(bc_off + 16u * (jq - 1)), t0 * 4, 0);
-      };
-      auto ld = [&](int jq, StepVals& sv, bool with_dout) {
-        const int li = lane ^ bws_swz(jq);
-        sv.dl = sSt[buf][0][jq][li];
-        sv.du = sSt[buf][1][jq][li];
-        if (with_dout) sv.dout = sSt[buf][2][jq][li];
-      };
-      // fixed schedule F0 F1 F2 F3 R3 R2 R1 R0 (recompute, then reverse)
-      ld(0, X, false); fwd(0, X);
-      ld(1, Y, false); fwd(1, Y);
-      ld(2, X, false); fwd(2, X);
-      ld(3, Y, true);  fwd(3, Y);
-      // the reverse re-reads the block registers: hide their values from
-      // the recompute's, so each DPP broadcast folds into its own multiply
-      // (shared, it is materialised with an extra v_mov_dpp and a register)
+          for (int k = 0; k < 16; ++k) vals[16 * half + k] = v16[k];
+        };
+        // sum over the 64 channels of blocks jq and jq - 1 together
+        auto reduce_store = [&](int jq, float (&vals)[32], auto old) {
+          wave_reduce32<decltype(old)::value>(vals, lane);
+          const uint32_t off = rn + 16 * g < N ? bc_off + (uint32_t)(16 * g * Lp) * 4u : kOffDrop;
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(vals[0]), bc_rsrc,
+                                                (int)(off + 16u * (jq - 1)), t0 * 4, 0);
+        };
+        auto ld = [&](int jq, StepVals& sv, bool with_dout) {
+          const int li = lane ^ bws_swz(jq);
+          sv.dl = sSt[buf][0][jq][li];
+          sv.du = sSt[buf][1][jq][li];
+          if (with_dout) sv.dout = sSt[buf][2][jq][li];
+        };
+        // fixed schedule F0 F1 F2 F3 R3 R2 R1 R0 (recompute, then reverse)
+        ld(0, X, false); fwd(0, X);
+        ld(1, Y, false); fwd(1, Y);
+        ld(2, X, false); fwd(2, X);
+        ld(3, Y, true);  fwd(3, Y);
+        // the previous tile's slices have been read (see above)
+        if constexpr (kSG > 1 && kFirst) __syncthreads();
+        // the reverse re-reads the block registers: hide their values from
+        // the recompute's, so each DPP broadcast folds into its own multiply
+        // (shared, it is materialised with an extra v_mov_dpp and a register)
 #pragma unroll
-      for (int jq = 0; jq < kT4; ++jq) asm volatile("" : "+v"(bcg[jq]));
-      // blocks 3 and 2 are reduced after block 1's reverse, so their terms
-      // are not fresh VALU results at the folds
-      float v32[32], w32[32];
-      // X still holds block 2's delta and delta*u: read its dout only, and
-      // block 1's values a block ahead of their use
-      X.dout = sSt[buf][2][2][lane ^ bws_swz(2)];
-      StepVals Z;
-      ld(1, Z, true);
-      rev(3, Y, v32, 0);
-      rev(2, X, v32, 1);
-      ld(0, Y, true);
-      rev(1, Z, w32, 0);
-      reduce_store(3, v32, std::true_type{});
-      rev(0, Y, w32, 1);
-      reduce_store(1, w32, std::false_type{});
+        for (int jq = 0; jq < kT4; ++jq) asm volatile("" : "+v"(bcg[jq]));
+        // blocks 3 and 2 are reduced after block 1's reverse, so their terms
+        // are not fresh VALU results at the folds
+        float v32[32], w32[32];
+        // X still holds block 2's delta and delta*u: read its dout only, and
+        // block 1's values a block ahead of their use
+        X.dout = sSt[buf][2][2][lane ^ bws_swz(2)];
+        StepVals Z;
+        ld(1, Z, true);
+        rev(3, Y, v32, 0);
+        rev(2, X, v32, 1);
+        ld(0, Y, true);
+        rev(1, Z, w32, 0);
+        reduce_store(3, v32, std::true_type{});
+        rev(0, Y, w32, 1);
+        reduce_store(1, w32, std::false_type{});
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          if constexpr (kSG == 1) {
+            gam[0][s] = pG[s];
+            dA[0][s] = pD[s];
+          } else {
+            sPair[w][g][s][1][lane] = pG[s];
+            sPair[w][g][s][2][lane] = pD[s];
+          }
+        }
+      };
+      // (the first pair apart: a choice inside one loop would leave branches
+      // around the barrier and the LDS reads, and with them register copies)
+      pair(0, std::true_type{});
+      if constexpr (kSG > 1) {
+#pragma unroll 1
+        for (int g = 1; g < kSG; ++g) pair(g, std::false_type{});
+      }
     };
-    // nbar - 1 is a multiple of 4: iteration 0, then pairs of parity 1, 0
-    iteration(0, std::integral_constant<int, 0>{});
-    for (int i = 1; i < nbar; i += 2) {
-      iteration(i, std::integral_constant<int, 1>{});
-      iteration(i + 1, std::integral_constant<int, 0>{});
+    if constexpr (kSG == 1) {
+      // nbar - 1 is a multiple of 4: iteration 0, then pairs of parity 1, 0
+      iteration(0, std::integral_constant<int, 0>{});
+      for (int i = 1; i < nbar; i += 2) {
+        iteration(i, std::integral_constant<int, 1>{});
+        iteration(i + 1, std::integral_constant<int, 0>{});
+      }
+    } else {
+      for (int i = 0; i < nbar; ++i) iteration(i, i & 1);
     }
     // per-row partials
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int n = 2 * w + s;
-      if (ch_ok && n < N) {
-        ws_A[(srow * Dm + ch) * N + n] = dA[s];
-        if (dh_init && seg == 0) dh_init[(rb + ch) * N + n] = gam[s];
+    for (int g = 0; g < kSG; ++g)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int n = 2 * (g * kWsCons + w) + s;
+        if (ch_ok && n < N) {
+          ws_A[(srow * Dm + ch) * N + n] = kSG == 1 ? dA[g][s] : sPair[w][g][s][2][lane];
+          if (dh_init && seg == 0)
+            dh_init[(rb + ch) * N + n] = kSG == 1 ? gam[g][s] : sPair[w][g][s][1][lane];
+        }
       }
-    }
     return;
   }
 
@@ -927,12 +1033,12 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
   const bool softplus = p.softplus != 0;
   // B/C staging: lane pt -> state n = (pt / 16) % 16 and step pt % 16 of B
   // (first element) and of C (second)
+  // (states 16 g + bc_n of pair group g; clamped into the rows, zeroed at
+  // staging past N)
   const int bc_n = (pt / kTileB) % (2 * kWsCons);
   const int bc_j = pt % kTileB;
-  const bool bc_ok = bc_n < N;
-  const size_t bc_row = (size_t)b * p.bc_bstride + (size_t)min(bc_n, N - 1) * L;
-  const T* __restrict__ B_row = Bp + bc_row;
-  const T* __restrict__ C_row = Cp + bc_row;
+  const T* __restrict__ B_rows = Bp + (size_t)b * p.bc_bstride;
+  const T* __restrict__ C_rows = Cp + (size_t)b * p.bc_bstride;
   const int bc_slot = (bc_j & 3) * 4 + (bc_n & 1) * 2;  // B; C at + 1
   // tile index of iteration i (clamped to the segment: tiles past it are
   // staged from valid rows and never used)
@@ -962,9 +1068,10 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
   const uint32_t bc_bytes = (uint32_t)((size_t)N * L * sizeof(T));
   const auto B_ld = raw_rsrc(const_cast<T*>(Bp) + (size_t)b * p.bc_bstride, bc_bytes);
   const auto C_ld = raw_rsrc(const_cast<T*>(Cp) + (size_t)b * p.bc_bstride, bc_bytes);
-  const uint32_t bc_row_off = (uint32_t)((size_t)min(bc_n, N - 1) * L * sizeof(T));
+  auto bc_row = [&](int g) { return (size_t)min(16 * g + bc_n, N - 1) * L; };
 
-  auto issue = [&](BwsRows<T>& r, int i) {
+  using Rows = BwsRows<T, kSG>;
+  auto issue = [&](Rows& r, int i) {
     if constexpr (kAligned) {
       const int t0 = tile_of(i) * kTileB;
       const uint32_t off = row_off + (uint32_t)min(t0 + 4 * q, L - 4) * sizeof(T);
@@ -977,9 +1084,12 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
       } else {
         r.z = r.y = typename Raw4<T>::type{};
       }
-      const uint32_t boff = bc_row_off + (uint32_t)min(t0 + bc_j, L - 1) * sizeof(T);
-      r.B = buffer_load_bits1<T>(B_ld, boff);
-      r.C = buffer_load_bits1<T>(C_ld, boff);
+#pragma unroll
+      for (int g = 0; g < kSG; ++g) {
+        const uint32_t boff = (uint32_t)((bc_row(g) + min(t0 + bc_j, L - 1)) * sizeof(T));
+        r.B[g] = buffer_load_bits1<T>(B_ld, boff);
+        r.C[g] = buffer_load_bits1<T>(C_ld, boff);
+      }
       return;
     }
     const int t = tile_of(i) * kTileB + 4 * q;
@@ -992,9 +1102,12 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
     } else {
       r.z = r.y = typename Raw4<T>::type{};
     }
-    const int tb = min(tile_of(i) * kTileB + bc_j, L - 1);
-    r.B = elem_bits(B_row[tb]);
-    r.C = elem_bits(C_row[tb]);
+#pragma unroll
+    for (int g = 0; g < kSG; ++g) {
+      const size_t tb = bc_row(g) + min(tile_of(i) * kTileB + bc_j, L - 1);
+      r.B[g] = elem_bits(B_rows[tb]);
+      r.C[g] = elem_bits(C_rows[tb]);
+    }
   };
 
   // What a tile's finish needs from its staging besides delta and dout (read
@@ -1006,7 +1119,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
   };
 
   // stage iteration i's tile into buffer i & 1 and write its dz
-  auto stage = [&](const BwsRows<T>& r, int i, Kept& k) {
+  auto stage = [&](const Rows& r, int i, Kept& k) {
     const int tile = tile_of(i);
     const int t0 = tile * kTileB;
     const int t = t0 + 4 * q;
@@ -1064,9 +1177,13 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
     sSt[sb][0][q][sw] = make_float4(de[0], de[1], de[2], de[3]);
     sSt[sb][1][q][sw] = make_float4(du[0], du[1], du[2], du[3]);
     sSt[sb][2][q][sw] = make_float4(dov[0], dov[1], dov[2], dov[3]);
-    float* const blk_dst = &sBlk[sb][bc_n >> 1][bc_j >> 2][bc_slot];
-    blk_dst[0] = bc_ok ? bits_to_f32<T>(r.B) : 0.0f;
-    blk_dst[1] = bc_ok ? bits_to_f32<T>(r.C) : 0.0f;
+#pragma unroll
+    for (int g = 0; g < kSG; ++g) {
+      const bool bc_ok = 16 * g + bc_n < N;
+      float* const blk_dst = &sBlk[sb][g * kWsCons + (bc_n >> 1)][bc_j >> 2][bc_slot];
+      blk_dst[0] = bc_ok ? bits_to_f32<T>(r.B[g]) : 0.0f;
+      blk_dst[1] = bc_ok ? bits_to_f32<T>(r.C[g]) : 0.0f;
+    }
     // a tile past the segment (i >= nt) writes nothing
     const bool st_ok = pch_ok && i < nt;
     if constexpr (kHasZ) {
@@ -1084,15 +1201,16 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
     const int tile = tile_of(i);
     const int t = tile * kTileB + 4 * q;
     const int sb = i & 1;
-    float4 gb = sGB[sb][0][q][sw], gd = sDD[sb][0][q][sw];
+    const int sl = kSG == 1 ? sb : 0;
+    float4 gb = sGB[sl][0][q][sw], gd = sDD[sl][0][q][sw];
 #pragma unroll
     for (int ww = 1; ww < kWsCons; ++ww) {
-      const float4 q1 = sGB[sb][ww][q][sw];
+      const float4 q1 = sGB[sl][ww][q][sw];
       gb.x += q1.x; gb.y += q1.y; gb.z += q1.z; gb.w += q1.w;
     }
 #pragma unroll
     for (int ww = 1; ww < kWsCons; ++ww) {
-      const float4 q2 = sDD[sb][ww][q][sw];
+      const float4 q2 = sDD[sl][ww][q][sw];
       gd.x += q2.x; gd.y += q2.y; gd.z += q2.z; gd.w += q2.w;
     }
     const float gbv[4] = {gb.x, gb.y, gb.z, gb.w};
@@ -1132,13 +1250,14 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
   // 4 tiles (staged at iteration k - 1, finished at k + 1).  Iterations
   // 1 .. 4m run in unrolled groups of four with no conditions around memory
   // operations, so the compiler's waits for the ring's loads count exactly.
-  BwsRows<T> rows[kBwsRing];
+  Rows rows[kBwsRing];
   Kept kept[4];
 #pragma unroll
   for (int k2 = 0; k2 < kBwsRing; ++k2) issue(rows[k2], k2);
   stage(rows[0], 0, kept[0]);
   issue(rows[0], kBwsRing);
   __syncthreads();  // iteration 0
+  if constexpr (kSG > 1) __syncthreads();
   stage(rows[1], 1, kept[1]);
   issue(rows[1], kBwsRing + 1);
   for (int i0 = 1; i0 < nbar; i0 += 4) {
@@ -1147,6 +1266,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
       const int i = i0 + j;  // (i + 1) % 4 == (j + 2) % 4, (i - 1) % 4 == j
       __syncthreads();
       finish(i - 1, kept[j]);
+      if constexpr (kSG > 1) __syncthreads();  // the slices may be rewritten
       stage(rows[(j + 2) % kBwsRing], i + 1, kept[(j + 2) & 3]);
       issue(rows[(j + 2) % kBwsRing], i + 1 + kBwsRing);
     }
@@ -1409,7 +1529,7 @@ __global__ __launch_bounds__(kThreads) void scan_bwd_segsum_kernel(
   if (a_q == 0 && a_ok && n0 == 0) seg_dt[sb * Dm + a_ch] = dtsum;
 }
 
-// Role-split segment summaries of the backward for up to 16 states: the
+// Role-split segment summaries of the backward for up to 64 states: the
 // numbers scan_bwd_segsum_kernel computes, per sub-segment of seg_len / sub_k
 // steps (blockIdx.z = k: global sub-segment k + sub_k, so the sub-segments
 // of segments 1 .. nseg-1), with the forward's role split so that staging
@@ -1426,20 +1546,22 @@ __global__ __launch_bounds__(kThreads) void scan_bwd_segsum_kernel(
 // The main backward folds the summaries from the last sub-segment down to
 // the first one after its segment.  A sub-segment past the sequence end has
 // no tiles and leaves gamma = 0 and sum dt = 0 (the identity).
-template <typename T, bool kHasZ, bool kAligned>
-__global__ __launch_bounds__(kWsThreads, kAligned ? 6 : 5) void scan_bwd_segsum_ws_kernel(
+// kSG as in scan_bwd_ws_kernel (up to 16 kSG states).
+template <typename T, int kSG, bool kHasZ, bool kAligned>
+__global__ __launch_bounds__(kWsThreads, kSG == 1 && kAligned ? 6 : 5) void scan_bwd_segsum_ws_kernel(
     const ScanDims p, const T* __restrict__ dl, const T* __restrict__ dyp,
     const T* __restrict__ zp, const float* __restrict__ Ap, const T* __restrict__ Cp,
     const float* __restrict__ biasp, const int64_t* __restrict__ length,
     float* __restrict__ seg_g, float* __restrict__ seg_dt) {
   // raw rows in flight: 4 tiles; 2 for fp32, whose 16-byte pieces would
   // otherwise hold the producers above the registers of two workgroups per CU
-  constexpr int kTile = 16, kT4 = kTile / 4, kStage = 3, kRing = sizeof(T) == 4 ? 2 : 4;
+  constexpr int kTile = 16, kT4 = kTile / 4, kStage = 3;
+  constexpr int kRing = sizeof(T) == 4 || kSG > 1 ? 2 : 4;
   constexpr int kRow = kBlockCh + 2;  // column length in float4s (the forward's padding)
   static_assert(kWsProd * 64 == kBlockCh * kT4, "one producer lane per (row, column)");
   static_assert(2 * kWsCons * kTile == 64 * kWsProd, "one C element per producer lane");
   __shared__ float4 sSt[kStage][2][kT4][kRow];   // [delta | effective dout][column][row]
-  __shared__ float4 sC[kStage][kWsCons][kTile / 2];  // (C_2w, C_2w+1) of steps 2i, 2i+1
+  __shared__ float4 sC[kStage][kSG * kWsCons][kTile / 2];  // (C0, C1) of a pair, steps 2i, 2i+1
 
   const int lane = threadIdx.x & 63;
   const int w = wave_id_uniform();
@@ -1459,53 +1581,75 @@ __global__ __launch_bounds__(kWsThreads, kAligned ? 6 : 5) void scan_bwd_segsum_
     // ------------------------------------------------ consumer: the reverse recurrence
     const int ch = d0 + lane;
     const bool ch_ok = ch < Dm;
-    float gam[2] = {0.0f, 0.0f}, A2[2];
+    float gam[kSG][2], A2[kSG][2];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int n = 2 * w + s;
-      A2[s] = (ch_ok && n < N) ? Ap[(size_t)ch * N + n] * kLog2e : 0.0f;
-    }
-    // block k: delta and dout of steps 4k .. 4k+3, and (C0, C1) of those
-    // steps as two float4s (the same address in every lane: broadcast reads)
+    for (int g = 0; g < kSG; ++g)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int n = 2 * (g * kWsCons + w) + s;
+        gam[g][s] = 0.0f;
+        A2[g][s] = (ch_ok && n < N) ? Ap[(size_t)ch * N + n] * kLog2e : 0.0f;
+      }
+    // stage kk * kSG + g of a tile: block k = 3 - kk of pair g.  delta and dout
+    // of a block's steps 4k .. 4k+3, and a pair's (C0, C1) of those steps as
+    // two float4s (the same address in every lane: broadcast reads)
     float4 dlb[2], dob[2], cb[2][2];
-    auto read_block = [&](int buf, int k, float4& dl4, float4& do4, float4 (&c)[2]) {
+    auto read_c = [&](int buf, int k, int g, float4 (&c)[2]) {
+      c[0] = sC[buf][g * kWsCons + w][2 * k];
+      c[1] = sC[buf][g * kWsCons + w][2 * k + 1];
+    };
+    auto read_steps = [&](int buf, int k, float4& dl4, float4& do4) {
       const float4* __restrict__ st = &sSt[buf][0][0][lane];
       dl4 = st[k * kRow];
       do4 = st[(kT4 + k) * kRow];
-      c[0] = sC[buf][w][2 * k];
-      c[1] = sC[buf][w][2 * k + 1];
     };
     int buf = 0;
     for (int i = 0; i < nbar; ++i) {
       __syncthreads();
       if (i >= ntiles) continue;
-      if (i == 0) read_block(0, kT4 - 1, dlb[0], dob[0], cb[0]);
+      if (i == 0) {
+        read_steps(0, kT4 - 1, dlb[0], dob[0]);
+        read_c(0, kT4 - 1, 0, cb[0]);
+      }
       const int nbuf = buf == kStage - 1 ? 0 : buf + 1;
-      // block k - 1's LDS reads are issued before block k is computed; after
-      // block 0, the next tile's last block (staged one iteration ago)
+      // the next stage's LDS reads are issued before a stage is computed;
+      // after block 0, the next tile's last block (staged one iteration ago)
 #pragma unroll
       for (int kk = 0; kk < kT4; ++kk) {
-        const int c = kk & 1;
-        if (kk + 1 < kT4) read_block(buf, kT4 - 2 - kk, dlb[c ^ 1], dob[c ^ 1], cb[c ^ 1]);
-        else read_block(nbuf, kT4 - 1, dlb[c ^ 1], dob[c ^ 1], cb[c ^ 1]);
-        const float dlv[4] = {dlb[c].x, dlb[c].y, dlb[c].z, dlb[c].w};
-        const float dov[4] = {dob[c].x, dob[c].y, dob[c].z, dob[c].w};
-        const float c0[4] = {cb[c][0].x, cb[c][0].z, cb[c][1].x, cb[c][1].z};
-        const float c1[4] = {cb[c][0].y, cb[c][0].w, cb[c][1].y, cb[c][1].w};
+        const int d = kk & 1;
 #pragma unroll
-        for (int j = 3; j >= 0; --j) {
-          gam[0] = fast_exp2(dlv[j] * A2[0]) * fmaf(dov[j], c0[j], gam[0]);
-          gam[1] = fast_exp2(dlv[j] * A2[1]) * fmaf(dov[j], c1[j], gam[1]);
+        for (int g = 0; g < kSG; ++g) {
+          const int c = (kk * kSG + g) & 1;
+          if (g + 1 < kSG) {
+            read_c(buf, kT4 - 1 - kk, g + 1, cb[c ^ 1]);
+          } else if (kk + 1 < kT4) {
+            read_steps(buf, kT4 - 2 - kk, dlb[d ^ 1], dob[d ^ 1]);
+            read_c(buf, kT4 - 2 - kk, 0, cb[c ^ 1]);
+          } else {
+            read_steps(nbuf, kT4 - 1, dlb[d ^ 1], dob[d ^ 1]);
+            read_c(nbuf, kT4 - 1, 0, cb[c ^ 1]);
+          }
+          const float dlv[4] = {dlb[d].x, dlb[d].y, dlb[d].z, dlb[d].w};
+          const float dov[4] = {dob[d].x, dob[d].y, dob[d].z, dob[d].w};
+          const float c0[4] = {cb[c][0].x, cb[c][0].z, cb[c][1].x, cb[c][1].z};
+          const float c1[4] = {cb[c][0].y, cb[c][0].w, cb[c][1].y, cb[c][1].w};
+#pragma unroll
+          for (int j = 3; j >= 0; --j) {
+            gam[g][0] = fast_exp2(dlv[j] * A2[g][0]) * fmaf(dov[j], c0[j], gam[g][0]);
+            gam[g][1] = fast_exp2(dlv[j] * A2[g][1]) * fmaf(dov[j], c1[j], gam[g][1]);
+          }
         }
       }
       static_assert(kT4 % 2 == 0, "the last block of every tile in register set 0");
       buf = nbuf;
     }
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int n = 2 * w + s;
-      if (ch_ok && n < N) seg_g[(sb * N + n) * Dm + ch] = gam[s];
-    }
+    for (int g = 0; g < kSG; ++g)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int n = 2 * (g * kWsCons + w) + s;
+        if (ch_ok && n < N) seg_g[(sb * N + n) * Dm + ch] = gam[g][s];
+      }
     return;
   }
 
@@ -1527,9 +1671,8 @@ __global__ __launch_bounds__(kWsThreads, kAligned ? 6 : 5) void scan_bwd_segsum_
   const int c_half = pt / (kWsCons * kTile);
   const int c_G = (pt / kTile) % kWsCons;
   const int c_step = pt % kTile;
-  const int c_n = 2 * c_G + c_half;
-  const bool c_ok = c_n < N;
-  const size_t c_row = (size_t)b * p.bc_bstride + (size_t)min(c_n, N - 1) * L;
+  auto c_n = [&](int g) { return 2 * (g * kWsCons + c_G) + c_half; };  // of pair group g
+  auto c_row = [&](int g) { return (size_t)min(c_n(g), N - 1) * L; };
   // aligned rows: buffer ranges over the wave's 16 channel rows (the launch
   // keeps 16 * L * sizeof(T) below 2^31) and over the batch row's C rows
   const int wrow0 = d0 + (w - kWsCons) * (kBlockCh / kWsProd);
@@ -1542,14 +1685,13 @@ __global__ __launch_bounds__(kWsThreads, kAligned ? 6 : 5) void scan_bwd_segsum_
                              kHasZ ? wbytes : 0u);
   const auto C_ld = raw_rsrc(const_cast<T*>(Cp) + (size_t)b * p.bc_bstride,
                              (uint32_t)((size_t)N * L * sizeof(T)));
-  const uint32_t c_row_off = (uint32_t)((size_t)min(c_n, N - 1) * L * sizeof(T));
   const T* __restrict__ d_row = dl + (rb + chc) * L;
   const T* __restrict__ y_row = dyp + (rb + chc) * L;
   const T* __restrict__ z_row = kHasZ ? zp + (rb + chc) * L : y_row;
 
   struct Rows {
     typename Raw4<T>::type d, y, z;
-    uint32_t C;
+    uint32_t C[kSG];
   };
   // raw loads of tile i, the step clamped into the row (tiles past the walk
   // load data that is never used)
@@ -1561,13 +1703,17 @@ __global__ __launch_bounds__(kWsThreads, kAligned ? 6 : 5) void scan_bwd_segsum_
       r.y = buffer_load_raw4<T>(y_ld, off);
       if constexpr (kHasZ) r.z = buffer_load_raw4<T>(z_ld, off);
       else r.z = typename Raw4<T>::type{};
-      r.C = buffer_load_bits1<T>(C_ld, c_row_off + (uint32_t)min(t0 + c_step, L - 1) * sizeof(T));
+#pragma unroll
+      for (int g = 0; g < kSG; ++g)
+        r.C[g] = buffer_load_bits1<T>(C_ld, (uint32_t)((c_row(g) + min(t0 + c_step, L - 1)) * sizeof(T)));
     } else {
       r.d = load_raw4_nb<T, kAligned>(d_row, t0 + 4 * q, L, pch_ok);
       r.y = load_raw4_nb<T, kAligned>(y_row, t0 + 4 * q, L, pch_ok);
       if constexpr (kHasZ) r.z = load_raw4_nb<T, kAligned>(z_row, t0 + 4 * q, L, pch_ok);
       else r.z = typename Raw4<T>::type{};
-      r.C = elem_bits(Cp[c_row + min(t0 + c_step, L - 1)]);
+#pragma unroll
+      for (int g = 0; g < kSG; ++g)
+        r.C[g] = elem_bits(Cp[(size_t)b * p.bc_bstride + c_row(g) + min(t0 + c_step, L - 1)]);
     }
   };
   float dtsum = 0.0f;
@@ -1590,8 +1736,10 @@ __global__ __launch_bounds__(kWsThreads, kAligned ? 6 : 5) void scan_bwd_segsum_
     }
     sSt[sbuf][0][q][row] = make_float4(de[0], de[1], de[2], de[3]);
     sSt[sbuf][1][q][row] = make_float4(dov[0], dov[1], dov[2], dov[3]);
-    reinterpret_cast<float*>(&sC[sbuf][c_G][0])[2 * c_step + c_half] =
-        c_ok ? bits_to_f32<T>(r.C) : 0.0f;
+#pragma unroll
+    for (int g = 0; g < kSG; ++g)
+      reinterpret_cast<float*>(&sC[sbuf][g * kWsCons + c_G][0])[2 * c_step + c_half] =
+          c_n(g) < N ? bits_to_f32<T>(r.C[g]) : 0.0f;
   };
 
   // Iteration i after barrier i stages tile i + 2 into buffer (i + 2) % 3
@@ -1716,7 +1864,9 @@ static hipError_t launch_bwd4(const ScanParams& p, const float* bc, hipStream_t 
   // the role-split kernels' buffer ranges must fit 2^31 bytes: a wave's 16
   // channel rows, all of the dB/dC partials, and a batch row's saved states
   const bool ws =
-      kSG == 1 && !kPart && (size_t)(kBlockCh / kWsProd) * p.seqlen * sizeof(T) < (1u << 31) &&
+      !kPart && (size_t)p.nstate * p.seqlen * sizeof(T) < (1u << 31) &&
+      (size_t)p.dim * p.nstate * sizeof(float) < (1u << 31) &&
+      (size_t)(kBlockCh / kWsProd) * p.seqlen * sizeof(T) < (1u << 31) &&
       2 * (size_t)p.nblk * p.batch * p.nstate * bc_part_len(p.seqlen) * sizeof(float) < (1u << 31) &&
       (size_t)p.nchunks * p.nstate * p.hs * p.dim * sizeof(float) < (1u << 31);
   if (p.nseg > 1) {
@@ -1724,7 +1874,7 @@ static hipError_t launch_bwd4(const ScanParams& p, const float* bc, hipStream_t 
     // the role-split summaries per sub-segment (p.sub_k per segment), the
     // general ones per segment
     if (ws) {
-      hipLaunchKernelGGL((scan_bwd_segsum_ws_kernel<T, kHasZ, kAligned>),
+      hipLaunchKernelGGL((scan_bwd_segsum_ws_kernel<T, kSG, kHasZ, kAligned>),
                          dim3(p.nblk, p.batch, (p.nseg - 1) * p.sub_k), dim3(kWsThreads), 0, st,
                          dims_of(p), (const T*)p.delta, (const T*)p.dout, (const T*)p.z, p.A,
                          (const T*)p.C, p.bias, p.length, p.seg_h, p.seg_dt);
@@ -1743,7 +1893,7 @@ static hipError_t launch_bwd4(const ScanParams& p, const float* bc, hipStream_t 
   dim3 grid(p.nblk, p.batch, p.nseg * nsc);
   if (ws) {
     ProfScope prof("scan_bwd", st);
-    hipLaunchKernelGGL((scan_bwd_ws_kernel<T, kHasZ, kAligned>), grid, dim3(kWsThreads), 0, st,
+    hipLaunchKernelGGL((scan_bwd_ws_kernel<T, kSG, kHasZ, kAligned>), grid, dim3(kWsThreads), 0, st,
                        dims_of(p), (const T*)p.u, (const T*)p.delta, p.A, (const T*)p.B,
                        (const T*)p.C, p.D, p.bias, p.h_init, p.length, (const T*)p.z,
                        (const T*)p.out_ungated, p.h_chunks_in, (const T*)p.dout, p.dh_last,

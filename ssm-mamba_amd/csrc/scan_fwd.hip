@@ -6,8 +6,10 @@
 //   h_t     = exp(delta_t * A_dn) * h_{t-1} + delta_t * u_t * B_nt
 //   out_t   = D_d * u_t + sum_n C_nt * h_t     (* silu(z_t) when z is given)
 //
-// Work decomposition (one workgroup = one batch row b x 64 channels, 8 waves,
-// two waves per SIMD):
+// Two kernels share the work by state count.  Up to 64 states (and within the
+// buffer ranges) the role-split kernel, scan_fwd_ws_kernel below; past that
+// the general kernel, described here (one workgroup = one batch row b x 64
+// channels, 8 waves, two waves per SIMD):
 //   phase A  the 512 threads stream a 64-channel x 32-step tile of u / delta
 //            (/ z) (4 consecutive steps per thread, coalesced rows), evaluate
 //            softplus once per element and stage delta and delta*u in LDS as
@@ -15,13 +17,9 @@
 //            are loaded during the previous tile's phase B;
 //   phase B  lane = channel, wave w = state pairs G = g*8 + w: a sequential
 //            recurrence over the tile held in registers.  B and C are
-//            wave-uniform (same b, n, t across the wave).  With N <= 16 phase A
-//            reads them straight from B and C (coalesced along the steps) and
-//            stages the super-tile's (B0, C0, B1, C1) per pair and step in LDS,
-//            read back with broadcast loads; larger N read the prepped fp32
-//            block layout through scalar loads.  Each 4-step block's loads are
-//            issued one block ahead.  Each wave leaves its partial sum over its
-//            states of C*h in its own LDS slice;
+//            wave-uniform (same b, n, t across the wave), read from the prepped
+//            fp32 block layout through scalar loads.  Each wave leaves its
+//            partial sum over its states of C*h in its own LDS slice;
 //   phase C  the phase-A threads add the eight slices in a fixed order, D*u
 //            and the z gate, and store the tile.
 // The state after every kChunk steps is saved for the backward (h_chunks,
@@ -111,6 +109,10 @@ __device__ __forceinline__ void fwd_block_state(const float4 dl4, const float4 d
   }
 }
 
+// State pairs of a wave in the general kernels: up to 256 states in 8 waves
+// (pairs past N are skipped, wave-uniformly).
+constexpr int kGenSG = 16;
+
 // Every pointer is its own __restrict__ argument: with that no-alias
 // information the compiler can prove the output stores never clobber the
 // prepped B/C block, which is what lets its wave-uniform reads be scalar loads.
@@ -122,15 +124,15 @@ __device__ __forceinline__ void fwd_block_state(const float4 dl4, const float4 d
 //
 // kZ: 0 no gate; 1 out = y * silu(z); 2 the same and the ungated y also
 // written to yu (the value the backward needs for dz).
-template <typename T, int kSG, int kZ, bool kAligned>
+template <typename T, int kZ, bool kAligned>
 __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
     const ScanDims p, const T* __restrict__ u, const T* __restrict__ dl,
-    const float* __restrict__ Ap, const float* __restrict__ bc, const T* __restrict__ Bp,
-    const T* __restrict__ Cp, const float* __restrict__ Dp, const float* __restrict__ biasp,
-    const float* __restrict__ h_init, const int64_t* __restrict__ length,
-    const T* __restrict__ zp, T* __restrict__ out, T* __restrict__ yu,
-    float* __restrict__ h_chunks, float* __restrict__ h_last, void* __restrict__ dummy,
+    const float* __restrict__ Ap, const float* __restrict__ bc, const float* __restrict__ Dp,
+    const float* __restrict__ biasp, const float* __restrict__ h_init,
+    const int64_t* __restrict__ length, const T* __restrict__ zp, T* __restrict__ out,
+    T* __restrict__ yu, float* __restrict__ h_chunks, float* __restrict__ h_last,
     const float* __restrict__ seg_h, const float* __restrict__ seg_dt) {
+  constexpr int kSG = kGenSG;
   using R4 = typename Raw4<T>::type;
   constexpr bool kHasZ = kZ != 0;
   constexpr bool kSaveY = kZ == 2;
@@ -141,8 +143,6 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
   __shared__ float4 sDelta[kSubF * kT4][kBlockCh];
   __shared__ float4 sDu[kSubF * kT4][kBlockCh];
   __shared__ float4 sY[kWaves][kT4][kBlockCh];
-  // prepped B/C of the super-tile for state pairs 0..7: [sub][pair][step]
-  __shared__ float4 sBC[kSubF][kWaves][kTileF];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -199,7 +199,6 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
   const bool softplus = p.softplus != 0;
   const bool save = h_chunks != nullptr;
   const size_t hsD = (size_t)p.hs * Dm;  // floats between the saved rows of two states
-  float* const dummyf = static_cast<float*>(dummy);
 
   // Raw row pieces of the next super-tile, all loads issued at once right
   // after the current super-tile's phase A.  They are consumed together at
@@ -208,16 +207,6 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
   // registers free of merges).
   const int last_t0 = (Lend - 1) / kTileF * kTileF;
   R4 qu[kSubF], qd[kSubF], qz[kSubF];
-  // B/C staging (kSG == 1): thread -> (pair, step) of the super-tile,
-  // kBCPer items of (B0, C0, B1, C1) read straight from B and C (the states
-  // 2G, 2G+1 of the pair; masked to zero at staging for states past N, so
-  // those waves run the common path and add nothing)
-  constexpr int kBCItems = kSubF * kWaves * kTileF;
-  constexpr int kBCPer = kBCItems / kThreads;
-  static_assert(kBCItems % kThreads == 0, "whole B/C items per thread");
-  const T* __restrict__ Braw = static_cast<const T*>(Bp) + (size_t)b * p.bc_bstride;
-  const T* __restrict__ Craw = static_cast<const T*>(Cp) + (size_t)b * p.bc_bstride;
-  float qbc[kBCPer][4];
   auto issue = [&](int T0) {
 #pragma unroll
     for (int i = 0; i < kSubF; ++i) {
@@ -227,31 +216,8 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
       if constexpr (kHasZ) qz[i] = load_raw4_nb<T, kAligned>(z_row, t, L, a_ok);
       else qz[i] = R4{};
     }
-    if constexpr (kSG == 1) {
-#pragma unroll
-      for (int r = 0; r < kBCPer; ++r) {
-        const int item = r * kThreads + tid;
-        const int step = item % kTileF;
-        const int G = (item / kTileF) % kWaves;
-        const int sub = item / (kTileF * kWaves);
-        // clamped into the rows (steps past L only meet delta = 0 and are
-        // never stored; states past N are zeroed at staging)
-        const int t = min(min(T0, last_t0) + sub * kTileF + step, L - 1);
-        const size_t o0 = (size_t)min(2 * G, N - 1) * L + t;
-        const size_t o1 = (size_t)min(2 * G + 1, N - 1) * L + t;
-        qbc[r][0] = Elem<T>::load1(Braw + o0);
-        qbc[r][1] = Elem<T>::load1(Craw + o0);
-        qbc[r][2] = Elem<T>::load1(Braw + o1);
-        qbc[r][3] = Elem<T>::load1(Craw + o1);
-      }
-    }
   };
 
-  // kFull (whole super-tile inside the sequence, kSG == 1): the steady
-  // state, with no branches around memory operations, so the compiler's
-  // waits for the prefetched rows count exactly what is needed.  Otherwise
-  // the general code (last super-tile, N > 16).
-  //
   // The loop is rotated: a super-tile's phase A runs at the end of the
   // previous iteration, so the wait for its rows sits in the same iteration
   // as their loads and the stores issued after them (no loop-header merge in
@@ -259,12 +225,11 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
   float skip[kSubF][4], gate[kSubF][4];  // phase A -> phase C: D*u, silu(z)
   // ---- phase A: softplus once per element, stage delta and delta*u for
   // the whole super-tile; D*u and silu(z) are kept for phase C.
-  auto phase_a = [&](const int T0, auto full_tag) {
-    constexpr bool kFull = decltype(full_tag)::value;
+  auto phase_a = [&](const int T0) {
 #pragma unroll
     for (int i = 0; i < kSubF; ++i) {
       const int t0 = T0 + i * kTileF;
-      if (kFull || t0 < Lend) {
+      if (t0 < Lend) {
         float uv[4], dv[4], de[4], du[4];
         decode4(qu[i], uv);
         decode4(qd[i], dv);
@@ -288,29 +253,17 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
         sDu[i * kT4 + a_q][a_sw] = make_float4(du[0], du[1], du[2], du[3]);
       }
     }
-    if constexpr (kSG == 1) {
-#pragma unroll
-      for (int r = 0; r < kBCPer; ++r) {
-        const int item = r * kThreads + tid;
-        const int G = (item / kTileF) % kWaves;
-        const bool ok0 = 2 * G < N, ok1 = 2 * G + 1 < N;
-        sBC[item / (kTileF * kWaves)][G][item % kTileF] =
-            make_float4(ok0 ? qbc[r][0] : 0.0f, ok0 ? qbc[r][1] : 0.0f, ok1 ? qbc[r][2] : 0.0f,
-                        ok1 ? qbc[r][3] : 0.0f);
-      }
-    }
   };
 
   // ---- phases B and C of the super-tile staged by the last phase A
-  auto body = [&](const int T0, auto full_tag) {
-    constexpr bool kFull = decltype(full_tag)::value;
+  auto body = [&](const int T0) {
     __syncthreads();
     issue(T0 + kSup);
 
 #pragma unroll
     for (int i = 0; i < kSubF; ++i) {
       const int t0 = T0 + i * kTileF;
-      if (!kFull && t0 >= Lend) break;
+      if (t0 >= Lend) break;
       const float4* __restrict__ cDelta = sDelta[i * kT4];
       const float4* __restrict__ cDu = sDu[i * kT4];
       // ---- phase B over sub-tile i
@@ -330,127 +283,22 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
             }
         }
       };
-      if constexpr (kFull) {
-        // every wave: full sub-tile, fully unrolled, static B/C offsets and
-        // buffers; carries after blocks 3 and 7 (masked-off ones go to the
-        // dummy slot).  Block k+1's LDS loads are issued right after block
-        // k's have arrived, then block k is computed.
-        const float4* __restrict__ cBC = sBC[i][w];
-        const bool hc_ok = save && ch_ok && w < ngroups;
-        const bool hc2_ok = hc_ok && 2 * w + 1 < N;
-        float* const hc = h_chunks + (((size_t)b * p.nchunks + t0 / kChunk) * N + 2 * w) * hsD + ch;
-        BC2 bcb[2];
-        float4 dlb[2], dub[2];
-        lds_bc_block(cBC, 0, bcb[0]);
-        dlb[0] = cDelta[lane ^ col_swz(0)];
-        dub[0] = cDu[lane ^ col_swz(0)];
+      for (int t4 = 0; t4 < nT4; ++t4) {
+        const float4 dl4 = cDelta[t4 * kBlockCh + (lane ^ col_swz(t4))];
+        const float4 du4 = cDu[t4 * kBlockCh + (lane ^ col_swz(t4))];
+        float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        const int tb = t0 + 4 * t4;
 #pragma unroll
-        for (int k = 0; k < kT4; ++k) {
-          const int c = k & 1;
-          if (k + 1 < kT4) {
-            dlb[c ^ 1] = cDelta[(k + 1) * kBlockCh + (lane ^ col_swz(k + 1))];
-            dub[c ^ 1] = cDu[(k + 1) * kBlockCh + (lane ^ col_swz(k + 1))];
-            lds_bc_block(cBC, 4 * (k + 1), bcb[c ^ 1]);
-          }
-          float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-          fwd_block(dlb[c], dub[c], bcb[c], A2[0], h[0], y);
-          sY[w][k][lane ^ col_swz(k)] = make_float4(y[0], y[1], y[2], y[3]);
-          if ((k & 3) == 3) {
-            const size_t off = (size_t)(k / 4) * N * hsD;
-            *(hc_ok ? hc + off : dummyf) = h[0][0];
-            *(hc2_ok ? hc + off + hsD : dummyf) = h[0][1];
+        for (int g = 0; g < kSG; ++g) {
+          const int G = g * kWaves + w;
+          if (G < ngroups) {
+            BC2 v;
+            load_bc_block(bc, bc_offset(b, G, npair, Lp, tb), v);
+            fwd_block(dl4, du4, v, A2[g], h[g], y);
           }
         }
-      } else if constexpr (kSG == 1) {
-        if (w < ngroups && nT4 == kT4) {
-          // full sub-tile, fully unrolled: static B/C offsets and buffers,
-          // carries after blocks 3 and 7.  Block k+1's LDS and scalar loads
-          // are issued right after block k's have arrived, then block k is
-          // computed.
-          const float4* __restrict__ cBC = sBC[i][w];
-          float* hc = (save && ch_ok)
-                          ? h_chunks + (((size_t)b * p.nchunks + t0 / kChunk) * N + 2 * w) * hsD + ch
-                          : nullptr;
-          const bool second = 2 * w + 1 < N;
-          BC2 bcb[2];
-          float4 dlb[2], dub[2];
-          lds_bc_block(cBC, 0, bcb[0]);
-          dlb[0] = cDelta[lane ^ col_swz(0)];
-          dub[0] = cDu[lane ^ col_swz(0)];
-#pragma unroll
-          for (int k = 0; k < kT4; ++k) {
-            const int c = k & 1;
-            if (k + 1 < kT4) {
-              dlb[c ^ 1] = cDelta[(k + 1) * kBlockCh + (lane ^ col_swz(k + 1))];
-              dub[c ^ 1] = cDu[(k + 1) * kBlockCh + (lane ^ col_swz(k + 1))];
-              lds_bc_block(cBC, 4 * (k + 1), bcb[c ^ 1]);
-            }
-            float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            fwd_block(dlb[c], dub[c], bcb[c], A2[0], h[0], y);
-            sY[w][k][lane ^ col_swz(k)] = make_float4(y[0], y[1], y[2], y[3]);
-            if ((k & 3) == 3 && hc) {
-              float* q = hc + (size_t)(k / 4) * N * hsD;
-              q[0] = h[0][0];
-              if (second) q[hsD] = h[0][1];
-            }
-          }
-        } else if (w < ngroups) {
-          // partial last sub-tile: pairs of blocks; every prefetch is
-          // unconditional (the index is clamped to the last block) so the
-          // buffers stay in scalar registers
-          const float4* __restrict__ cBC = sBC[i][w];
-          float4 dlA = cDelta[lane ^ col_swz(0)], duA = cDu[lane ^ col_swz(0)], dlB, duB;
-          BC2 bcA, bcB;
-          lds_bc_block(cBC, 0, bcA);
-          int t4 = 0;
-          for (; t4 + 1 < nT4; t4 += 2) {
-            dlB = cDelta[(t4 + 1) * kBlockCh + (lane ^ col_swz(t4 + 1))];
-            duB = cDu[(t4 + 1) * kBlockCh + (lane ^ col_swz(t4 + 1))];
-            lds_bc_block(cBC, 4 * (t4 + 1), bcB);
-            {
-              float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-              fwd_block(dlA, duA, bcA, A2[0], h[0], y);
-              sY[w][t4][lane ^ col_swz(t4)] = make_float4(y[0], y[1], y[2], y[3]);
-              store_carry(t4);
-            }
-            const int n2 = min(t4 + 2, nT4 - 1);
-            dlA = cDelta[n2 * kBlockCh + (lane ^ col_swz(n2))];
-            duA = cDu[n2 * kBlockCh + (lane ^ col_swz(n2))];
-            lds_bc_block(cBC, 4 * n2, bcA);
-            {
-              float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-              fwd_block(dlB, duB, bcB, A2[0], h[0], y);
-              sY[w][t4 + 1][lane ^ col_swz(t4 + 1)] = make_float4(y[0], y[1], y[2], y[3]);
-              store_carry(t4 + 1);
-            }
-          }
-          if (t4 < nT4) {  // odd last block
-            float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            fwd_block(dlA, duA, bcA, A2[0], h[0], y);
-            sY[w][t4][lane ^ col_swz(t4)] = make_float4(y[0], y[1], y[2], y[3]);
-            store_carry(t4);
-          }
-        } else {
-          for (int t4 = 0; t4 < nT4; ++t4) sY[w][t4][lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-      } else {
-        for (int t4 = 0; t4 < nT4; ++t4) {
-          const float4 dl4 = cDelta[t4 * kBlockCh + (lane ^ col_swz(t4))];
-          const float4 du4 = cDu[t4 * kBlockCh + (lane ^ col_swz(t4))];
-          float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-          const int tb = t0 + 4 * t4;
-#pragma unroll
-          for (int g = 0; g < kSG; ++g) {
-            const int G = g * kWaves + w;
-            if (G < ngroups) {
-              BC2 v;
-              load_bc_block(bc, bc_offset(b, G, npair, Lp, tb), v);
-              fwd_block(dl4, du4, v, A2[g], h[g], y);
-            }
-          }
-          sY[w][t4][lane ^ col_swz(t4)] = make_float4(y[0], y[1], y[2], y[3]);
-          store_carry(t4);
-        }
+        sY[w][t4][lane ^ col_swz(t4)] = make_float4(y[0], y[1], y[2], y[3]);
+        store_carry(t4);
       }
       __syncthreads();
 
@@ -458,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
       // D*u and the gate
       {
         const int t = t0 + a_col;
-        if (kFull || (a_ok && t < Lend)) {
+        if (a_ok && t < Lend) {
           float y[4];
           float4 acc = sY[0][a_q][a_sw];
 #pragma unroll
@@ -471,39 +319,27 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
           y[2] = skip[i][2] + acc.z;
           y[3] = skip[i][3] + acc.w;
           if constexpr (kSaveY) {
-            if constexpr (kFull) store4_nb<T, kAligned>(yu + (rb + a_ch) * L, t, L, a_ok, dummy, y);
-            else store4<T, kAligned>(yu + (rb + a_ch) * L, t, L, y);
+            store4<T, kAligned>(yu + (rb + a_ch) * L, t, L, y);
           }
           if constexpr (kHasZ) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) y[j] *= gate[i][j];
           }
-          if constexpr (kFull) store4_nb<T, kAligned>(out + (rb + a_ch) * L, t, L, a_ok, dummy, y);
-          else store4<T, kAligned>(out + (rb + a_ch) * L, t, L, y);
+          store4<T, kAligned>(out + (rb + a_ch) * L, t, L, y);
         }
       }
       // the next sub-tile's phase B rewrites the slices
-      if (i + 1 < kSubF && (kFull || t0 + kTileF < Lend)) __syncthreads();
+      if (i + 1 < kSubF && t0 + kTileF < Lend) __syncthreads();
     }
-    // the next phase A rewrites only sDelta / sDu / sBC, last read by the
+    // the next phase A rewrites only sDelta / sDu, last read by the
     // final phase B before the barrier that preceded the final phase C
   };
 
   issue(Tbeg);
-  if (kSG == 1 && Tbeg + kSup <= Lend) phase_a(Tbeg, std::true_type{});
-  else phase_a(Tbeg, std::false_type{});
-  int T0 = Tbeg;
-  if constexpr (kSG == 1) {
-    for (; T0 + kSup <= Lend; T0 += kSup) {
-      body(T0, std::true_type{});
-      const int Tn = T0 + kSup;
-      if (Tn + kSup <= Lend) phase_a(Tn, std::true_type{});
-      else if (Tn < Lend) phase_a(Tn, std::false_type{});
-    }
-  }
-  for (; T0 < Lend; T0 += kSup) {
-    body(T0, std::false_type{});
-    if (T0 + kSup < Lend) phase_a(T0 + kSup, std::false_type{});
+  phase_a(Tbeg);
+  for (int T0 = Tbeg; T0 < Lend; T0 += kSup) {
+    body(T0);
+    if (T0 + kSup < Lend) phase_a(T0 + kSup);
   }
 
   if (!save && h_last && ch_ok && Lend == L) {
@@ -517,12 +353,13 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(
   }
 }
 
-// ---------------------------------------------------------------- forward, N <= 16
+// ---------------------------------------------------------------- forward, N <= 64
 
-// Role-split forward for up to 16 states.  A workgroup of 12 waves covers one
+// Role-split forward for up to 64 states.  A workgroup of 12 waves covers one
 // batch row b x 64 channels and walks its segment in 16-step tiles (one saved
 // chunk each):
-//   consumer waves 0..7   lane = channel, wave w = states 2w and 2w+1: the
+//   consumer waves 0..7   lane = channel, wave w = states 2w and 2w+1 (and
+//                         16 g + 2w, + 1 for g < kSG past 16 states): the
 //                         recurrence over tile i, reading delta, delta*u and
 //                         B/C from LDS; each wave leaves its partial sums of
 //                         C*h in its own LDS slice;
@@ -565,17 +402,17 @@ constexpr int kWsRow = kBlockCh + 2;
 
 // One tile's raw loads of a producer lane, kept as loaded bits: converting
 // at the load would make the compiler wait for it right there.
-template <typename T, bool kDt = false>
+template <typename T, int kSG, bool kDt = false>
 struct WsRows {
   typename Raw4<T>::type u, d, z;
-  uint32_t B, C;  // element bits
+  uint32_t B[kSG], C[kSG];  // element bits
 };
 // With the fused step-size projection: the tile's dt^T operand in place of
 // the delta row piece.
 template <typename T>
-struct WsRows<T, true> {
+struct WsRows<T, 1, true> {
   typename Raw4<T>::type u, z;
-  uint32_t B, C;
+  uint32_t B[1], C[1];
   u32x4_v pa[kDtK];
 };
 
@@ -594,7 +431,12 @@ struct WsRows<T, true> {
 // kDt (1, or 2 to also store delta_raw to dtp.delta_out): delta_raw from the
 // fused step-size projection (DtProj) instead of dl, and B / C from the token
 // rows of dtp.params instead of Bp / Cp.
-template <typename T, int kZ, bool kAligned, bool kSum, int kDt = 0>
+//
+// kSG: state pairs of a consumer wave, for up to 16 kSG states (wave w: pairs
+// g * 8 + w, g < kSG).  The staged tile, its softplus and the finish serve all
+// of them, so a tile of 64 states costs the producers what one of 16 does,
+// and the consumers reuse each delta / delta*u read kSG times.
+template <typename T, int kSG, int kZ, bool kAligned, bool kSum, int kDt = 0>
 __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
     const ScanDims p, const T* __restrict__ u, const T* __restrict__ dl,
     const float* __restrict__ Ap, const T* __restrict__ Bp, const T* __restrict__ Cp,
@@ -606,6 +448,10 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
   static_assert(!kSum || kZ == 0, "the summaries read no gate");
   static_assert(!kDt || sizeof(T) == 2, "the fused projection reads bf16");
   static_assert(kDt != 2 || !kSum, "the summaries store no delta_raw");
+  static_assert(!kDt || kSG == 1, "the fused projection takes 16 states");
+  // producer register ring: with more pairs a tile takes kSG times as long,
+  // so two tiles ahead cover the loads and leave registers for B and C
+  constexpr int kRing = kSG > 1 ? 2 : kWsRing;
   constexpr bool kDtOut = kDt == 2;
   constexpr bool kHasZ = kZ != 0;
   constexpr bool kSaveY = kZ == 2;
@@ -613,7 +459,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
 
   // [buffer][delta | delta * u][column][channel row]
   __shared__ float4 sSt[kWsStage][2][kT4][kWsRow];
-  __shared__ float4 sBC[kWsStage][kWsCons][kWsTile];       // (B0, C0, B1, C1) per pair and step
+  __shared__ float4 sBC[kWsStage][kSG * kWsCons][kWsTile]; // (B0, C0, B1, C1) per pair and step
   __shared__ float4 sY[2][kWsCons][kT4][kWsRow];           // per-wave partial sums of C*h
   // aligned rows: each producer wave's outputs of four tiles (its 16 rows x
   // 64 steps: one 128-byte line per row in bf16, two in fp32), as pieces of
@@ -645,36 +491,44 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
     // ------------------------------------------------ consumer: the recurrence
     const int ch = d0 + lane;
     const bool ch_ok = ch < Dm;
-    float h[2], A2[2];
+    float h[kSG][2], A2[kSG][2];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int n = 2 * w + s;
-      const bool ok = ch_ok && n < N;
-      A2[s] = ok ? Ap[(size_t)ch * N + n] * kLog2e : 0.0f;
-      float hv = (!kSum && ok && h_init) ? h_init[(rb + ch) * N + n] : 0.0f;
-      // carry in through the earlier summaries' affine maps, in order
-      if (!kSum && ok)
-        hv = fold_carry(hv, A2[s], seg_dt, seg_h, 0, 1, seg * p.sub_k, p.batch, b, Dm, N, n, ch);
-      h[s] = hv;
-    }
+    for (int g = 0; g < kSG; ++g)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int n = 2 * (g * kWsCons + w) + s;
+        const bool ok = ch_ok && n < N;
+        A2[g][s] = ok ? Ap[(size_t)ch * N + n] * kLog2e : 0.0f;
+        float hv = (!kSum && ok && h_init) ? h_init[(rb + ch) * N + n] : 0.0f;
+        // carry in through the earlier summaries' affine maps, in order
+        if (!kSum && ok && kSG == 1)
+          hv = fold_carry(hv, A2[g][s], seg_dt, seg_h, 0, 1, seg * p.sub_k, p.batch, b, Dm, N, n, ch);
+        h[g][s] = hv;
+      }
+    if constexpr (!kSum && kSG > 1)
+      fold_carry_pairs<kSG>(h, A2, seg_dt, seg_h, 0, 1, seg * p.sub_k, p.batch, b, Dm, N, 2 * w, ch,
+                            ch_ok);
     const bool save = !kSum && h_chunks != nullptr;
     const size_t hsD = (size_t)p.hs * Dm;  // floats between the saved rows of two states
     const size_t cstride = (size_t)N * hsD;  // floats between the saves of two chunks
-    // the saves go through a buffer range over the wave's two state rows of
-    // the chunk: lanes past the last channel, and a second state past N,
-    // get offsets outside it (the launch keeps 2 * hsD * 4 bytes < 2^31)
+    // the saves go through buffer ranges over a pair's state rows below N of
+    // the chunk: lanes past the last channel, and a second state past N, get
+    // offsets outside it (the launch keeps 2 * hsD * 4 bytes < 2^31)
     float* const hc0 = save ? h_chunks + ((size_t)b * p.nchunks + Tbeg / kChunk) * cstride +
                                   (size_t)(2 * w) * hsD
                             : nullptr;
-    const bool ok0 = ch_ok && 2 * w < N, ok1 = ch_ok && 2 * w + 1 < N;
-    const uint32_t hoff0 = ok0 ? (uint32_t)ch * 4u : kOffDrop;
-    const uint32_t hoff1 = ok1 ? (uint32_t)(hsD + ch) * 4u : kOffDrop;
+    const uint32_t hoff0 = ch_ok ? (uint32_t)ch * 4u : kOffDrop;
+    const uint32_t hoff1 = ch_ok ? (uint32_t)(hsD + ch) * 4u : kOffDrop;
 
-    // block 0 of a tile: read at the end of the previous tile
+    // stage st = k * kSG + g of a tile: block k (4 steps) of pair g; the B/C
+    // of stage 0 and the delta and delta*u of block 0 are read at the end of
+    // the previous tile
     BC2 bcb[2];
     float4 dlb[2], dub[2];
-    auto read_block = [&](int buf, int k, BC2& bc, float4& dl4, float4& du4) {
-      lds_bc_block(sBC[buf][w], 4 * k, bc);
+    auto read_bc = [&](int buf, int k, int g, BC2& bc) {
+      lds_bc_block(sBC[buf][g * kWsCons + w], 4 * k, bc);
+    };
+    auto read_steps = [&](int buf, int k, float4& dl4, float4& du4) {
       const float4* __restrict__ st = &sSt[buf][0][0][lane];
       dl4 = st[k * kWsRow];
       du4 = st[(kT4 + k) * kWsRow];
@@ -685,43 +539,63 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
     for (int i = 0; i < nbar; ++i) {
       __syncthreads();
       if (i >= ntiles) continue;
-      if (i == 0) read_block(0, 0, bcb[0], dlb[0], dub[0]);
+      if (i == 0) {
+        read_bc(0, 0, 0, bcb[0]);
+        read_steps(0, 0, dlb[0], dub[0]);
+      }
       const int nbuf = buf == kWsStage - 1 ? 0 : buf + 1;
       float4* __restrict__ cY = &sY[i & 1][w][0][lane];
-      // block k+1's LDS reads are issued before block k is computed; after
-      // the last block, the next tile's first block (staged one iteration
-      // ago, so complete since this tile's barrier)
+      // the next stage's LDS reads are issued before a stage is computed;
+      // after the last one, the next tile's first (staged one iteration ago,
+      // so complete since this tile's barrier)
 #pragma unroll
       for (int k = 0; k < kT4; ++k) {
-        const int c = k & 1;
-        if (k + 1 < kT4) read_block(buf, k + 1, bcb[c ^ 1], dlb[c ^ 1], dub[c ^ 1]);
-        else read_block(nbuf, 0, bcb[c ^ 1], dlb[c ^ 1], dub[c ^ 1]);
-        if constexpr (kSum) {
-          fwd_block_state(dlb[c], dub[c], bcb[c], A2, h);
-        } else {
-          float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-          fwd_block(dlb[c], dub[c], bcb[c], A2, h, y);
-          cY[k * kWsRow] = make_float4(y[0], y[1], y[2], y[3]);
+        float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int g = 0; g < kSG; ++g) {
+          const int c = (k * kSG + g) & 1;
+          if (g + 1 < kSG) {
+            read_bc(buf, k, g + 1, bcb[c ^ 1]);
+          } else if (k + 1 < kT4) {
+            read_bc(buf, k + 1, 0, bcb[c ^ 1]);
+            read_steps(buf, k + 1, dlb[(k + 1) & 1], dub[(k + 1) & 1]);
+          } else {
+            read_bc(nbuf, 0, 0, bcb[c ^ 1]);
+            read_steps(nbuf, 0, dlb[0], dub[0]);
+          }
+          if constexpr (kSum) fwd_block_state(dlb[k & 1], dub[k & 1], bcb[c], A2[g], h[g]);
+          else fwd_block(dlb[k & 1], dub[k & 1], bcb[c], A2[g], h[g], y);
         }
+        if constexpr (!kSum) cY[k * kWsRow] = make_float4(y[0], y[1], y[2], y[3]);
       }
-      // kT4 is even: the next tile's block 0 sits in buffer 0 again
+      // kT4 is even: the next tile's first stage and block sit in set 0 again
       static_assert(kT4 % 2 == 0, "block 0 of every tile in register set 0");
       if (save) {
         // layout (batch, nchunks, nstate, dim): one contiguous 256 B run per
         // state; nontemporal, as the backward alone reads the saved states
-        const auto hr = raw_rsrc(hc0 + (size_t)i * cstride, (uint32_t)(2 * hsD * sizeof(float)));
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(h[0]), hr, (int)hoff0, 0, kCacheNT);
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(h[1]), hr, (int)hoff1, 0, kCacheNT);
+#pragma unroll
+        for (int g = 0; g < kSG; ++g) {
+          const int rows = min(max(N - 2 * (g * kWsCons + w), 0), 2);
+          const auto hr = raw_rsrc(hc0 + (size_t)i * cstride + (size_t)(2 * kWsCons * g) * hsD,
+                                   (uint32_t)(rows * hsD * sizeof(float)));
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(h[g][0]), hr, (int)hoff0, 0, kCacheNT);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(h[g][1]), hr, (int)hoff1, 0, kCacheNT);
+        }
       }
       buf = nbuf;
     }
-    if constexpr (kSum) {
-      if (ok0) seg_h[(sb * N + 2 * w) * Dm + ch] = h[0];
-      if (ok1) seg_h[(sb * N + 2 * w + 1) * Dm + ch] = h[1];
-    } else if (!save && h_last && Lend == L) {
-      if (ok0) h_last[(rb + ch) * N + 2 * w] = h[0];
-      if (ok1) h_last[(rb + ch) * N + 2 * w + 1] = h[1];
-    }
+#pragma unroll
+    for (int g = 0; g < kSG; ++g)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int n = 2 * (g * kWsCons + w) + s;
+        if (!ch_ok || n >= N) continue;
+        if constexpr (kSum) {
+          seg_h[(sb * N + n) * Dm + ch] = h[g][s];
+        } else if (!save && h_last && Lend == L) {
+          h_last[(rb + ch) * N + n] = h[g][s];
+        }
+      }
     return;
   }
 
@@ -758,11 +632,10 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
   const int bc_half = kDt ? lane & 1 : pt / (kWsCons * kWsTile);
   const int bc_G = kDt ? (lane >> 1) & 7 : (pt / kWsTile) % kWsCons;
   const int bc_step = kDt ? (w - kWsCons) * 4 + (lane >> 4) : pt % kWsTile;
-  const int bc_n = 2 * bc_G + bc_half;
-  const bool bc_ok = bc_n < N;
-  const size_t bc_row = (size_t)b * p.bc_bstride + (size_t)min(bc_n, N - 1) * L;
-  const T* __restrict__ B_row = Bp + bc_row;
-  const T* __restrict__ C_row = Cp + bc_row;
+  // (state of pair group g; clamped into the rows, zeroed at staging past N)
+  auto bc_n = [&](int g) { return 2 * (g * kWsCons + bc_G) + bc_half; };
+  const T* __restrict__ B_rows = Bp + (size_t)b * p.bc_bstride;
+  const T* __restrict__ C_rows = Cp + (size_t)b * p.bc_bstride;
 
   // raw rows of tile i (clamped to the last tile; the loads of tiles past it
   // are never used)
@@ -783,7 +656,10 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
   const uint32_t bc_bytes = (uint32_t)((size_t)N * L * sizeof(T));
   const auto B_ld = raw_rsrc(const_cast<T*>(Bp) + (size_t)b * p.bc_bstride, bc_bytes);
   const auto C_ld = raw_rsrc(const_cast<T*>(Cp) + (size_t)b * p.bc_bstride, bc_bytes);
-  const uint32_t bc_row_off = (uint32_t)((size_t)min(bc_n, N - 1) * L * sizeof(T));
+  uint32_t bc_row_off[kSG];
+#pragma unroll
+  for (int g = 0; g < kSG; ++g)
+    bc_row_off[g] = (uint32_t)((size_t)min(bc_n(g), N - 1) * L * sizeof(T));
 
   // kDt: the batch row's token rows of params (the launch keeps L * P * 2 <
   // 2^31), this lane's byte offsets from a tile's first token row -- its
@@ -801,7 +677,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
   uint32_t pa_off[kDtK] = {}, pbc_off = 0;
   bf16x8_v wdt[kDtK];
   if constexpr (kDt) {
-    pbc_off = (uint32_t)bc_step * prow_bytes + (uint32_t)(dtp.rank + min(bc_n, N - 1)) * 2u;
+    pbc_off = (uint32_t)bc_step * prow_bytes + (uint32_t)(dtp.rank + min(bc_n(0), N - 1)) * 2u;
     const int pw = w - kWsCons;
     const int wch = d0 + 16 * pw + (lane & 15);
     const __hip_bfloat16* wrow =
@@ -817,15 +693,16 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
     }
   }
 
-  auto issue = [&](WsRows<T, kDt != 0>& r, int i) {
+  using Rows = WsRows<T, kSG, kDt != 0>;
+  auto issue = [&](Rows& r, int i) {
     const int t0 = min(Tbeg + i * kWsTile, last_t0);
     if constexpr (kDt) {
       const uint32_t tb = (uint32_t)t0 * prow_bytes;  // wave-uniform
 #pragma unroll
       for (int s = 0; s < kDtK; ++s)
         r.pa[s] = __builtin_amdgcn_raw_buffer_load_b128(pr_ld, (int)(tb + pa_off[s]), 0, 0);
-      r.B = buffer_load_bits1<T>(pr_ld, tb + pbc_off);
-      r.C = buffer_load_bits1<T>(pr_ld, tb + pbc_off + (uint32_t)N * 2u);
+      r.B[0] = buffer_load_bits1<T>(pr_ld, tb + pbc_off);
+      r.C[0] = buffer_load_bits1<T>(pr_ld, tb + pbc_off + (uint32_t)N * 2u);
       if constexpr (kAligned) {
         const uint32_t off = row_off + (uint32_t)min(t0 + 4 * q, L - 4) * sizeof(T);
         r.u = buffer_load_raw4<T>(u_ld, off);
@@ -842,17 +719,23 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
       r.d = buffer_load_raw4<T>(d_ld, off);
       if constexpr (kHasZ) r.z = buffer_load_raw4<T>(z_ld, off);
       else r.z = typename Raw4<T>::type{};
-      const uint32_t boff = bc_row_off + (uint32_t)min(t0 + bc_step, L - 1) * sizeof(T);
-      r.B = buffer_load_bits1<T>(B_ld, boff);
-      r.C = buffer_load_bits1<T>(C_ld, boff);
+#pragma unroll
+      for (int g = 0; g < kSG; ++g) {
+        const uint32_t boff = bc_row_off[g] + (uint32_t)min(t0 + bc_step, L - 1) * sizeof(T);
+        r.B[g] = buffer_load_bits1<T>(B_ld, boff);
+        r.C[g] = buffer_load_bits1<T>(C_ld, boff);
+      }
     } else {
       r.u = load_raw4_nb<T, kAligned>(u_row, t0 + 4 * q, L, pch_ok);
       r.d = load_raw4_nb<T, kAligned>(d_row, t0 + 4 * q, L, pch_ok);
       if constexpr (kHasZ) r.z = load_raw4_nb<T, kAligned>(z_row, t0 + 4 * q, L, pch_ok);
       else r.z = typename Raw4<T>::type{};
-      const int tb = min(t0 + bc_step, L - 1);
-      r.B = elem_bits(B_row[tb]);
-      r.C = elem_bits(C_row[tb]);
+#pragma unroll
+      for (int g = 0; g < kSG; ++g) {
+        const size_t tb = (size_t)min(bc_n(g), N - 1) * L + min(t0 + bc_step, L - 1);
+        r.B[g] = elem_bits(B_rows[tb]);
+        r.C[g] = elem_bits(C_rows[tb]);
+      }
     }
   };
 
@@ -870,7 +753,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
   // kDt: a tile's delta_raw (steps 4 (lane / 16) .. + 3 of channel lane % 16
   // of the wave's 16), issued an iteration before the tile is staged so that
   // the MFMA latency runs under that iteration's other work
-  auto proj = [&](const WsRows<T, kDt != 0>& r) {
+  auto proj = [&](const Rows& r) {
     f32x4_v acc = {0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (kDt) {
 #pragma unroll
@@ -880,7 +763,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
     }
     return acc;
   };
-  auto stage = [&](const WsRows<T, kDt != 0>& r, const f32x4_v acc, int i, int sbuf, float (&sk)[4],
+  auto stage = [&](const Rows& r, const f32x4_v acc, int i, int sbuf, float (&sk)[4],
                    float (&gt)[4], int par) {
     const int t_tile = Tbeg + i * kWsTile;
     const int t = t_tile + 4 * q;
@@ -947,8 +830,11 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
     }
     sSt[sbuf][0][q][row] = make_float4(de[0], de[1], de[2], de[3]);
     sSt[sbuf][1][q][row] = make_float4(du[0], du[1], du[2], du[3]);
-    reinterpret_cast<float2*>(&sBC[sbuf][bc_G][bc_step])[bc_half] =
-        bc_ok ? make_float2(bits_to_f32<T>(r.B), bits_to_f32<T>(r.C)) : make_float2(0.0f, 0.0f);
+#pragma unroll
+    for (int g = 0; g < kSG; ++g)
+      reinterpret_cast<float2*>(&sBC[sbuf][g * kWsCons + bc_G][bc_step])[bc_half] =
+          bc_n(g) < N ? make_float2(bits_to_f32<T>(r.B[g]), bits_to_f32<T>(r.C[g]))
+                      : make_float2(0.0f, 0.0f);
   };
 
   const auto out_rsrc = raw_rsrc(out + ((size_t)rb + wrow0) * L, wbytes);
@@ -1051,8 +937,8 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
 
   // Iteration i after barrier i: read tile i-1's slices (written during
   // iteration i-1), stage tile i+2 into buffer (i+2) % 3 (last read during
-  // iteration i-1), finish tile i-1.  Raw rows travel in a ring of kWsRing
-  // tiles: tile k's loads are issued when tile k - kWsRing is staged, kWsRing
+  // iteration i-1), finish tile i-1.  Raw rows travel in a ring of kRing
+  // tiles: tile k's loads are issued when tile k - kRing is staged, kRing
   // iterations ahead of their use.  D*u and the gates ride in a ring of 4
   // tiles (staged at iteration k - 2, finished at k + 1).
   //
@@ -1062,19 +948,19 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
   // into the loop header makes it wait for nearly all of them).  Work past
   // the last tile is harmless: its loads are clamped into the rows, its
   // staging buffers are never read and its stores fall outside the range.
-  WsRows<T, kDt != 0> rows[kWsRing];
+  Rows rows[kRing];
   float sk[4][4], gt[4][4];
   float4 v[kWsCons];
 #pragma unroll
-  for (int k = 0; k < kWsRing; ++k) issue(rows[k], k);
+  for (int k = 0; k < kRing; ++k) issue(rows[k], k);
   stage(rows[0], proj(rows[0]), 0, 0, sk[0], gt[0], 0);
-  issue(rows[0], kWsRing);
+  issue(rows[0], kRing);
   stage(rows[1], proj(rows[1]), 1, 1, sk[1], gt[1], 1);
-  issue(rows[1], kWsRing + 1);
+  issue(rows[1], kRing + 1);
   __syncthreads();  // iteration 0
-  stage(rows[2], proj(rows[2]), 2, 2, sk[2], gt[2], 0);
-  issue(rows[2], kWsRing + 2);
-  f32x4_v dacc = proj(rows[3]);  // kDt: tile 3, staged at iteration 1
+  stage(rows[2 % kRing], proj(rows[2 % kRing]), 2, 2, sk[2], gt[2], 0);
+  issue(rows[2 % kRing], kRing + 2);
+  f32x4_v dacc = proj(rows[3 % kRing]);  // kDt: tile 3, staged at iteration 1
   int sbuf = 0;  // staging buffer of tile i + 2
   for (int i0 = 1; i0 <= ntiles; i0 += 4) {
 #pragma unroll
@@ -1083,9 +969,9 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
       __syncthreads();
       if constexpr (!kSum) finish_read(i - 1, v);
       // i0 % 4 == 1, so tile i + 2 has the parity of j + 3
-      stage(rows[(j + 3) % kWsRing], dacc, i + 2, sbuf, sk[(j + 3) & 3], gt[(j + 3) & 3],
+      stage(rows[(j + 3) % kRing], dacc, i + 2, sbuf, sk[(j + 3) & 3], gt[(j + 3) & 3],
             (j + 3) & 1);
-      issue(rows[(j + 3) % kWsRing], i + 2 + kWsRing);
+      issue(rows[(j + 3) % kRing], i + 2 + kRing);
       if constexpr (!kSum) {
         if constexpr (kAligned) {
           finish_lds(i - 1, v, sk[j], gt[j], j);
@@ -1094,8 +980,8 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
           finish(i - 1, v, sk[j], gt[j]);
         }
       }
-      // tile i + 3 sits in ring slot (i + 3) % 4 == j
-      dacc = proj(rows[j]);
+      // tile i + 3 sits in ring slot (i + 3) % 4 == j (kDt: kRing is 4)
+      if constexpr (kDt != 0) dacc = proj(rows[j % kRing]);
       sbuf = sbuf == kWsStage - 1 ? 0 : sbuf + 1;
     }
   }
@@ -1126,17 +1012,17 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
 // stages delta and delta*u in LDS (double-buffered by tile parity, so one
 // barrier per tile suffices), phase B runs the recurrence with B read as
 // wave-uniform values of the prepped layout.
-template <typename T, int kSG, bool kAligned>
+template <typename T, bool kAligned>
 __global__ __launch_bounds__(kThreads) void scan_fwd_segsum_kernel(
     const ScanDims p, const T* __restrict__ u, const T* __restrict__ dl,
     const float* __restrict__ Ap, const float* __restrict__ bc, const float* __restrict__ biasp,
     const int64_t* __restrict__ length, float* __restrict__ seg_h, float* __restrict__ seg_dt) {
   using R4 = typename Raw4<T>::type;
+  constexpr int kSG = kGenSG;
   constexpr int kT4 = kTileF / 4;
   static_assert(kBlockCh * kT4 == kThreads, "one 4-step row piece per thread");
   __shared__ float4 sDelta[2][kT4][kBlockCh];
   __shared__ float4 sDu[2][kT4][kBlockCh];
-  __shared__ float4 sB[2][kWaves][kTileF / 2];  // (B0, B1) of steps 2i, 2i+1 per pair
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1180,16 +1066,8 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_segsum_kernel(
   const float4* __restrict__ bc4 = reinterpret_cast<const float4*>(bc);
   float dtsum = 0.0f;
 
-  // B staging (kSG == 1): thread tid < 256 owns (pair tid / 32, step tid % 32)
-  const int bc_G = (tid / kTileF) % kWaves;
-  const int bc_t = tid % kTileF;
-  auto load_b = [&](int T0) {
-    const int t = min(T0 + bc_t, Lp - 1);
-    return bc4[((size_t)b * npair + bc_G) * Lp + t];
-  };
   R4 qu = load_raw4_nb<T, kAligned>(u_row, Tbeg + a_col, L, a_ok);
   R4 qd = load_raw4_nb<T, kAligned>(d_row, Tbeg + a_col, L, a_ok);
-  float4 qb = kSG == 1 ? load_b(Tbeg) : make_float4(0.f, 0.f, 0.f, 0.f);
   int buf = 0;
   for (int T0 = Tbeg; T0 < Lend; T0 += kTileF) {
     {
@@ -1208,50 +1086,13 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_segsum_kernel(
       }
       sDelta[buf][a_q][a_sw] = make_float4(de[0], de[1], de[2], de[3]);
       sDu[buf][a_q][a_sw] = make_float4(du[0], du[1], du[2], du[3]);
-      if (kSG == 1 && tid < kWaves * kTileF) {
-        // (B0, B1) of this step into the pair's row: two steps per float4
-        float* row = reinterpret_cast<float*>(&sB[buf][bc_G][0]);
-        row[2 * bc_t] = qb.x;
-        row[2 * bc_t + 1] = qb.z;
-      }
     }
     // next tile's rows (the last tile re-reads itself)
     const int Tn = min(T0 + kTileF, last_t0);
     qu = load_raw4_nb<T, kAligned>(u_row, Tn + a_col, L, a_ok);
     qd = load_raw4_nb<T, kAligned>(d_row, Tn + a_col, L, a_ok);
-    if constexpr (kSG == 1) qb = load_b(Tn);
     __syncthreads();
     const int nT4 = min(kT4, (Lend - T0 + 3) / 4);
-    if (kSG == 1 && nT4 == kT4) {
-      // full tile: 8 blocks unrolled, each block's LDS reads one block ahead
-      const float4* __restrict__ bro = sB[buf][w];
-      float4 dlb[2], dub[2], bb[2][2];
-      dlb[0] = sDelta[buf][0][lane ^ col_swz(0)];
-      dub[0] = sDu[buf][0][lane ^ col_swz(0)];
-      bb[0][0] = bro[0];
-      bb[0][1] = bro[1];
-#pragma unroll
-      for (int k = 0; k < kT4; ++k) {
-        const int c = k & 1;
-        if (k + 1 < kT4) {
-          dlb[c ^ 1] = sDelta[buf][k + 1][lane ^ col_swz(k + 1)];
-          dub[c ^ 1] = sDu[buf][k + 1][lane ^ col_swz(k + 1)];
-          bb[c ^ 1][0] = bro[2 * (k + 1)];
-          bb[c ^ 1][1] = bro[2 * (k + 1) + 1];
-        }
-        const float dlv[4] = {dlb[c].x, dlb[c].y, dlb[c].z, dlb[c].w};
-        const float duv[4] = {dub[c].x, dub[c].y, dub[c].z, dub[c].w};
-        const float b0[4] = {bb[c][0].x, bb[c][0].z, bb[c][1].x, bb[c][1].z};
-        const float b1[4] = {bb[c][0].y, bb[c][0].w, bb[c][1].y, bb[c][1].w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          h[0][0] = fmaf(fast_exp2(dlv[j] * A2[0][0]), h[0][0], duv[j] * b0[j]);
-          h[0][1] = fmaf(fast_exp2(dlv[j] * A2[0][1]), h[0][1], duv[j] * b1[j]);
-        }
-      }
-      buf ^= 1;
-      continue;
-    }
     for (int t4 = 0; t4 < nT4; ++t4) {
       const float4 dl4 = sDelta[buf][t4][lane ^ col_swz(t4)];
       const float4 du4 = sDu[buf][t4][lane ^ col_swz(t4)];
@@ -1495,77 +1336,74 @@ hipError_t launch_bc_prep(const ScanParams& p, int dtype, float* bc, hipStream_t
   return hipGetLastError();
 }
 
-// The role-split forward serves N <= 16 when its buffer ranges fit 2^31
-// bytes (a wave's 16 rows of output, 16 * L * elem, and a wave's two saved
-// state rows, 2 * hs * dim * 4); the general kernel serves the rest.
+// The role-split forward serves N <= 64 when its buffer ranges fit 2^31
+// bytes (a wave's 16 rows of output, 16 * L * elem, a batch row's B or C, and
+// a pair's two saved state rows, 2 * hs * dim * 4); the general kernel serves
+// the rest.
 static bool ws_forward(const ScanParams& p, size_t elem) {
-  return p.nstate <= 16 && (size_t)(kBlockCh / kWsProd) * p.seqlen * elem < (1u << 31) &&
+  return p.nstate <= 64 && (size_t)p.nstate * p.seqlen * elem < (1u << 31) &&
+         (size_t)(kBlockCh / kWsProd) * p.seqlen * elem < (1u << 31) &&
          (size_t)2 * p.hs * p.dim * sizeof(float) < (1u << 31);
 }
 
 template <typename T, int kSG, int kZ, bool kAligned>
-static hipError_t launch_fwd4(const ScanParams& p, const float* bc, hipStream_t st) {
-  const bool ws = ws_forward(p, sizeof(T));
+static hipError_t launch_ws(const ScanParams& p, hipStream_t st) {
   if (p.nseg > 1) {
     ProfScope prof("scan_fwd_segsum", st);
-    if (ws)
-      hipLaunchKernelGGL((scan_fwd_ws_kernel<T, 0, kAligned, true>),
-                         dim3(p.nblk, p.batch, (p.nseg - 1) * p.sub_k), dim3(kWsThreads), 0, st,
-                         dims_of(p), (const T*)p.u, (const T*)p.delta, p.A, (const T*)p.B,
-                         (const T*)p.C, p.D, p.bias, p.h_init, p.length, (const T*)nullptr,
-                         (T*)p.out, (T*)nullptr, (float*)nullptr, (float*)nullptr, p.dummy,
-                         p.seg_h, p.seg_dt, DtProj{});
-    else
-      hipLaunchKernelGGL((scan_fwd_segsum_kernel<T, kSG, kAligned>),
-                         dim3(p.nblk, p.batch, (p.nseg - 1) * p.sub_k), dim3(kThreads), 0, st,
-                         dims_of(p),
-                         (const T*)p.u, (const T*)p.delta, p.A, bc, p.bias, p.length, p.seg_h,
-                         p.seg_dt);
+    hipLaunchKernelGGL((scan_fwd_ws_kernel<T, kSG, 0, kAligned, true>),
+                       dim3(p.nblk, p.batch, (p.nseg - 1) * p.sub_k), dim3(kWsThreads), 0, st,
+                       dims_of(p), (const T*)p.u, (const T*)p.delta, p.A, (const T*)p.B,
+                       (const T*)p.C, p.D, p.bias, p.h_init, p.length, (const T*)nullptr,
+                       (T*)p.out, (T*)nullptr, (float*)nullptr, (float*)nullptr, p.dummy,
+                       p.seg_h, p.seg_dt, DtProj{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   ProfScope prof("scan_fwd", st);
-  if (ws) {
-    hipLaunchKernelGGL((scan_fwd_ws_kernel<T, kZ, kAligned, false>), dim3(p.nblk, p.batch, p.nseg),
-                       dim3(kWsThreads), 0, st, dims_of(p), (const T*)p.u, (const T*)p.delta, p.A,
-                       (const T*)p.B, (const T*)p.C, p.D, p.bias, p.h_init, p.length,
-                       (const T*)p.z, (T*)p.out, (T*)p.out_ungated, p.h_chunks, p.h_last, p.dummy,
-                       p.seg_h, p.seg_dt, DtProj{});
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL((scan_fwd_kernel<T, kSG, kZ, kAligned>),
-                     dim3(p.nblk, p.batch, p.nseg), dim3(kThreads), 0, st, dims_of(p),
-                     (const T*)p.u, (const T*)p.delta, p.A, bc, (const T*)p.B, (const T*)p.C, p.D,
+  hipLaunchKernelGGL((scan_fwd_ws_kernel<T, kSG, kZ, kAligned, false>),
+                     dim3(p.nblk, p.batch, p.nseg), dim3(kWsThreads), 0, st, dims_of(p),
+                     (const T*)p.u, (const T*)p.delta, p.A, (const T*)p.B, (const T*)p.C, p.D,
                      p.bias, p.h_init, p.length, (const T*)p.z, (T*)p.out, (T*)p.out_ungated,
-                     p.h_chunks, p.h_last, p.dummy, p.seg_h, p.seg_dt);
+                     p.h_chunks, p.h_last, p.dummy, p.seg_h, p.seg_dt, DtProj{});
   return hipGetLastError();
 }
 
-template <typename T, int kSG>
-static hipError_t launch_fwd3(const ScanParams& p, const float* bc, bool aligned, hipStream_t st) {
-  if (p.z && p.out_ungated)
-    return aligned ? launch_fwd4<T, kSG, 2, true>(p, bc, st)
-                   : launch_fwd4<T, kSG, 2, false>(p, bc, st);
-  if (p.z)
-    return aligned ? launch_fwd4<T, kSG, 1, true>(p, bc, st)
-                   : launch_fwd4<T, kSG, 1, false>(p, bc, st);
-  return aligned ? launch_fwd4<T, kSG, 0, true>(p, bc, st)
-                 : launch_fwd4<T, kSG, 0, false>(p, bc, st);
+// The role-split kernel by state count: 16 (one pair a wave), 32 or 64.
+template <typename T, int kZ, bool kAligned>
+static hipError_t launch_fwd4(const ScanParams& p, const float* bc, hipStream_t st) {
+  if (ws_forward(p, sizeof(T))) {
+    if (p.nstate <= 16) return launch_ws<T, 1, kZ, kAligned>(p, st);
+    if (p.nstate <= 32) return launch_ws<T, 2, kZ, kAligned>(p, st);
+    return launch_ws<T, 4, kZ, kAligned>(p, st);
+  }
+  if (p.nseg > 1) {
+    ProfScope prof("scan_fwd_segsum", st);
+    hipLaunchKernelGGL((scan_fwd_segsum_kernel<T, kAligned>),
+                       dim3(p.nblk, p.batch, (p.nseg - 1) * p.sub_k), dim3(kThreads), 0, st,
+                       dims_of(p), (const T*)p.u, (const T*)p.delta, p.A, bc, p.bias, p.length,
+                       p.seg_h, p.seg_dt);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  ProfScope prof("scan_fwd", st);
+  hipLaunchKernelGGL((scan_fwd_kernel<T, kZ, kAligned>), dim3(p.nblk, p.batch, p.nseg),
+                     dim3(kThreads), 0, st, dims_of(p), (const T*)p.u, (const T*)p.delta, p.A, bc,
+                     p.D, p.bias, p.h_init, p.length, (const T*)p.z, (T*)p.out,
+                     (T*)p.out_ungated, p.h_chunks, p.h_last, p.seg_h, p.seg_dt);
+  return hipGetLastError();
 }
 
 template <typename T>
 static hipError_t launch_fwd2(const ScanParams& p, const float* bc, bool aligned, hipStream_t st) {
-  if (p.nstate <= 16) return launch_fwd3<T, 1>(p, bc, aligned, st);
-  if (p.nstate <= 32) return launch_fwd3<T, 2>(p, bc, aligned, st);
-  if (p.nstate <= 64) return launch_fwd3<T, 4>(p, bc, aligned, st);
-  return launch_fwd3<T, 16>(p, bc, aligned, st);
+  if (p.z && p.out_ungated)
+    return aligned ? launch_fwd4<T, 2, true>(p, bc, st) : launch_fwd4<T, 2, false>(p, bc, st);
+  if (p.z) return aligned ? launch_fwd4<T, 1, true>(p, bc, st) : launch_fwd4<T, 1, false>(p, bc, st);
+  return aligned ? launch_fwd4<T, 0, true>(p, bc, st) : launch_fwd4<T, 0, false>(p, bc, st);
 }
 
-// The prepped B/C layout serves state counts past 16 and the general
-// kernel's segment summaries; the role-split kernels read B and C directly.
-static bool fwd_needs_bc_prep(const ScanParams& p, size_t elem) {
-  return p.nstate > 16 || (p.nseg > 1 && !ws_forward(p, elem));
-}
+// The prepped B/C layout serves the general kernels; the role-split kernels
+// read B and C directly.
+static bool fwd_needs_bc_prep(const ScanParams& p, size_t elem) { return !ws_forward(p, elem); }
 
 // bc must hold bc_prep_floats() floats; it is filled here before the scan
 // when a kernel reads the prepped layout.
@@ -1589,7 +1427,7 @@ static void launch_ws_dt(const ScanParams& p, const DtProj& dt, hipStream_t st) 
   using T = __hip_bfloat16;
   const int gz = kSum ? (p.nseg - 1) * p.sub_k : p.nseg;
   const T* prm = static_cast<const T*>(dt.params);
-  hipLaunchKernelGGL((scan_fwd_ws_kernel<T, kZ, kAligned, kSum, kDt>), dim3(p.nblk, p.batch, gz),
+  hipLaunchKernelGGL((scan_fwd_ws_kernel<T, 1, kZ, kAligned, kSum, kDt>), dim3(p.nblk, p.batch, gz),
                      dim3(kWsThreads), 0, st, dims_of(p), (const T*)p.u, (const T*)p.u, p.A, prm,
                      prm, p.D, p.bias, p.h_init, p.length, (const T*)p.z, (T*)p.out,
                      (T*)nullptr, (float*)nullptr, p.h_last, p.dummy, p.seg_h, p.seg_dt, dt);

@@ -111,6 +111,42 @@ __device__ __forceinline__ float fold_carry(float x, float A2, const float* __re
   }
   return x;
 }
+
+// The same for the 2 kSG states n0 + 16 g + s (g < kSG, s < 2) of a wave:
+// each summary's step sum is read once and four summaries' loads for every
+// state are in flight together (state by state, eight states would wait for
+// memory eight times as often).  States past N and channels past the last
+// read clamped addresses and keep their value.
+template <int kSG>
+__device__ __forceinline__ void fold_carry_pairs(float (&x)[kSG][2], const float (&A2)[kSG][2],
+                                                 const float* __restrict__ dtp,
+                                                 const float* __restrict__ gp, int k_first, int step,
+                                                 int count, int batch, int b, int Dm, int N, int n0,
+                                                 int ch, bool ch_ok) {
+  constexpr int kIn = 4;
+  const int chc = min(ch, Dm - 1);
+  for (int c0 = 0; c0 < count; c0 += kIn) {
+    float dt[kIn], gv[kIn][kSG][2];
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) {
+      const size_t kb = (size_t)(k_first + step * min(c0 + u, count - 1)) * batch + b;
+      dt[u] = dtp[kb * Dm + chc];
+#pragma unroll
+      for (int g = 0; g < kSG; ++g)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          gv[u][g][s] = gp[(kb * N + min(n0 + 16 * g + s, N - 1)) * Dm + chc];
+    }
+#pragma unroll
+    for (int u = 0; u < kIn; ++u)
+#pragma unroll
+      for (int g = 0; g < kSG; ++g)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          if (c0 + u < count && ch_ok && n0 + 16 * g + s < N)
+            x[g][s] = fmaf(fast_exp2(A2[g][s] * dt[u]), x[g][s], gv[u][g][s]);
+  }
+}
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 

@@ -24,7 +24,7 @@ constexpr int kTileB = 16;    // steps staged through LDS per backward tile
 constexpr int kBlockCh = 64;  // channels per workgroup (one per lane)
 constexpr int kWaves = 8;     // waves per workgroup; wave w owns state pairs G = g*8 + w
 constexpr int kThreads = 64 * kWaves;
-// role-split kernels (N <= 16): consumer waves run the recurrences, producer
+// role-split kernels (N <= 64): consumer waves run the recurrences, producer
 // waves stage tiles and finish per-position outputs
 constexpr int kWsCons = 8;    // consumer waves: state pair w
 constexpr int kWsProd = 4;    // producer waves: (channel row, 4-step column) per lane

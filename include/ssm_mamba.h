@@ -232,6 +232,44 @@ int ssm_rms_norm_cm(int64_t batch, int64_t channels, int64_t seqlen, int dtype, 
                     const void* weight, float eps, void* out, void* stream);
 
 /*
+ * The RMSNorm in front of a Mamba block (modules/rms_norm.py:11-31 at
+ * modules/block.py:78-90) from the reference's token-major layout to the
+ * channel-major one in one pass: x (batch, seqlen, channels) ->
+ *   h_cm[b, c, t] = x[b, t, c] * rstd[b, t] * (1 + weight[c]),
+ *   rstd[b, t] = rsqrt(mean_c x[b, t, c]^2 + eps)
+ * with h_tm (batch, seqlen, channels; nullable) the same values token-major and
+ * rstd (batch, seqlen; nullable) fp32, for the backward.  channels a multiple
+ * of 16 bytes of elements, at most 2048 (bf16) or 1024 (fp32); x, weight and
+ * h_tm 16-byte aligned.
+ */
+int ssm_rms_norm_tc_fwd(int64_t batch, int64_t seqlen, int64_t channels, int dtype, const void* x,
+                        const void* weight, float eps, void* h_cm, void* h_tm, float* rstd,
+                        void* stream);
+
+/* Device workspace (bytes) for ssm_rms_norm_tc_bwd. */
+size_t ssm_rms_norm_tc_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t channels);
+
+/*
+ * Backward of ssm_rms_norm_tc_fwd for the upstream gradient dh_cm (batch,
+ * channels, seqlen): dx (batch, seqlen, channels), with dres (the same shape;
+ * nullable) added, and dweight (channels), summed in a fixed order.
+ */
+int ssm_rms_norm_tc_bwd(int64_t batch, int64_t seqlen, int64_t channels, int dtype, const void* x,
+                        const void* weight, const float* rstd, const void* dh_cm, const void* dres,
+                        void* dx, void* dweight, void* workspace, size_t workspace_bytes,
+                        void* stream);
+
+/* out (batch, cols, rows) = the transposed matrices of in (batch, rows, cols),
+ * each contiguous and in_batch_stride elements apart (0: rows * cols). */
+int ssm_transpose(int64_t batch, int64_t rows, int64_t cols, int dtype, const void* in,
+                  int64_t in_batch_stride, void* out, void* stream);
+
+/* out (rows, cols), or (cols, rows) when transposed = the sum over the batch of
+ * in (batch, rows, cols), added in fp32 in batch order and rounded once. */
+int ssm_batch_sum(int64_t batch, int64_t rows, int64_t cols, int dtype, const void* in,
+                  int transposed, void* out, void* stream);
+
+/*
  * Causal depthwise conv1d (+ SiLU) over channel-major rows: the prefill
  * convolution of the Mamba layer, nn.Conv1d(dim, dim, width, groups=dim,
  * padding=width-1)(x)[..., :seqlen] followed by F.silu

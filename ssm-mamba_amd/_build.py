@@ -23,7 +23,7 @@ LIB_DIR = os.path.join(PKG_DIR, "_lib")
 LIB_NAME = "libssm_mamba_hip.so"
 LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
 SOURCES = ["scan_fwd.hip", "scan_bwd.hip", "state_update.hip", "conv1d.hip", "decode.hip",
-           "decode_rows.hip", "norm.hip", "capi.hip"]
+           "decode_rows.hip", "layout.hip", "norm.hip", "capi.hip"]
 EXT_DIR = os.path.join(PKG_DIR, "_ext")
 EXT_MODULES = ["selective_scan", "selective_update"]
 EXT_SUFFIX = sysconfig.get_config_var("EXT_SUFFIX") or ".so"

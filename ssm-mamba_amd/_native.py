@@ -133,6 +133,18 @@ SIGNATURES = {
         _p, _i64, _i64, _p,                    # tokens, tokens_ld, tokens_cols, pos
         _p, _i64, _p,                          # workspace, workspace_bytes, stream
     ]),
+    "ssm_rms_norm_tc_fwd": (_i32, [
+        _i64, _i64, _i64, _i32,                # batch, seqlen, channels, dtype
+        _p, _p, ctypes.c_float, _p, _p, _p, _p,  # x, weight, eps, h_cm, h_tm, rstd, stream
+    ]),
+    "ssm_rms_norm_tc_bwd_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "ssm_rms_norm_tc_bwd": (_i32, [
+        _i64, _i64, _i64, _i32,                # batch, seqlen, channels, dtype
+        _p, _p, _p, _p, _p, _p, _p,            # x, weight, rstd, dh_cm, dres, dx, dweight
+        _p, _sz, _p,                           # workspace, bytes, stream
+    ]),
+    "ssm_transpose": (_i32, [_i64, _i64, _i64, _i32, _p, _i64, _p, _p]),
+    "ssm_batch_sum": (_i32, [_i64, _i64, _i64, _i32, _p, _i32, _p, _p]),
     "ssm_rms_norm_cm": (_i32, [
         _i64, _i64, _i64, _i32,                # batch, channels, seqlen, dtype
         _p, _p, ctypes.c_float, _p, _p,        # x, weight, eps, out, stream

@@ -41,6 +41,8 @@ import torch.nn.functional as F
 
 from . import _native as _N
 from . import decode as _dec
+from . import layer_train as _lt
+from . import layout as _lay
 from .causal_conv1d import causal_conv1d_fn
 from .ops import selective_scan_fn, selective_state_update
 
@@ -63,6 +65,15 @@ def _proj_cm(weight: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor]
     if bias is None:
         return torch.bmm(w, x)
     return torch.baddbmm(bias[None, :, None].expand(x.shape[0], weight.shape[0], x.shape[2]), w, x)
+
+
+def _channel_major(x: torch.Tensor) -> torch.Tensor:
+    """x.transpose(1, 2).contiguous() (its own inverse: also channel-major to
+    token-major); without autograd on the GPU one tiled kernel (6.8 us for 16.8
+    MB, against 42 us for torch's strided copy)."""
+    if torch.is_grad_enabled() or x.dim() != 3:
+        return x.transpose(1, 2).contiguous()
+    return _lay.transposed(x)
 
 
 def rms_norm_cm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -296,9 +307,8 @@ class Mamba(nn.Module):
         """hidden_states (batch, seq_len, model_dim) -> ((batch, seq_len,
         model_dim), last_ssm_hiddens (batch, inner, N)), as
         ``modules/mamba.py:82-187``."""
-        y, last = self.forward_cm(hidden_states.transpose(1, 2).contiguous(), ssm_hiddens,
-                                  lengths, use_cache)
-        return y.transpose(1, 2).contiguous(), last
+        y, last = self.forward_cm(_channel_major(hidden_states), ssm_hiddens, lengths, use_cache)
+        return _channel_major(y), last
 
     def forward_cm(self, x: torch.Tensor, ssm_hiddens: Optional[torch.Tensor] = None,
                    lengths: Optional[torch.Tensor] = None, use_cache: bool = False,
@@ -306,6 +316,37 @@ class Mamba(nn.Module):
         """Channel-major forward: x (batch, model_dim, L) -> (batch, model_dim, L)
         (plus ``residual`` when given, added by the out-projection GEMM) and
         the last SSM state."""
+        y, last = self._mix_cm(x, ssm_hiddens, lengths, use_cache)
+        if residual is not None and self.out_proj.bias is None:
+            w = self.out_proj.weight.expand(y.shape[0], *self.out_proj.weight.shape)
+            if residual_inplace:
+                out = residual.baddbmm_(w, y)       # the stream is updated in place
+            else:
+                out = torch.baddbmm(residual, w, y)
+        else:
+            out = _proj_cm(self.out_proj.weight, y, self.out_proj.bias)
+            if residual is not None:
+                out = residual + out
+        return out, last
+
+    def _mix_train(self, xs: torch.Tensor, z: torch.Tensor, ssm_hiddens: Optional[torch.Tensor],
+                   lengths: Optional[torch.Tensor], use_cache: bool):
+        """``_mix_cm`` with autograd from the in-projection's halves on."""
+        window = self._conv_window(xs) if use_cache else None
+        xc = causal_conv_silu(xs, self.conv.weight, self.conv.bias, window=window,
+                              lengths=lengths if use_cache else None)
+        if use_cache:
+            self._conv_context = window
+        A, D, dt_bias = self._scan_params()
+        y, last = _lt.SsmFn.apply(xc, z, self.ssm_param_proj.weight, self.delta_proj.weight, A, D,
+                                  dt_bias, ssm_hiddens, lengths, "left")
+        if use_cache:
+            self._ssm_hiddens = self._keep(self._ssm_hiddens, last.detach())
+        return y, last
+
+    def _mix_cm(self, x: torch.Tensor, ssm_hiddens: Optional[torch.Tensor],
+                lengths: Optional[torch.Tensor], use_cache: bool):
+        """The mixer up to the out-projection: (y (batch, inner, L), last state)."""
         inner, rank, nstate = self.inner_dim, self.delta_rank, self.state_dim
         w_in, b_in = self.input_proj.weight, self.input_proj.bias
         fused = self._dt_fusable(x, ssm_hiddens, lengths)
@@ -340,17 +381,7 @@ class Mamba(nn.Module):
                                         length=lengths, padding_side="left")
         if use_cache:
             self._ssm_hiddens = self._keep(self._ssm_hiddens, last.detach())
-        if residual is not None and self.out_proj.bias is None:
-            w = self.out_proj.weight.expand(y.shape[0], *self.out_proj.weight.shape)
-            if residual_inplace:
-                out = residual.baddbmm_(w, y)       # the stream is updated in place
-            else:
-                out = torch.baddbmm(residual, w, y)
-        else:
-            out = _proj_cm(self.out_proj.weight, y, self.out_proj.bias)
-            if residual is not None:
-                out = residual + out
-        return out, last
+        return y, last
 
     # ---- decode ----------------------------------------------------------
     def step(self, hidden_states: torch.Tensor) -> torch.Tensor:
@@ -415,9 +446,28 @@ class Block(nn.Module):
     def forward(self, hidden_states: torch.Tensor, lengths: Optional[torch.Tensor] = None,
                 ssm_hiddens: Optional[torch.Tensor] = None, use_cache: bool = False):
         """(batch, seq_len, model_dim) -> ((batch, seq_len, model_dim), last state)."""
+        if self._fused(hidden_states):
+            # token-major in and out: the norm kernel writes the channel-major
+            # activations, the out-projection's product the token-major sum
+            drop = self.training and self.dropout.p > 0.0
+            w_out = self.ssm.out_proj.weight
+            if torch.is_grad_enabled():
+                xs, z, x = _lt.NormInProjFn.apply(hidden_states, self.norm.weight,
+                                                  self.ssm.input_proj.weight, self.norm.eps)
+                y, last = self.ssm._mix_train(xs, z, ssm_hiddens, lengths, use_cache)
+                out = _lt.OutProjFn.apply(y, w_out, None if drop else x)
+            else:
+                h, _, _, x = _lay.norm_tc(hidden_states, self.norm.weight, self.norm.eps)
+                y, last = self.ssm._mix_cm(h, ssm_hiddens, lengths, use_cache)
+                out = _lt.out_proj(y, w_out, None if drop else x)
+            return (x + self.dropout(out) if drop else out), last
         y, last = self.forward_cm(hidden_states.transpose(1, 2).contiguous(), lengths,
                                   ssm_hiddens, use_cache)
         return y.transpose(1, 2).contiguous(), last
+
+    def _fused(self, x: torch.Tensor) -> bool:
+        """Whether ``forward`` of token-major x runs on the fused layer kernels."""
+        return _dec.plain(self.norm, RMSNorm) and _lt.supported(self, x)
 
     def forward_cm(self, x: torch.Tensor, lengths: Optional[torch.Tensor] = None,
                    ssm_hiddens: Optional[torch.Tensor] = None, use_cache: bool = False,
@@ -511,11 +561,17 @@ class CausalLM(nn.Module):
     def forward(self, input_ids: torch.Tensor, lengths: Optional[torch.Tensor] = None,
                 use_cache: bool = False) -> torch.Tensor:
         """input_ids (batch, seq_len) -> logits (batch, seq_len, vocab)."""
-        x = self.embedding(input_ids).transpose(1, 2).contiguous()
+        x = self.embedding(input_ids)
+        if torch.is_grad_enabled() and all(layer._fused(x) for layer in self.layers):
+            # training: each layer token-major in and out
+            for layer in self.layers:
+                x, _ = layer.forward(x, lengths=lengths, use_cache=use_cache)
+            return self.lm_head(self.norm(x))
+        x = _channel_major(x)
         for layer in self.layers:
             # x is this method's own stream: layers may update it in place
             x, _ = layer.forward_cm(x, lengths=lengths, use_cache=use_cache, inplace=True)
-        x = self.norm(x, dim=1).transpose(1, 2).contiguous()
+        x = _channel_major(self.norm(x, dim=1))
         return self.lm_head(x)
 
     def forward_last(self, input_ids: torch.Tensor, lengths: Optional[torch.Tensor] = None,
@@ -525,7 +581,7 @@ class CausalLM(nn.Module):
         (``models/causal_lm.py:104-113``, the same index, negative wrapping
         included).  The final norm and the LM head run on those rows only."""
         batch, seqlen = input_ids.shape
-        x = self.embedding(input_ids).transpose(1, 2).contiguous()
+        x = _channel_major(self.embedding(input_ids))
         for layer in self.layers:
             x, _ = layer.forward_cm(x, lengths=lengths, use_cache=use_cache, inplace=True)
         last = (torch.full((batch,), seqlen, dtype=torch.long, device=input_ids.device)

@@ -53,6 +53,18 @@ int decode_layers_max_width();
 hipError_t launch_decode_layers(int bf16, const void* table, int nlayers, int B, int K, int dim,
                                 int width, int R, int nout, float eps, const void* x, void* out,
                                 void* ws, hipStream_t st);
+int rms_norm_tc_max_channels(int bf16);
+int rms_norm_tc_part_rows(int B, int L);
+hipError_t launch_rms_norm_tc(int bf16, const void* x, const void* w, float eps, void* h_cm,
+                              void* h_tm, float* rstd, int B, int L, int C, bool vec,
+                              hipStream_t st);
+hipError_t launch_rms_norm_tc_bwd(int bf16, const void* x, const void* w, const float* rstd,
+                                  const void* dh, const void* dres, void* dx, void* dw, float* part,
+                                  int B, int L, int C, bool vec, hipStream_t st);
+hipError_t launch_transpose(int bf16, const void* in, int64_t ibs, void* out, int B, int R, int S,
+                            bool vec, hipStream_t st);
+hipError_t launch_batch_sum(int bf16, const void* in, void* out, int B, int R, int S, bool trans,
+                            bool vec, hipStream_t st);
 int decode_rows_max_batch();
 hipError_t launch_decode_rows_linear(int bf16, const void* W, const void* x, const void* nw,
                                      float eps, const void* bias, const void* res, void* y, int B,
@@ -965,6 +977,102 @@ int ssm_rms_norm_cm(int64_t batch, int64_t channels, int64_t seqlen, int dtype, 
                                             (int)channels, (int)seqlen, pair,
                                             static_cast<hipStream_t>(stream)),
                     "rms_norm_cm launch");
+}
+
+namespace {
+int check_rms_norm_tc(int64_t batch, int64_t seqlen, int64_t channels, int dtype,
+                      std::initializer_list<const void*> aligned) {
+  if (dtype != SSM_F32 && dtype != SSM_BF16)
+    return fail(SSM_ERR_INVALID, "dtype must be SSM_F32 or SSM_BF16 (got %d)", dtype);
+  if (batch < 1 || channels < 1 || seqlen < 1)
+    return fail(SSM_ERR_INVALID, "batch, seqlen and channels must be >= 1");
+  const int e = elems16(dtype), most = ssm::rms_norm_tc_max_channels(dtype == SSM_BF16);
+  if (channels % e || channels > most)
+    return fail(SSM_ERR_UNSUPPORTED, "rms_norm_tc takes channels a multiple of %d and <= %d (got %lld)",
+                e, most, (long long)channels);
+  if (seqlen > INT_MAX / 2 || batch * ((seqlen + 31) / 32) > INT_MAX / 4)
+    return fail(SSM_ERR_UNSUPPORTED, "rms_norm_tc sizes too large");
+  for (const void* p : aligned)
+    if (!aligned16(p))
+      return fail(SSM_ERR_UNSUPPORTED, "rms_norm_tc needs 16-byte aligned token-major tensors and weight");
+  return SSM_OK;
+}
+}  // namespace
+
+int ssm_rms_norm_tc_fwd(int64_t batch, int64_t seqlen, int64_t channels, int dtype, const void* x,
+                        const void* weight, float eps, void* h_cm, void* h_tm, float* rstd,
+                        void* stream) {
+  g_err.clear();
+  if (!x || !weight || !h_cm) return fail(SSM_ERR_INVALID, "x, weight and h_cm must be non-NULL");
+  if (int rc = check_rms_norm_tc(batch, seqlen, channels, dtype, {x, weight, h_tm})) return rc;
+  const bool vec = seqlen % elems16(dtype) == 0 && aligned16(h_cm);
+  return hip_status(ssm::launch_rms_norm_tc(dtype == SSM_BF16, x, weight, eps, h_cm, h_tm, rstd,
+                                            (int)batch, (int)seqlen, (int)channels, vec,
+                                            static_cast<hipStream_t>(stream)),
+                    "rms_norm_tc launch");
+}
+
+size_t ssm_rms_norm_tc_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t channels) {
+  if (batch < 1 || seqlen < 1 || channels < 1 || seqlen > INT_MAX / 2 ||
+      batch * ((seqlen + 31) / 32) > INT_MAX / 4)
+    return 0;
+  return round256((size_t)ssm::rms_norm_tc_part_rows((int)batch, (int)seqlen) * channels * sizeof(float));
+}
+
+int ssm_rms_norm_tc_bwd(int64_t batch, int64_t seqlen, int64_t channels, int dtype, const void* x,
+                        const void* weight, const float* rstd, const void* dh_cm, const void* dres,
+                        void* dx, void* dweight, void* workspace, size_t workspace_bytes,
+                        void* stream) {
+  g_err.clear();
+  if (!x || !weight || !rstd || !dh_cm || !dx || !dweight)
+    return fail(SSM_ERR_INVALID, "x, weight, rstd, dh_cm, dx and dweight must be non-NULL");
+  if (int rc = check_rms_norm_tc(batch, seqlen, channels, dtype, {x, weight, dres, dx})) return rc;
+  const size_t need = ssm_rms_norm_tc_bwd_workspace_bytes(batch, seqlen, channels);
+  if (!workspace || workspace_bytes < need)
+    return fail(SSM_ERR_INVALID, "workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
+  const bool vec = seqlen % elems16(dtype) == 0 && aligned16(dh_cm);
+  return hip_status(ssm::launch_rms_norm_tc_bwd(dtype == SSM_BF16, x, weight, rstd, dh_cm, dres, dx,
+                                                dweight, static_cast<float*>(workspace), (int)batch,
+                                                (int)seqlen, (int)channels, vec,
+                                                static_cast<hipStream_t>(stream)),
+                    "rms_norm_tc backward launch");
+}
+
+int ssm_transpose(int64_t batch, int64_t rows, int64_t cols, int dtype, const void* in,
+                  int64_t in_batch_stride, void* out, void* stream) {
+  g_err.clear();
+  if (dtype != SSM_F32 && dtype != SSM_BF16)
+    return fail(SSM_ERR_INVALID, "dtype must be SSM_F32 or SSM_BF16 (got %d)", dtype);
+  if (batch < 1 || rows < 1 || cols < 1 || !in || !out)
+    return fail(SSM_ERR_INVALID, "batch, rows and cols must be >= 1, in and out non-NULL");
+  if (in_batch_stride != 0 && in_batch_stride < rows * cols)
+    return fail(SSM_ERR_INVALID, "in_batch_stride must be 0 (contiguous) or at least rows * cols (got %lld)",
+                (long long)in_batch_stride);
+  if (batch > 65535 || rows > (int64_t)65535 * 64 || cols > INT_MAX / 2)
+    return fail(SSM_ERR_UNSUPPORTED, "transpose sizes too large");
+  const int64_t ibs = in_batch_stride ? in_batch_stride : rows * cols;
+  const int e = elems16(dtype);
+  const bool vec = rows % e == 0 && cols % e == 0 && ibs % e == 0 && aligned16(in) && aligned16(out);
+  return hip_status(ssm::launch_transpose(dtype == SSM_BF16, in, ibs, out, (int)batch, (int)rows,
+                                          (int)cols, vec, static_cast<hipStream_t>(stream)),
+                    "transpose launch");
+}
+
+int ssm_batch_sum(int64_t batch, int64_t rows, int64_t cols, int dtype, const void* in,
+                  int transposed, void* out, void* stream) {
+  g_err.clear();
+  if (dtype != SSM_F32 && dtype != SSM_BF16)
+    return fail(SSM_ERR_INVALID, "dtype must be SSM_F32 or SSM_BF16 (got %d)", dtype);
+  if (batch < 1 || rows < 1 || cols < 1 || !in || !out)
+    return fail(SSM_ERR_INVALID, "batch, rows and cols must be >= 1, in and out non-NULL");
+  if (batch > INT_MAX / 2 || rows > (int64_t)65535 * 32 || cols > INT_MAX / 2)
+    return fail(SSM_ERR_UNSUPPORTED, "batch_sum sizes too large");
+  const int e = elems16(dtype);
+  const bool vec = cols % e == 0 && (!transposed || rows % e == 0) && aligned16(in) && aligned16(out);
+  return hip_status(ssm::launch_batch_sum(dtype == SSM_BF16, in, out, (int)batch, (int)rows,
+                                          (int)cols, transposed != 0, vec,
+                                          static_cast<hipStream_t>(stream)),
+                    "batch_sum launch");
 }
 
 size_t ssm_causal_conv1d_bwd_workspace_bytes(int64_t batch, int64_t dim, int64_t width) {

@@ -1,0 +1,213 @@
+"""The training forward and backward of one ``Block`` (``modules/block.py:78-90``
+with ``modules/mamba.py:82-187``) as four autograd functions over the HIP
+kernels: norm and in-projection, the conv (``CausalConv1dFn``), the x- and
+step-size projections with the scan, and the out-projection with the residual.
+
+Against one torch op per line, what each function's backward saves is passes
+over memory: the norm's chain of float32 elementwise kernels, the transpositions
+around the layer, the additions of gradients that meet (the residual's into the
+norm's backward, the scan's du into the x-projection's product), the zero-filled
+gradients of slices.  The weight gradients are batched products per batch row of
+contiguous operands, summed over the batch in float32 and rounded once.
+
+``supported`` says which layers and inputs take this path; every other one runs
+op by op (``Block.forward_cm``).  When a backward is itself being differentiated
+(create_graph), the functions of this module fall back to differentiating their
+op-by-op form.
+"""
+from __future__ import annotations
+
+from typing import Optional
+
+import torch
+
+from . import layout as _lay
+from . import selective_scan
+from .ops import selective_scan_fn
+
+
+def _bmm(w: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """w @ x per batch row, for one (m, k) weight (or its transposed view) and
+    contiguous (batch, k, n) x; added to ``out`` in place when given."""
+    w = w.expand(x.shape[0], *w.shape)
+    return torch.bmm(w, x) if out is None else out.baddbmm_(w, x)
+
+
+def _grads_op_by_op(ctx, fn, inputs, grads):
+    """Gradients of fn(*inputs) as differentiable torch ops (create_graph)."""
+    with torch.enable_grad():
+        outs = fn(*inputs)
+        pairs = [(o, g) for o, g in zip(outs, grads) if g is not None]
+        want = [i for i, t in enumerate(inputs)
+                if isinstance(t, torch.Tensor) and t.requires_grad and ctx.needs_input_grad[i]]
+        got = torch.autograd.grad([o for o, _ in pairs], [inputs[i] for i in want],
+                                  [g for _, g in pairs], create_graph=True, allow_unused=True)
+    res = [None] * len(ctx.needs_input_grad)
+    for i, g in zip(want, got):
+        res[i] = g
+    return tuple(res)
+
+
+class NormInProjFn(torch.autograd.Function):
+    """(xs, z, x) of token-major x: the two halves of W_in @ rmsnorm(x),
+    channel-major, and x itself for the residual, whose gradient then enters
+    the norm's backward."""
+
+    @staticmethod
+    def forward(ctx, x, norm_weight, w_in, eps):
+        h, h_tm, rstd, xr = _lay.norm_tc(x, norm_weight, eps, token_major=True)
+        inner = w_in.shape[0] // 2
+        xs, z = _bmm(w_in[:inner], h), _bmm(w_in[inner:], h)
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(x, norm_weight, w_in, h_tm, rstd)
+        ctx.eps = eps
+        return xs, z, x.view_as(x)
+
+    @staticmethod
+    def _op_by_op(x, norm_weight, w_in, eps):
+        xf = x.transpose(1, 2).float()
+        h = (xf * torch.rsqrt(xf.pow(2).mean(1, keepdim=True) + eps)
+             * (1.0 + norm_weight.float())[:, None]).type_as(x).contiguous()
+        inner = w_in.shape[0] // 2
+        return _bmm(w_in[:inner], h), _bmm(w_in[inner:], h), x.view_as(x)
+
+    @staticmethod
+    def backward(ctx, dxs, dz, dres):
+        x, norm_weight, w_in, h_tm, rstd = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _grads_op_by_op(ctx, NormInProjFn._op_by_op, (x, norm_weight, w_in, ctx.eps),
+                                   (dxs, dz, dres))
+        need_x, need_nw, need_w = ctx.needs_input_grad[:3]
+        inner = w_in.shape[0] // 2
+        halves = [(slice(0, inner), dxs), (slice(inner, 2 * inner), dz)]
+        halves = [(s, g.contiguous()) for s, g in halves if g is not None]
+        dw = None
+        if need_w:
+            dw = torch.empty(w_in.shape, dtype=w_in.dtype, device=w_in.device)
+            if len(halves) < 2:
+                dw.zero_()
+            for s, g in halves:
+                _lay.batch_sum(torch.bmm(g, h_tm), out=dw[s])
+        dx = dnw = None
+        if need_x or need_nw:
+            dh = None
+            for s, g in halves:
+                dh = _bmm(w_in[s].t(), g, dh)
+            if dh is None:
+                dx = dres
+            else:
+                xr = _lay.aligned(x)
+                dx, dnw = _lay.norm_tc_backward(xr, norm_weight, rstd, dh, dres)
+        return dx if need_x else None, dnw if need_nw else None, dw, None
+
+
+class SsmFn(torch.autograd.Function):
+    """(y, last state) from the conv output xc and the gate z, channel-major:
+    params = W_x xc, delta = W_dt params[:R], and the gated scan with B and C
+    read from params (``modules/mamba.py:141-182``)."""
+
+    @staticmethod
+    def forward(ctx, xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, side):
+        rank, nstate = w_dt.shape[1], A.shape[1]
+        params = _bmm(w_x, xc)
+        delta = _bmm(w_dt, params[:, :rank])
+        f32 = lambda t: None if t is None else t.float().contiguous()
+        A32, D32, b32, h0 = f32(A), f32(D), f32(dt_bias), f32(h_init)
+        y = torch.empty_like(xc)
+        out, h = selective_scan.forward(
+            xc, A32, params[:, rank:rank + nstate], params[:, rank + nstate:], D32, delta, b32, h0,
+            lengths, side, z=z, out_ungated=y)
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, params, delta, y, h)
+        ctx.side = side
+        return out, selective_scan.last_state(h)
+
+    @staticmethod
+    def _op_by_op(xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, side):
+        rank, nstate = w_dt.shape[1], A.shape[1]
+        params = _bmm(w_x, xc)
+        delta = _bmm(w_dt, params[:, :rank])
+        return selective_scan_fn(xc, delta, A, params[:, rank:rank + nstate],
+                                 params[:, rank + nstate:], D, z=z, delta_bias=dt_bias,
+                                 return_last_state=True, h_init=h_init, length=lengths,
+                                 padding_side=side)
+
+    @staticmethod
+    def backward(ctx, dout, dlast):
+        xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, params, delta, y, h = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _grads_op_by_op(ctx, SsmFn._op_by_op,
+                                   (xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, ctx.side),
+                                   (dout, dlast))
+        need = ctx.needs_input_grad
+        rank, nstate = w_dt.shape[1], A.shape[1]
+        f32 = lambda t: None if t is None else t.float().contiguous()
+        if dout is None:
+            dout = torch.zeros_like(xc)
+        du, dA, dB, dC, dD, ddelta, dbias, dh0, dz = selective_scan.backward(
+            xc, f32(A), params[:, rank:rank + nstate], params[:, rank + nstate:], f32(D), delta,
+            f32(dt_bias), h, f32(h_init), dout.contiguous(), f32(dlast), lengths, ctx.side, z=z,
+            out_ungated=y)
+        dw_dt = dw_x = None
+        if need[3]:
+            dw_dt = _lay.batch_sum(torch.bmm(ddelta, _lay.transposed(params[:, :rank])))
+        if need[0] or need[2]:
+            dparams = torch.cat([_bmm(w_dt.t(), ddelta), dB, dC], dim=1)
+            if need[2]:
+                dw_x = _lay.batch_sum(torch.bmm(xc, _lay.transposed(dparams)), transpose=True)
+            if need[0]:
+                du = _bmm(w_x.t(), dparams, du)
+        return (du if need[0] else None, dz, dw_x, dw_dt, dA, dD, dbias, dh0, None, None)
+
+
+class OutProjFn(torch.autograd.Function):
+    """Token-major W_out @ y (+ residual) of channel-major y."""
+
+    @staticmethod
+    def forward(ctx, y, w_out, residual):
+        ctx.save_for_backward(y, w_out)
+        ctx.has_residual = residual is not None
+        return out_proj(y, w_out, residual)
+
+    @staticmethod
+    def _op_by_op(y, w_out, residual):
+        out = _bmm(w_out, y).transpose(1, 2)
+        return (out if residual is None else residual + out,)
+
+    @staticmethod
+    def backward(ctx, dout):
+        y, w_out = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            dy, dw, _ = _grads_op_by_op(ctx, OutProjFn._op_by_op, (y, w_out, None), (dout,))
+            return dy, dw, dout if need[2] else None
+        dout = dout.contiguous()
+        dy = _bmm(w_out.t(), _lay.transposed(dout)) if need[0] else None
+        dw = _lay.batch_sum(torch.bmm(y, dout), transpose=True) if need[1] else None
+        return dy, dw, dout if need[2] else None
+
+
+def out_proj(y: torch.Tensor, w_out: torch.Tensor, residual: Optional[torch.Tensor]) -> torch.Tensor:
+    """(batch, seq_len, out) = y^T W_out^T (+ residual, added in the product) for
+    channel-major y.  The batched product takes W_out^T as a contiguous copy;
+    one batch row is a plain product and takes the views."""
+    if y.shape[0] == 1:
+        a, b = y[0].t(), w_out.t()
+        return (torch.mm(a, b) if residual is None else torch.addmm(residual[0], a, b))[None]
+    wt = _lay.transposed(w_out[None]).expand(y.shape[0], w_out.shape[1], w_out.shape[0])
+    return torch.bmm(y.transpose(1, 2), wt) if residual is None \
+        else torch.baddbmm(residual, y.transpose(1, 2), wt)
+
+
+def supported(block, x: torch.Tensor) -> bool:
+    """Whether token-major x through ``block`` takes the fused layer: float32 or
+    bfloat16 on the GPU with every projection weight in x's dtype, no
+    projection biases, a width the norm kernel takes, no autocast."""
+    ssm, w = block.ssm, block.norm.weight
+    if torch.is_autocast_enabled() or not _lay.norm_tc_supported(x, w):
+        return False
+    if ssm.input_proj.bias is not None or ssm.out_proj.bias is not None:
+        return False
+    return all(p.dtype == x.dtype and p.device == x.device
+               for p in (ssm.input_proj.weight, ssm.ssm_param_proj.weight, ssm.delta_proj.weight,
+                         ssm.out_proj.weight, ssm.conv.weight))

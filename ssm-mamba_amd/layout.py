@@ -1,0 +1,103 @@
+"""Host side of the kernels between token-major activations (batch, seq_len,
+channels), the layout of the reference's ``Block`` (``modules/block.py:78-90``),
+and the channel-major layout the conv and scan kernels stream
+(``ssm_rms_norm_tc_*``, ``ssm_transpose`` and ``ssm_batch_sum`` of
+include/ssm_mamba.h).  No autograd here."""
+from __future__ import annotations
+
+from typing import Optional
+
+import torch
+
+from . import _native as N
+
+DTYPES = {torch.float32: N.SSM_F32, torch.bfloat16: N.SSM_BF16}
+_MAX_CHANNELS = {torch.float32: 1024, torch.bfloat16: 2048}
+
+
+def _stream(dev: torch.device) -> int:
+    return torch.cuda.current_stream(dev).cuda_stream
+
+
+def norm_tc_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``norm_tc`` takes token-major x (batch, seq_len, channels)."""
+    if not (x.is_cuda and x.dim() == 3 and x.dtype in DTYPES and x.numel() > 0):
+        return False
+    c = x.shape[2]
+    return (weight.dtype == x.dtype and weight.device == x.device and weight.is_contiguous()
+            and tuple(weight.shape) == (c,) and c * x.element_size() % 16 == 0
+            and c <= _MAX_CHANNELS[x.dtype] and weight.data_ptr() % 16 == 0)
+
+
+def aligned(x: torch.Tensor) -> torch.Tensor:
+    """x contiguous at a 16-byte aligned address."""
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
+def norm_tc(x: torch.Tensor, weight: torch.Tensor, eps: float, token_major: bool = False):
+    """(h (batch, channels, seq_len), h token-major or None, 1 / rms (batch,
+    seq_len) float32 or None, x as read) of RMSNorm(x) for token-major x;
+    ``token_major`` asks for the two that a backward needs."""
+    x = aligned(x)
+    batch, seqlen, ch = x.shape
+    h = torch.empty(batch, ch, seqlen, dtype=x.dtype, device=x.device)
+    h_tm = torch.empty_like(x) if token_major else None
+    rstd = torch.empty(batch, seqlen, dtype=torch.float32, device=x.device) if token_major else None
+    with torch.cuda.device(x.device):
+        N.check(N.lib().ssm_rms_norm_tc_fwd(
+            batch, seqlen, ch, DTYPES[x.dtype], x.data_ptr(), weight.data_ptr(), float(eps),
+            h.data_ptr(), None if h_tm is None else h_tm.data_ptr(),
+            None if rstd is None else rstd.data_ptr(), _stream(x.device)))
+    return h, h_tm, rstd, x
+
+
+def norm_tc_backward(x: torch.Tensor, weight: torch.Tensor, rstd: torch.Tensor, dh: torch.Tensor,
+                     dres: Optional[torch.Tensor]):
+    """(dx, dweight) of ``norm_tc`` for dh (batch, channels, seq_len); dres, the
+    gradient of a residual use of x, is added to dx."""
+    batch, seqlen, ch = x.shape
+    dh = dh.contiguous()
+    dres = None if dres is None else aligned(dres)
+    dx, dw = torch.empty_like(x), torch.empty_like(weight)
+    lib = N.lib()
+    ws = torch.empty(lib.ssm_rms_norm_tc_bwd_workspace_bytes(batch, seqlen, ch), dtype=torch.uint8,
+                     device=x.device)
+    with torch.cuda.device(x.device):
+        N.check(lib.ssm_rms_norm_tc_bwd(
+            batch, seqlen, ch, DTYPES[x.dtype], x.data_ptr(), weight.data_ptr(), rstd.data_ptr(),
+            dh.data_ptr(), None if dres is None else dres.data_ptr(), dx.data_ptr(), dw.data_ptr(),
+            ws.data_ptr(), ws.numel(), _stream(x.device)))
+    return dx, dw
+
+
+def transposed(x: torch.Tensor) -> torch.Tensor:
+    """x.transpose(1, 2).contiguous() for x (batch, rows, cols) whose matrices
+    are contiguous (a slice along dim 1 of a contiguous tensor is read in place
+    through its batch stride)."""
+    batch, rows, cols = x.shape
+    if not (x.is_cuda and x.dtype in DTYPES and x.numel() > 0) or batch > 65535 \
+            or rows > 65535 * 64:
+        return x.transpose(1, 2).contiguous()
+    if x.stride(2) != 1 or x.stride(1) != cols or (batch > 1 and x.stride(0) < rows * cols):
+        x = x.contiguous()
+    out = torch.empty(batch, cols, rows, dtype=x.dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        N.check(N.lib().ssm_transpose(batch, rows, cols, DTYPES[x.dtype], x.data_ptr(),
+                                      0 if batch == 1 else x.stride(0), out.data_ptr(),
+                                      _stream(x.device)))
+    return out
+
+
+def batch_sum(x: torch.Tensor, transpose: bool = False,
+              out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x.sum(0), or its transpose, for contiguous x (batch, rows, cols), added
+    in float32 and rounded once; into ``out`` (contiguous) when given."""
+    batch, rows, cols = x.shape
+    x = x.contiguous()
+    if out is None:
+        out = torch.empty((cols, rows) if transpose else (rows, cols), dtype=x.dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        N.check(N.lib().ssm_batch_sum(batch, rows, cols, DTYPES[x.dtype], x.data_ptr(),
+                                      int(transpose), out.data_ptr(), _stream(x.device)))
+    return out

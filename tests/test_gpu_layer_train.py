@@ -1,0 +1,146 @@
+"""The fused layer of a training step and its kernels: the norm between the
+layouts and its backward against float64, the transposition and the batch sum
+bit for bit, and a Block's outputs and gradients against the op-by-op
+path (which tests/test_gpu_lm.py checks against float64)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.bfloat16]
+
+
+# one token; ragged tiles of 32 tokens, element-wise rows (odd lengths); channel
+# counts of one chunk, past a 64-chunk group, and the largest of each tile size
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batch,seqlen,ch", [(1, 1, 8), (2, 33, 64), (3, 100, 1000), (2, 77, 512),
+                                              (1, 64, 1024), (1, 50, 2048)])
+def test_norm_between_layouts(cuda, dtype, batch, seqlen, ch):
+    from ssm_mamba_amd import layout as LY
+    ch = min(ch, 1024) if dtype == torch.float32 else ch
+    g = torch.Generator().manual_seed(ch + seqlen)
+    x = torch.randn(batch, seqlen, ch, generator=g).to(dtype)
+    w = (0.3 * torch.randn(ch, generator=g)).to(dtype)
+    dh = torch.randn(batch, ch, seqlen, generator=g).to(dtype)
+    dres = torch.randn(batch, seqlen, ch, generator=g).to(dtype)
+    d = lambda t: t.to(cuda)
+    assert LY.norm_tc_supported(d(x), d(w))
+    h, h_tm, rstd, xr = LY.norm_tc(d(x), d(w), 1e-6, token_major=True)
+    assert torch.equal(LY.norm_tc(d(x), d(w), 1e-6)[0], h)
+    assert torch.equal(h.transpose(1, 2), h_tm)
+    dx, dw = LY.norm_tc_backward(xr, d(w), rstd, d(dh), d(dres))
+    dx0, _ = LY.norm_tc_backward(xr, d(w), rstd, d(dh), None)
+    again = LY.norm_tc_backward(xr, d(w), rstd, d(dh), d(dres))
+    assert torch.equal(dx, again[0]) and torch.equal(dw, again[1])
+    x64, w64 = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    r = x64 * torch.rsqrt(x64.pow(2).mean(-1, keepdim=True) + 1e-6) * (1.0 + w64)
+    g64 = dh.double().transpose(1, 2)
+    rx, rw = torch.autograd.grad(r, [x64, w64], g64)
+    # one rounding of the result; in float32 the rsqrt and the sums on top
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -19
+    assert bool(((h_tm.cpu().double() - r).abs() <= u * r.abs()).all())
+    # sums of |terms|: g xh over the channels, dh xh over the tokens
+    rs = torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6)
+    xh, gw = x.double() * rs, (g64 * (1.0 + w.double())).abs()
+    size = rs * (gw + xh.abs() * (gw * xh.abs()).mean(-1, keepdim=True))
+    for got, ref, sz in ((dx, rx + dres.double(), size + dres.double().abs()), (dx0, rx, size),
+                         (dw, rw, (g64 * xh).abs().sum((0, 1)))):
+        err = (got.cpu().double() - ref).abs()
+        assert bool((err <= u * ref.abs() + 64 * 2.0 ** -24 * sz).all())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batch,rows,cols", [(1, 1, 1), (3, 65, 130), (2, 64, 72), (2, 96, 40),
+                                              (5, 200, 64)])
+def test_transpose_and_batch_sum(cuda, dtype, batch, rows, cols):
+    from ssm_mamba_amd import layout as LY
+    g = torch.Generator().manual_seed(rows * cols)
+    x = torch.randn(batch, rows, cols, generator=g).to(dtype).to(cuda)
+    assert torch.equal(LY.transposed(x), x.transpose(1, 2).contiguous())
+    part = x[:, : rows // 2 + 1]  # read through its batch stride
+    assert torch.equal(LY.transposed(part), part.transpose(1, 2).contiguous())
+    ref = torch.zeros(rows, cols, device=cuda)
+    for b in range(batch):
+        ref = ref + x[b].float()
+    ref = ref.to(dtype)
+    assert torch.equal(LY.batch_sum(x), ref)
+    assert torch.equal(LY.batch_sum(x, transpose=True), ref.t())
+
+
+def _block(dtype, model_dim, conv_bias, seed):
+    from ssm_mamba_amd.causal_lm import Block
+    torch.manual_seed(seed)
+    blk = Block(model_dim=model_dim, dropout_rate=0.0, conv_bias=conv_bias)
+    with torch.no_grad():
+        blk.norm.weight.normal_(0.0, 0.3)
+        blk.ssm.D.normal_(1.0, 0.1)
+    return blk.cuda().to(dtype).train()
+
+
+def _grads(blk, x, dout, dlast, h0, lengths, fused):
+    from ssm_mamba_amd import layer_train as LT
+    keep = LT.supported
+    if not fused:
+        LT.supported = lambda *a: False
+    try:
+        assert blk._fused(x) == fused
+        out, last = blk(x, lengths=lengths, ssm_hiddens=h0)
+        names, ps = zip(*blk.named_parameters())
+        got = torch.autograd.grad([out, last], [x, h0, *ps], [dout, dlast])
+    finally:
+        LT.supported = keep
+    return {"out": out.detach(), "last": last.detach(), **dict(zip(["x", "h0", *names], got))}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batch,seqlen,model_dim,conv_bias", [
+    (2, 37, 64, False),    # odd length: element-wise rows in every kernel
+    (1, 100, 72, True),    # one batch row: the plain out-projection product
+    (3, 256, 256, False),
+])
+def test_block_gradients(cuda, dtype, batch, seqlen, model_dim, conv_bias):
+    """Against the op-by-op path: the two round the same intermediate tensors
+    to the layer's dtype, so they differ by float32 sums in other orders, in
+    bf16 amplified to single roundings of those tensors."""
+    blk = _block(dtype, model_dim, conv_bias, seed=seqlen)
+    g = torch.Generator().manual_seed(model_dim)
+    r = lambda *s: torch.randn(*s, generator=g).to(cuda)
+    x = r(batch, seqlen, model_dim).to(dtype).requires_grad_(True)
+    h0 = (0.1 * r(batch, 2 * model_dim, 16)).requires_grad_(True)
+    lengths = torch.randint(1, seqlen + 1, (batch,), generator=g).to(cuda)
+    dout, dlast = r(batch, seqlen, model_dim).to(dtype), r(batch, 2 * model_dim, 16)
+    a = _grads(blk, x, dout, dlast, h0, lengths, True)
+    b = _grads(blk, x, dout, dlast, h0, lengths, False)
+    for k in a:
+        assert a[k].dtype == b[k].dtype and a[k].shape == b[k].shape, k
+        rel = float((a[k].double() - b[k].double()).norm() / b[k].double().norm())
+        assert rel <= (2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -18), (k, rel)
+
+
+def test_block_second_derivatives_and_frozen_parameters(cuda):
+    """create_graph differentiates the op-by-op form; parameters and inputs
+    that need no gradient get none."""
+    from ssm_mamba_amd import layer_train as LT
+    blk = _block(torch.float32, 64, False, seed=3)
+    x0 = torch.randn(2, 40, 64, generator=torch.Generator().manual_seed(4)).to(cuda)
+
+    def penalty(fused):
+        keep = LT.supported
+        if not fused:
+            LT.supported = lambda *a: False
+        try:
+            x = x0.clone().requires_grad_(True)
+            out, _ = blk(x)
+            gx, = torch.autograd.grad(out.pow(2).sum(), x, create_graph=True)
+            return torch.autograd.grad(gx.pow(2).sum(), [x, blk.norm.weight, blk.ssm.out_proj.weight,
+                                                         blk.ssm.input_proj.weight])
+        finally:
+            LT.supported = keep
+
+    for u, v in zip(penalty(True), penalty(False)):
+        assert float((u - v).norm() / v.norm()) <= 1e-5
+    blk.ssm.input_proj.weight.requires_grad_(False)
+    blk.norm.weight.requires_grad_(False)
+    blk(x0)[0].sum().backward()
+    assert blk.ssm.input_proj.weight.grad is None and blk.norm.weight.grad is None
+    assert all(p.grad is not None for n, p in blk.named_parameters() if p.requires_grad)

@@ -707,9 +707,9 @@ constexpr int kCacheNTb = 2;  // cache-policy bit NT (nontemporal) of a buffer a
 // whole-column accesses are permutations of 64 consecutive float4s.
 __device__ __forceinline__ constexpr int bws_swz(int q) { return 2 * q + 8 * (q & 1); }
 
-template <typename T, int kSG>
+template <typename T, int kSG, bool kAligned>
 struct BwsRows {  // one tile's raw loads of a producer lane, as loaded
-  typename Raw4<T>::type u, d, dy, z, y;
+  typename RowRaw<T, kAligned>::type u, d, dy, z, y;
   uint32_t B[kSG], C[kSG];  // element bits
 };
 
@@ -1020,14 +1020,8 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
   const int sw = row ^ bws_swz(q);
   const int pch = d0 + row;
   const bool pch_ok = pch < Dm;
-  const int chc = min(pch, Dm - 1);
   const float Dv = (pch_ok && Dp) ? Dp[pch] : 0.0f;
   const float Bias = (pch_ok && biasp) ? biasp[pch] : 0.0f;
-  const T* __restrict__ u_row = u + (rb + chc) * L;
-  const T* __restrict__ d_row = dl + (rb + chc) * L;
-  const T* __restrict__ dy_row = dyp + (rb + chc) * L;
-  const T* __restrict__ z_row = kHasZ ? zp + (rb + chc) * L : u_row;
-  const T* __restrict__ y_row = kHasZ ? yup + (rb + chc) * L : u_row;
   int vlo, vhi;
   valid_window(length, p.pad_right, b, L, vlo, vhi);
   const bool softplus = p.softplus != 0;
@@ -1037,76 +1031,54 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
   // staging past N)
   const int bc_n = (pt / kTileB) % (2 * kWsCons);
   const int bc_j = pt % kTileB;
-  const T* __restrict__ B_rows = Bp + (size_t)b * p.bc_bstride;
-  const T* __restrict__ C_rows = Cp + (size_t)b * p.bc_bstride;
   const int bc_slot = (bc_j & 3) * 4 + (bc_n & 1) * 2;  // B; C at + 1
   // tile index of iteration i (clamped to the segment: tiles past it are
   // staged from valid rows and never used)
   auto tile_of = [&](int i) { return max(tile_end - 1 - i, tile_beg); };
-  // Output buffers of this wave's 16 channel rows (aligned path; the launch
-  // keeps 16 * L * sizeof(T) < 2^31): a masked lane, a step past L or a tile
-  // past the segment gets an offset outside the range and the store is dropped.
+  // Buffer ranges over this wave's 16 channel rows (the launch keeps 16 * L *
+  // sizeof(T) < 2^31), and over the batch row's B and C rows, at 32-bit offsets
+  // (no 64-bit address arithmetic per tile).  Loads clamp the step into the
+  // row, and a row past the last channel reads zero; for stores a masked lane,
+  // a step past L or a tile past the segment gets an offset outside the range
+  // and the store is dropped.
+  using Range = RowRange<T, kAligned>;
   const int wrow0 = d0 + (w - kWsCons) * (kBlockCh / kWsProd);
   const uint32_t wbytes =
       (uint32_t)(max(0, min(kBlockCh / kWsProd, Dm - wrow0)) * (size_t)L * sizeof(T));
-  const auto du_rsrc = raw_rsrc(dup + ((size_t)rb + wrow0) * L, wbytes);
-  const auto dd_rsrc = raw_rsrc(ddp + ((size_t)rb + wrow0) * L, wbytes);
-  const auto dz_rsrc = raw_rsrc(kHasZ ? dzp + ((size_t)rb + wrow0) * L : dup, kHasZ ? wbytes : 0u);
-  const uint32_t row_off = (uint32_t)((row % (kBlockCh / kWsProd)) * (size_t)L * sizeof(T));
-
-  // The aligned path's loads go through buffer ranges over the same 16 rows,
-  // and over the batch row's B and C rows, at 32-bit offsets (no 64-bit
-  // address arithmetic per tile).  The step is clamped into the row as on the
-  // pointer path; a row past the last channel reads zero.
-  const auto u_ld = raw_rsrc(const_cast<T*>(u) + ((size_t)rb + wrow0) * L, wbytes);
-  const auto d_ld = raw_rsrc(const_cast<T*>(dl) + ((size_t)rb + wrow0) * L, wbytes);
-  const auto dy_ld = raw_rsrc(const_cast<T*>(dyp) + ((size_t)rb + wrow0) * L, wbytes);
-  const auto z_ld = raw_rsrc(kHasZ ? const_cast<T*>(zp) + ((size_t)rb + wrow0) * L : const_cast<T*>(u),
-                             kHasZ ? wbytes : 0u);
-  const auto y_ld = raw_rsrc(kHasZ ? const_cast<T*>(yup) + ((size_t)rb + wrow0) * L : const_cast<T*>(u),
-                             kHasZ ? wbytes : 0u);
+  const size_t wbase = ((size_t)rb + wrow0) * L;
+  const auto du_rsrc = raw_rsrc(dup + wbase, wbytes);
+  const auto dd_rsrc = raw_rsrc(ddp + wbase, wbytes);
+  const auto dz_rsrc = raw_rsrc(kHasZ ? dzp + wbase : dup, kHasZ ? wbytes : 0u);
+  uint32_t row_off = (uint32_t)((row % (kBlockCh / kWsProd)) * (size_t)L * sizeof(T));
+  if constexpr (!kAligned) row_off = pch_ok ? row_off : kOffDrop;
+  const Range u_ld(u + wbase, wbytes);
+  const Range d_ld(dl + wbase, wbytes);
+  const Range dy_ld(dyp + wbase, wbytes);
+  const Range z_ld(kHasZ ? zp + wbase : u, kHasZ ? wbytes : 0u);
+  const Range y_ld(kHasZ ? yup + wbase : u, kHasZ ? wbytes : 0u);
   const uint32_t bc_bytes = (uint32_t)((size_t)N * L * sizeof(T));
   const auto B_ld = raw_rsrc(const_cast<T*>(Bp) + (size_t)b * p.bc_bstride, bc_bytes);
   const auto C_ld = raw_rsrc(const_cast<T*>(Cp) + (size_t)b * p.bc_bstride, bc_bytes);
   auto bc_row = [&](int g) { return (size_t)min(16 * g + bc_n, N - 1) * L; };
 
-  using Rows = BwsRows<T, kSG>;
+  using Rows = BwsRows<T, kSG, kAligned>;
   auto issue = [&](Rows& r, int i) {
-    if constexpr (kAligned) {
-      const int t0 = tile_of(i) * kTileB;
-      const uint32_t off = row_off + (uint32_t)min(t0 + 4 * q, L - 4) * sizeof(T);
-      r.u = buffer_load_raw4<T>(u_ld, off);
-      r.d = buffer_load_raw4<T>(d_ld, off);
-      r.dy = buffer_load_raw4<T>(dy_ld, off);
-      if constexpr (kHasZ) {
-        r.z = buffer_load_raw4<T>(z_ld, off);
-        r.y = buffer_load_raw4<T>(y_ld, off);
-      } else {
-        r.z = r.y = typename Raw4<T>::type{};
-      }
-#pragma unroll
-      for (int g = 0; g < kSG; ++g) {
-        const uint32_t boff = (uint32_t)((bc_row(g) + min(t0 + bc_j, L - 1)) * sizeof(T));
-        r.B[g] = buffer_load_bits1<T>(B_ld, boff);
-        r.C[g] = buffer_load_bits1<T>(C_ld, boff);
-      }
-      return;
-    }
-    const int t = tile_of(i) * kTileB + 4 * q;
-    r.u = load_raw4_nb<T, kAligned>(u_row, t, L, pch_ok);
-    r.d = load_raw4_nb<T, kAligned>(d_row, t, L, pch_ok);
-    r.dy = load_raw4_nb<T, kAligned>(dy_row, t, L, pch_ok);
+    const int t0 = tile_of(i) * kTileB;
+    const uint32_t off = row_off + (uint32_t)min(t0 + 4 * q, kAligned ? L - 4 : L - 1) * sizeof(T);
+    r.u = u_ld.load4(off);
+    r.d = d_ld.load4(off);
+    r.dy = dy_ld.load4(off);
     if constexpr (kHasZ) {
-      r.z = load_raw4_nb<T, kAligned>(z_row, t, L, pch_ok);
-      r.y = load_raw4_nb<T, kAligned>(y_row, t, L, pch_ok);
+      r.z = z_ld.load4(off);
+      r.y = y_ld.load4(off);
     } else {
-      r.z = r.y = typename Raw4<T>::type{};
+      r.z = r.y = typename RowRaw<T, kAligned>::type{};
     }
 #pragma unroll
     for (int g = 0; g < kSG; ++g) {
-      const size_t tb = bc_row(g) + min(tile_of(i) * kTileB + bc_j, L - 1);
-      r.B[g] = elem_bits(B_rows[tb]);
-      r.C[g] = elem_bits(C_rows[tb]);
+      const uint32_t boff = (uint32_t)((bc_row(g) + min(t0 + bc_j, L - 1)) * sizeof(T));
+      r.B[g] = buffer_load_bits1<T>(B_ld, boff);
+      r.C[g] = buffer_load_bits1<T>(C_ld, boff);
     }
   };
 
@@ -1125,9 +1097,14 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
     const int t = t0 + 4 * q;
     const int sb = i & 1;
     float uv[4], dv[4], dyv[4];
-    decode4(r.u, uv);
-    decode4(r.d, dv);
-    decode4(r.dy, dyv);
+    k.u = Range::bits(r.u, u_ld.shift(row_off));
+    Range::decode(r.d, d_ld.shift(row_off), dv);
+    Range::decode(r.dy, dy_ld.shift(row_off), dyv);
+    float zv[4], yv[4];
+    if constexpr (kHasZ) {
+      Range::decode(r.z, z_ld.shift(row_off), zv);
+      Range::decode(r.y, y_ld.shift(row_off), yv);
+    }
     float de[4], du[4], dov[4], dzo[4], dym[4];
     // (softplus is uniform: a branch, not a select after both forms)
     if (softplus) {
@@ -1143,26 +1120,28 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j) dym[j] = dyv[j];
     // Steps outside the valid window are masked on the tiles that hold any (at
-    // most two per row).  Rows past the last channel read zero on the aligned
-    // path (outside the wave's buffer range), so their delta * u and dout, and
-    // every term those feed, are zero unmasked; the pointer path reads the
-    // clamped channel there and masks them on every tile.
-    if (!kAligned || !(t0 >= vlo && t0 + kTileB <= vhi)) {
+    // most two per row).  Rows past the last channel read zero (outside the
+    // wave's buffer range), so their delta * u and dout, and every term those
+    // feed, are zero unmasked.  Unaligned rows: u and z past the end are
+    // another row's, zeroed so that their products with the masked terms are.
+    if (!(t0 >= vlo && t0 + kTileB <= vhi)) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const uint32_t keep = (pch_ok & (t + j >= vlo) & (t + j < vhi)) ? ~0u : 0u;
+        const uint32_t keep = ((t + j >= vlo) & (t + j < vhi)) ? ~0u : 0u;
         de[j] = __uint_as_float(__float_as_uint(de[j]) & keep);
         k.sg[j] = __uint_as_float(__float_as_uint(k.sg[j]) & keep);
         dym[j] = __uint_as_float(__float_as_uint(dym[j]) & keep);
       }
+      if constexpr (!kAligned) {
+        Range::mask_end(k.u, t, L);
+        if constexpr (kHasZ) Range::mask_end(zv, t, L);
+      }
     }
+    decode4(k.u, uv);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       du[j] = de[j] * uv[j];
       if constexpr (kHasZ) {
-        float zv[4], yv[4];
-        decode4(r.z, zv);
-        decode4(r.y, yv);
         // silu(z) = z s and silu'(z) = s + z s (1 - s), s = sigmoid(z)
         const float sz = sigmoidf_fast(zv[j]);
         const float zs = zv[j] * sz;
@@ -1173,7 +1152,6 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
         dzo[j] = 0.0f;
       }
     }
-    k.u = r.u;
     sSt[sb][0][q][sw] = make_float4(de[0], de[1], de[2], de[3]);
     sSt[sb][1][q][sw] = make_float4(du[0], du[1], du[2], du[3]);
     sSt[sb][2][q][sw] = make_float4(dov[0], dov[1], dov[2], dov[3]);
@@ -1185,14 +1163,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
       blk_dst[1] = bc_ok ? bits_to_f32<T>(r.C[g]) : 0.0f;
     }
     // a tile past the segment (i >= nt) writes nothing
-    const bool st_ok = pch_ok && i < nt;
-    if constexpr (kHasZ) {
-      if constexpr (kAligned)
-        buffer_store4<T>(dz_rsrc, (i < nt && t < L) ? row_off + (uint32_t)t * sizeof(T) : kOffDrop,
-                         dzo);
-      else
-        store4_nb<T, kAligned>(dzp + (rb + pch) * L, t, L, st_ok, dummy, dzo);
-    }
+    if constexpr (kHasZ) store_row4<T, kAligned>(dz_rsrc, row_off, t, i < nt ? L : 0, dzo);
   };
 
   float accD = 0.0f, accB = 0.0f;
@@ -1233,14 +1204,8 @@ __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
         accB += ddo[j];
       }
     }
-    if constexpr (kAligned) {
-      const uint32_t off = (ok && t < L) ? row_off + (uint32_t)t * sizeof(T) : kOffDrop;
-      buffer_store4<T>(du_rsrc, off, duo);
-      buffer_store4<T>(dd_rsrc, off, ddo);
-    } else {
-      store4_nb<T, kAligned>(dup + (rb + pch) * L, t, L, ok && pch_ok, dummy, duo);
-      store4_nb<T, kAligned>(ddp + (rb + pch) * L, t, L, ok && pch_ok, dummy, ddo);
-    }
+    store_row4<T, kAligned>(du_rsrc, row_off, t, ok ? L : 0, duo);
+    store_row4<T, kAligned>(dd_rsrc, row_off, t, ok ? L : 0, ddo);
   };
 
   // Iteration i after barrier i: finish tile i-1 (its slices were written
@@ -1660,7 +1625,6 @@ __global__ __launch_bounds__(kWsThreads, kSG == 1 && kAligned ? 6 : 5) void scan
   const int pch = d0 + row;
   const bool pch_ok = pch < Dm;
   const float Bias = (pch_ok && biasp) ? biasp[pch] : 0.0f;
-  const int chc = min(pch, Dm - 1);
   const size_t rb = (size_t)b * Dm;
   int vlo, vhi;
   valid_window(length, p.pad_right, b, L, vlo, vhi);
@@ -1678,51 +1642,42 @@ __global__ __launch_bounds__(kWsThreads, kSG == 1 && kAligned ? 6 : 5) void scan
   const int wrow0 = d0 + (w - kWsCons) * (kBlockCh / kWsProd);
   const uint32_t wbytes =
       (uint32_t)(max(0, min(kBlockCh / kWsProd, Dm - wrow0)) * (size_t)L * sizeof(T));
-  const uint32_t row_off = (uint32_t)((row % (kBlockCh / kWsProd)) * (size_t)L * sizeof(T));
-  const auto d_ld = raw_rsrc(const_cast<T*>(dl) + (rb + wrow0) * L, wbytes);
-  const auto y_ld = raw_rsrc(const_cast<T*>(dyp) + (rb + wrow0) * L, wbytes);
-  const auto z_ld = raw_rsrc(kHasZ ? const_cast<T*>(zp) + (rb + wrow0) * L : const_cast<T*>(dyp),
-                             kHasZ ? wbytes : 0u);
+  uint32_t row_off = (uint32_t)((row % (kBlockCh / kWsProd)) * (size_t)L * sizeof(T));
+  if constexpr (!kAligned) row_off = pch_ok ? row_off : kOffDrop;
+  using Range = RowRange<T, kAligned>;
+  const Range d_ld(dl + (rb + wrow0) * L, wbytes);
+  const Range y_ld(dyp + (rb + wrow0) * L, wbytes);
+  const Range z_ld(kHasZ ? zp + (rb + wrow0) * L : dyp, kHasZ ? wbytes : 0u);
   const auto C_ld = raw_rsrc(const_cast<T*>(Cp) + (size_t)b * p.bc_bstride,
                              (uint32_t)((size_t)N * L * sizeof(T)));
-  const T* __restrict__ d_row = dl + (rb + chc) * L;
-  const T* __restrict__ y_row = dyp + (rb + chc) * L;
-  const T* __restrict__ z_row = kHasZ ? zp + (rb + chc) * L : y_row;
 
   struct Rows {
-    typename Raw4<T>::type d, y, z;
+    typename RowRaw<T, kAligned>::type d, y, z;
     uint32_t C[kSG];
   };
   // raw loads of tile i, the step clamped into the row (tiles past the walk
   // load data that is never used)
   auto issue = [&](Rows& r, int i) {
     const int t0 = max(tile_t(i), 0);
-    if constexpr (kAligned) {
-      const uint32_t off = row_off + (uint32_t)min(t0 + 4 * q, L - 4) * sizeof(T);
-      r.d = buffer_load_raw4<T>(d_ld, off);
-      r.y = buffer_load_raw4<T>(y_ld, off);
-      if constexpr (kHasZ) r.z = buffer_load_raw4<T>(z_ld, off);
-      else r.z = typename Raw4<T>::type{};
+    const uint32_t off = row_off + (uint32_t)min(t0 + 4 * q, kAligned ? L - 4 : L - 1) * sizeof(T);
+    r.d = d_ld.load4(off);
+    r.y = y_ld.load4(off);
+    if constexpr (kHasZ) r.z = z_ld.load4(off);
+    else r.z = typename RowRaw<T, kAligned>::type{};
 #pragma unroll
-      for (int g = 0; g < kSG; ++g)
-        r.C[g] = buffer_load_bits1<T>(C_ld, (uint32_t)((c_row(g) + min(t0 + c_step, L - 1)) * sizeof(T)));
-    } else {
-      r.d = load_raw4_nb<T, kAligned>(d_row, t0 + 4 * q, L, pch_ok);
-      r.y = load_raw4_nb<T, kAligned>(y_row, t0 + 4 * q, L, pch_ok);
-      if constexpr (kHasZ) r.z = load_raw4_nb<T, kAligned>(z_row, t0 + 4 * q, L, pch_ok);
-      else r.z = typename Raw4<T>::type{};
-#pragma unroll
-      for (int g = 0; g < kSG; ++g)
-        r.C[g] = elem_bits(Cp[(size_t)b * p.bc_bstride + c_row(g) + min(t0 + c_step, L - 1)]);
-    }
+    for (int g = 0; g < kSG; ++g)
+      r.C[g] = buffer_load_bits1<T>(C_ld, (uint32_t)((c_row(g) + min(t0 + c_step, L - 1)) * sizeof(T)));
   };
   float dtsum = 0.0f;
   auto stage = [&](const Rows& r, int i, int sbuf) {
     const int t = tile_t(i) + 4 * q;
     float dv[4], yv[4], zv[4], de[4], dov[4];
-    decode4(r.d, dv);
-    decode4(r.y, yv);
-    if constexpr (kHasZ) decode4(r.z, zv);
+    Range::decode(r.d, d_ld.shift(row_off), dv);
+    Range::decode(r.y, y_ld.shift(row_off), yv);
+    if constexpr (kHasZ) {
+      Range::decode(r.z, z_ld.shift(row_off), zv);
+      if constexpr (!kAligned) Range::mask_end(zv, t, L);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const bool valid = t + j >= vlo && t + j < vhi;

@@ -402,16 +402,16 @@ constexpr int kWsRow = kBlockCh + 2;
 
 // One tile's raw loads of a producer lane, kept as loaded bits: converting
 // at the load would make the compiler wait for it right there.
-template <typename T, int kSG, bool kDt = false>
+template <typename T, int kSG, bool kAligned, bool kDt = false>
 struct WsRows {
-  typename Raw4<T>::type u, d, z;
+  typename RowRaw<T, kAligned>::type u, d, z;
   uint32_t B[kSG], C[kSG];  // element bits
 };
 // With the fused step-size projection: the tile's dt^T operand in place of
 // the delta row piece.
-template <typename T>
-struct WsRows<T, 1, true> {
-  typename Raw4<T>::type u, z;
+template <typename T, bool kAligned>
+struct WsRows<T, 1, kAligned, true> {
+  typename RowRaw<T, kAligned>::type u, z;
   uint32_t B[1], C[1];
   u32x4_v pa[kDtK];
 };
@@ -611,16 +611,10 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
   const bool pch_ok = pch < Dm;
   const float Dv = (pch_ok && Dp) ? Dp[pch] : 0.0f;
   const float Bias = (pch_ok && biasp) ? biasp[pch] : 0.0f;
-  // rows of the clamped channel (valid addresses; lanes past the last channel
-  // are masked to delta = 0 and never stored)
-  const int chc = min(pch, Dm - 1);
-  const T* __restrict__ u_row = u + (rb + chc) * L;
-  const T* __restrict__ d_row = dl + (rb + chc) * L;
   // kDt: z's batch rows may lie dtp.zbstride elements apart (the gate half of
   // the in-projection output, read in place); zb offsets z so that the row
   // arithmetic below, which assumes dim * L, lands on them
   const T* __restrict__ zb = kDt ? zp + (size_t)b * dtp.zbstride - (size_t)rb * L : zp;
-  const T* __restrict__ z_row = zb + (rb + chc) * L;
   int vlo, vhi;
   valid_window(length, p.pad_right, b, L, vlo, vhi);
   vhi = min(vhi, Lend);  // steps past the segment are identity steps here
@@ -634,25 +628,21 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
   const int bc_step = kDt ? (w - kWsCons) * 4 + (lane >> 4) : pt % kWsTile;
   // (state of pair group g; clamped into the rows, zeroed at staging past N)
   auto bc_n = [&](int g) { return 2 * (g * kWsCons + bc_G) + bc_half; };
-  const T* __restrict__ B_rows = Bp + (size_t)b * p.bc_bstride;
-  const T* __restrict__ C_rows = Cp + (size_t)b * p.bc_bstride;
 
-  // raw rows of tile i (clamped to the last tile; the loads of tiles past it
-  // are never used)
   // This wave's 16 channel rows (the launch guarantees 16 * L * sizeof(T) <
-  // 2^31, so the byte offsets fit): the aligned path loads and stores through
-  // buffer ranges over them, and loads B and C through ranges over the batch
-  // row's state rows, at 32-bit offsets (no 64-bit address arithmetic per
-  // tile).  The step is clamped into the row as on the pointer path; a row
-  // past the last channel reads zero.
+  // 2^31, so the byte offsets fit): loads and stores go through buffer ranges
+  // over them, and B and C through ranges over the batch row's state rows, at
+  // 32-bit offsets (no 64-bit address arithmetic per tile).  The step is
+  // clamped into the row; a row past the last channel reads zero.
+  using Range = RowRange<T, kAligned>;
   const int wrow0 = d0 + (w - kWsCons) * (kBlockCh / kWsProd);
   const uint32_t wbytes =
       (uint32_t)(max(0, min(kBlockCh / kWsProd, Dm - wrow0)) * (size_t)L * sizeof(T));
-  const uint32_t row_off = (uint32_t)((row % (kBlockCh / kWsProd)) * (size_t)L * sizeof(T));
-  const auto u_ld = raw_rsrc(const_cast<T*>(u) + ((size_t)rb + wrow0) * L, wbytes);
-  const auto d_ld = raw_rsrc(const_cast<T*>(dl) + ((size_t)rb + wrow0) * L, wbytes);
-  const auto z_ld = raw_rsrc(kHasZ ? const_cast<T*>(zb) + ((size_t)rb + wrow0) * L : const_cast<T*>(u),
-                             kHasZ ? wbytes : 0u);
+  uint32_t row_off = (uint32_t)((row % (kBlockCh / kWsProd)) * (size_t)L * sizeof(T));
+  if constexpr (!kAligned) row_off = pch_ok ? row_off : kOffDrop;
+  const Range u_ld(u + ((size_t)rb + wrow0) * L, wbytes);
+  const Range d_ld(dl + ((size_t)rb + wrow0) * L, wbytes);
+  const Range z_ld(kHasZ ? zb + ((size_t)rb + wrow0) * L : u, kHasZ ? wbytes : 0u);
   const uint32_t bc_bytes = (uint32_t)((size_t)N * L * sizeof(T));
   const auto B_ld = raw_rsrc(const_cast<T*>(Bp) + (size_t)b * p.bc_bstride, bc_bytes);
   const auto C_ld = raw_rsrc(const_cast<T*>(Cp) + (size_t)b * p.bc_bstride, bc_bytes);
@@ -693,9 +683,15 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
     }
   }
 
-  using Rows = WsRows<T, kSG, kDt != 0>;
+  using Rows = WsRows<T, kSG, kAligned, kDt != 0>;
   auto issue = [&](Rows& r, int i) {
+    // tile i, clamped to the last tile (the loads of tiles past it are never used)
     const int t0 = min(Tbeg + i * kWsTile, last_t0);
+    const uint32_t off =
+        row_off + (uint32_t)min(t0 + 4 * q, kAligned ? L - 4 : L - 1) * sizeof(T);
+    r.u = u_ld.load4(off);
+    if constexpr (kHasZ) r.z = z_ld.load4(off);
+    else r.z = typename RowRaw<T, kAligned>::type{};
     if constexpr (kDt) {
       const uint32_t tb = (uint32_t)t0 * prow_bytes;  // wave-uniform
 #pragma unroll
@@ -703,38 +699,13 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
         r.pa[s] = __builtin_amdgcn_raw_buffer_load_b128(pr_ld, (int)(tb + pa_off[s]), 0, 0);
       r.B[0] = buffer_load_bits1<T>(pr_ld, tb + pbc_off);
       r.C[0] = buffer_load_bits1<T>(pr_ld, tb + pbc_off + (uint32_t)N * 2u);
-      if constexpr (kAligned) {
-        const uint32_t off = row_off + (uint32_t)min(t0 + 4 * q, L - 4) * sizeof(T);
-        r.u = buffer_load_raw4<T>(u_ld, off);
-        if constexpr (kHasZ) r.z = buffer_load_raw4<T>(z_ld, off);
-        else r.z = typename Raw4<T>::type{};
-      } else {
-        r.u = load_raw4_nb<T, kAligned>(u_row, t0 + 4 * q, L, pch_ok);
-        if constexpr (kHasZ) r.z = load_raw4_nb<T, kAligned>(z_row, t0 + 4 * q, L, pch_ok);
-        else r.z = typename Raw4<T>::type{};
-      }
-    } else if constexpr (kAligned) {
-      const uint32_t off = row_off + (uint32_t)min(t0 + 4 * q, L - 4) * sizeof(T);
-      r.u = buffer_load_raw4<T>(u_ld, off);
-      r.d = buffer_load_raw4<T>(d_ld, off);
-      if constexpr (kHasZ) r.z = buffer_load_raw4<T>(z_ld, off);
-      else r.z = typename Raw4<T>::type{};
+    } else {
+      r.d = d_ld.load4(off);
 #pragma unroll
       for (int g = 0; g < kSG; ++g) {
         const uint32_t boff = bc_row_off[g] + (uint32_t)min(t0 + bc_step, L - 1) * sizeof(T);
         r.B[g] = buffer_load_bits1<T>(B_ld, boff);
         r.C[g] = buffer_load_bits1<T>(C_ld, boff);
-      }
-    } else {
-      r.u = load_raw4_nb<T, kAligned>(u_row, t0 + 4 * q, L, pch_ok);
-      r.d = load_raw4_nb<T, kAligned>(d_row, t0 + 4 * q, L, pch_ok);
-      if constexpr (kHasZ) r.z = load_raw4_nb<T, kAligned>(z_row, t0 + 4 * q, L, pch_ok);
-      else r.z = typename Raw4<T>::type{};
-#pragma unroll
-      for (int g = 0; g < kSG; ++g) {
-        const size_t tb = (size_t)min(bc_n(g), N - 1) * L + min(t0 + bc_step, L - 1);
-        r.B[g] = elem_bits(B_rows[tb]);
-        r.C[g] = elem_bits(C_rows[tb]);
       }
     }
   };
@@ -768,7 +739,7 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
     const int t_tile = Tbeg + i * kWsTile;
     const int t = t_tile + 4 * q;
     float uv[4], dv[4], de[4], du[4];
-    decode4(r.u, uv);
+    Range::decode(r.u, u_ld.shift(row_off), uv);
     if constexpr (kDt) {
       // this lane's row (channel lane % 16) and 4-step column (lane / 16),
       // rounded to bf16
@@ -795,11 +766,11 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
         }
       }
     } else {
-      decode4(r.d, dv);
+      Range::decode(r.d, d_ld.shift(row_off), dv);
     }
     if constexpr (kHasZ) {
       float zv[4];
-      decode4(r.z, zv);
+      Range::decode(r.z, z_ld.shift(row_off), zv);
 #pragma unroll
       for (int j = 0; j < 4; ++j) gt[j] = silu_f(zv[j]);
     }
@@ -821,6 +792,8 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
         const uint32_t keep = (t + j >= vlo && t + j < vhi) ? 0xffffffffu : 0u;
         de[j] = __uint_as_float(__float_as_uint(de[j]) & keep);
       }
+      // u past the end is another row's: zero, so that delta * u is
+      if constexpr (!kAligned) Range::mask_end(uv, t, L);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) du[j] = de[j] * uv[j];
@@ -855,25 +828,12 @@ __global__ __launch_bounds__(kWsThreads) void scan_fwd_ws_kernel(
       acc.x += v[ww].x; acc.y += v[ww].y; acc.z += v[ww].z; acc.w += v[ww].w;
     }
     float y[4] = {sk[0] + acc.x, sk[1] + acc.y, sk[2] + acc.z, sk[3] + acc.w};
-    if constexpr (kAligned) {
-      // range-checked stores: rows past the last channel lie outside the
-      // wave's buffer range, and steps past the segment get an offset past it
-      const uint32_t off = t < Lend ? row_off + (uint32_t)t * sizeof(T) : kOffDrop;
-      if constexpr (kSaveY) buffer_store4<T>(yu_rsrc, off, y);
-      if constexpr (kHasZ) {
+    if constexpr (kSaveY) store_row4<T, kAligned>(yu_rsrc, row_off, t, Lend, y);
+    if constexpr (kHasZ) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) y[j] *= gt[j];
-      }
-      buffer_store4<T>(out_rsrc, off, y);
-    } else {
-      const bool st_ok = pch_ok && t < Lend;
-      if constexpr (kSaveY) store4_nb<T, kAligned>(yu + (rb + pch) * L, t, L, st_ok, dummy, y);
-      if constexpr (kHasZ) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) y[j] *= gt[j];
-      }
-      store4_nb<T, kAligned>(out + (rb + pch) * L, t, L, st_ok, dummy, y);
+      for (int j = 0; j < 4; ++j) y[j] *= gt[j];
     }
+    store_row4<T, kAligned>(out_rsrc, row_off, t, Lend, y);
   };
 
   // Aligned rows: the outputs of four consecutive tiles go to the wave's

@@ -242,6 +242,112 @@ __device__ __forceinline__ void buffer_store4(__amdgpu_buffer_rsrc_t r, uint32_t
   }
 }
 
+// ---------------------------------------------------------------- rows through buffer ranges
+
+// Four consecutive elements of a channel row, read through a buffer range over
+// a wave's rows.  kAligned: rows of a multiple of 16 bytes at 16-byte aligned
+// addresses, one 8-byte (bf16) or 16-byte (fp32) load.  Otherwise any element
+// alignment: fp32 reads its 16 bytes at dword alignment; bf16 the three dwords
+// that hold its 8 bytes, shifted into place when decoded (two v_alignbyte), so
+// that no access is misaligned and none touches a dword without an element of
+// the range.  Element by element with a bounds check each, as these rows were
+// read before, a wave issued four loads a piece behind four branches: at (3,
+// 1000, 1531) in bf16 with the gate the scan's forward took 104 us and its
+// backward 160, now 41 and 79 (1536 steps, aligned: 35 and 70); the summary
+// kernels 33 and 64, now 18 and 21.
+// Elements past the row's end are the next row's, or zero past the range: the
+// caller masks what they reach.  A row past the last channel must be given an
+// offset past the range (kOffDrop): the range of unaligned bf16 rows ends with
+// a dword, which may hold one element more.
+struct Raw3 { uint32_t x, y, z; };
+template <typename T, bool kAligned> struct RowRaw { using type = typename Raw4<T>::type; };
+template <> struct RowRaw<__hip_bfloat16, false> { using type = Raw3; };
+
+template <typename T, bool kAligned>
+struct RowRange {
+  static constexpr bool kShift = !kAligned && sizeof(T) == 2;
+  __amdgpu_buffer_rsrc_t r;
+  uint32_t extra;  // bytes from the range's (dword aligned) base to the first row: 0 or 2
+
+  __device__ __forceinline__ RowRange(const T* base, uint32_t bytes) {
+    extra = 0;
+    if constexpr (kShift) {
+      const uint64_t a = reinterpret_cast<uint64_t>(base);
+      extra = __builtin_amdgcn_readfirstlane((uint32_t)a & 2u);
+      r = raw_rsrc(reinterpret_cast<void*>(a & ~(uint64_t)3), bytes ? (extra + bytes + 3u) & ~3u : 0u);
+    } else {
+      r = raw_rsrc(const_cast<T*>(base), bytes);
+    }
+  }
+  // byte shift of a row whose first byte is row_off past the first row
+  __device__ __forceinline__ uint32_t shift(uint32_t row_off) const { return (extra + row_off) & 3u; }
+
+  __device__ __forceinline__ typename RowRaw<T, kAligned>::type load4(uint32_t off) const {
+    if constexpr (kShift) {
+      typedef unsigned int u32x3_v __attribute__((ext_vector_type(3)));
+      const u32x3_v v = __builtin_amdgcn_raw_buffer_load_b96(r, (int)((extra + off) & ~3u), 0, 0);
+      return Raw3{v.x, v.y, v.z};
+    } else {
+      return buffer_load_raw4<T>(r, off);
+    }
+  }
+  // the four elements' own bits
+  __device__ __forceinline__ static typename Raw4<T>::type bits(
+      const typename RowRaw<T, kAligned>::type& q, uint32_t shift) {
+    if constexpr (kShift)
+      return make_uint2(__builtin_amdgcn_alignbyte(q.y, q.x, shift),
+                        __builtin_amdgcn_alignbyte(q.z, q.y, shift));
+    else
+      return q;
+  }
+  __device__ __forceinline__ static void decode(const typename RowRaw<T, kAligned>::type& q,
+                                                uint32_t shift, float (&v)[4]) {
+    decode4(bits(q, shift), v);
+  }
+  // (unaligned rows) zero the elements of the piece at t that lie at or past
+  // `end`: they are the next row's
+  __device__ __forceinline__ static void mask_end(float (&v)[4], int t, int end) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      v[j] = __uint_as_float(__float_as_uint(v[j]) & (t + j < end ? ~0u : 0u));
+  }
+  __device__ __forceinline__ static void mask_end(uint2& q, int t, int end) {
+    q.x &= (t < end ? 0xffffu : 0u) | (t + 1 < end ? 0xffff0000u : 0u);
+    q.y &= (t + 2 < end ? 0xffffu : 0u) | (t + 3 < end ? 0xffff0000u : 0u);
+  }
+  __device__ __forceinline__ static void mask_end(uint4& q, int t, int end) {
+    q.x &= t < end ? ~0u : 0u;
+    q.y &= t + 1 < end ? ~0u : 0u;
+    q.z &= t + 2 < end ? ~0u : 0u;
+    q.w &= t + 3 < end ? ~0u : 0u;
+  }
+};
+
+// Four elements from column t of the row at byte row_off of a range over a
+// wave's rows, those below `end` (aligned rows: all or none of them).  Range-
+// checked stores with no branch: a dropped element gets an offset past the
+// range, as do rows past the last channel.
+template <typename T, bool kAligned>
+__device__ __forceinline__ void store_row4(__amdgpu_buffer_rsrc_t r, uint32_t row_off, int t, int end,
+                                           const float (&v)[4]) {
+  if constexpr (kAligned) {
+    buffer_store4<T>(r, t < end ? row_off + (uint32_t)t * sizeof(T) : kOffDrop, v);
+  } else {
+    const uint32_t p01 = sizeof(T) == 2 ? pack_bf16x2(v[0], v[1]) : 0u;
+    const uint32_t p23 = sizeof(T) == 2 ? pack_bf16x2(v[2], v[3]) : 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t off = t + j < end ? row_off + (uint32_t)(t + j) * sizeof(T) : kOffDrop;
+      if constexpr (sizeof(T) == 4) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j]), r, (int)off, 0, 0);
+      } else {
+        const uint32_t w = j < 2 ? p01 : p23;
+        __builtin_amdgcn_raw_buffer_store_b16((unsigned short)(j & 1 ? w >> 16 : w), r, (int)off, 0, 0);
+      }
+    }
+  }
+}
+
 // Wait until every outstanding LDS and scalar-memory load of this wave has
 // returned (s_waitcnt lgkmcnt(0)) and keep the scheduler from moving
 // instructions across this point.  Orders "consume block k" before "issue

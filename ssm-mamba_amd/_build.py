@@ -5,7 +5,8 @@
   shared object exporting the C ABI of include/ssm_mamba.h;
 * the PyTorch-ROCm extension modules ``_ext/selective_scan`` and
   ``_ext/selective_update`` (host C++ over that C ABI, the counterparts of
-  the reference's compiled modules), compiled with the host compiler against
+  the reference's compiled modules) and ``_ext/decode_step`` (the host work of
+  the model harness's decode step), compiled with the host compiler against
   torch's headers and linked to the HIP library (rpath ``$ORIGIN/../_lib``).
 """
 from __future__ import annotations
@@ -25,7 +26,7 @@ LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
 SOURCES = ["scan_fwd.hip", "scan_bwd.hip", "state_update.hip", "conv1d.hip", "decode.hip",
            "decode_rows.hip", "layout.hip", "norm.hip", "capi.hip"]
 EXT_DIR = os.path.join(PKG_DIR, "_ext")
-EXT_MODULES = ["selective_scan", "selective_update"]
+EXT_MODULES = ["selective_scan", "selective_update", "decode_step"]
 EXT_SUFFIX = sysconfig.get_config_var("EXT_SUFFIX") or ".so"
 
 
@@ -91,7 +92,7 @@ def _run(cmd, what):
 
 def build(verbose: bool = True, jobs: int = 4) -> str:
     """Compile every .hip source for gfx950 and link the shared library, then
-    the two extension modules against it.  Always rebuilds.  Returns the
+    the extension modules against it.  Always rebuilds.  Returns the
     library path."""
     os.makedirs(LIB_DIR, exist_ok=True)
     os.makedirs(EXT_DIR, exist_ok=True)

@@ -5,9 +5,11 @@
   argument order (``csrc/selective_scan/bindings.cpp:5-8``), plus the
   extended ``fwd_ext`` / ``bwd_ext``;
 * ``selective_update`` -- ``apply`` (``csrc/selective_update/bindings.cpp:5-7``)
-  plus ``apply_ext``.
+  plus ``apply_ext``;
+* ``decode_step``      -- the checks, addresses and launches of a decode step
+  of the model harness.
 
-Both are host C++ over the C ABI of ``_lib/libssm_mamba_hip.so``.  With this
+All are host C++ over the C ABI of ``_lib/libssm_mamba_hip.so``.  With this
 directory on ``sys.path`` they import under the reference's top-level names
 (``import selective_scan``), which is how the reference's ``ops/`` files find
 them.  There is no fallback: a missing module raises.
@@ -22,7 +24,7 @@ _mods = {}
 
 
 def module(name: str):
-    """The built extension module ``name`` (selective_scan or selective_update)."""
+    """The built extension module ``name`` (one of those above)."""
     m = _mods.get(name)
     if m is None:
         try:

@@ -485,6 +485,9 @@ class Block(nn.Module):
         return x + self.dropout(y), last
 
     def step(self, hidden_states: torch.Tensor) -> torch.Tensor:
+        out = _dec.plain_block_step(self, hidden_states, _LAYER_CLASSES)
+        if out is not None:
+            return out
         if _dec.block_step_supported(self.ssm, hidden_states, self.norm.weight):
             # norm, mixer and residual in the four fused decode kernels
             return _dec.block_step(self.ssm, hidden_states, self.norm.weight, self.norm.eps,
@@ -495,6 +498,10 @@ class Block(nn.Module):
             return _dec.rows_block_step(self.ssm, hidden_states, self.norm.weight, self.norm.eps,
                                         residual=True)
         return hidden_states + self.ssm.step(self.norm(hidden_states))
+
+
+# the classes a layer is made of, for the native step
+_LAYER_CLASSES = (Block, Mamba, RMSNorm, nn.Linear, nn.Conv1d, nn.ModuleList)
 
 
 @dataclass
@@ -604,9 +611,10 @@ class CausalLM(nn.Module):
     def step(self, input_ids: torch.Tensor) -> torch.Tensor:
         """input_ids (batch,) -> logits (batch, vocab), advancing every cache."""
         x = self.embedding(input_ids)
-        if _dec.layers_supported(self.layers, x):
+        ptrs = _dec.plain_layer_rows(self.layers, x, _LAYER_CLASSES)
+        if ptrs is not None or _dec.layers_supported(self.layers, x):
             # every layer's step in one launch
-            x = _dec.layers_step(self, self.layers, x)
+            x = _dec.layers_step(self, self.layers, x, ptrs)
             if not torch.cuda.is_current_stream_capturing():
                 _dec.layers_check(self)
         else:

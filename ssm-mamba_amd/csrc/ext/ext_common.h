@@ -1,5 +1,5 @@
-// Shared host code of the two PyTorch-ROCm extension modules (selective_scan,
-// selective_update): validation with the reference's messages, the device
+// Shared host code of the PyTorch-ROCm extension modules (selective_scan,
+// selective_update, decode_step): validation with the reference's messages, the device
 // guard and current stream, and the call into the C ABI of
 // libssm_mamba_hip.so (include/ssm_mamba.h).  No device code lives here.
 #pragma once

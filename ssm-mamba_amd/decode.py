@@ -12,10 +12,12 @@ otherwise.
 from __future__ import annotations
 
 import ctypes
+from array import array
 from typing import Optional
 
 import torch
 
+from . import _ext as _E
 from . import _native as N
 
 _DTYPES = {torch.float32: N.SSM_F32, torch.bfloat16: N.SSM_BF16}
@@ -198,6 +200,24 @@ def _step_supported(linear_supported, ssm, x, norm_weight) -> bool:
     return True
 
 
+def plain_block_step(block, x: torch.Tensor, classes) -> Optional[torch.Tensor]:
+    """Block.step of a layer built of exactly ``classes`` (Block, Mamba,
+    RMSNorm, Linear, Conv1d, ModuleList), checked and launched in native code;
+    None leaves the call to the checks above."""
+    if not ENABLED or not x.is_cuda:
+        return None
+    return _E.module("decode_step").block_step(block, x, classes, FOLD_XPROJ,
+                                               not torch.is_autocast_enabled())
+
+
+def plain_layer_rows(layers, x: torch.Tensor, classes) -> Optional[bytes]:
+    """``layers_supported`` and the layers' addresses (LayerChain.update) in
+    native code, for layers of exactly ``classes``; None: ask layers_supported."""
+    if not (ENABLED and LAYER_CHAIN and FOLD_XPROJ) or not x.is_cuda:
+        return None
+    return _E.module("decode_step").layer_rows(layers, x, classes)
+
+
 def block_step(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tensor] = None,
                eps: float = 1e-6, residual: bool = False) -> torch.Tensor:
     """Mamba.step(norm(x)) (+ x when residual): the fused path of
@@ -335,19 +355,24 @@ class LayerChain:
         self.workspace = torch.zeros(nbytes, dtype=torch.uint8, device=x.device)
         self.ptrs = None
         self.table = None
-        self.tables = {}  # pointer tuple -> device table; never pruned
+        self.tables = {}  # addresses (packed) -> device table; never pruned
 
-    def update(self, layers) -> None:
-        ptrs = tuple(0 if t is None else t.data_ptr() for blk in layers for t in _layer_tensors(blk))
+    def update(self, layers, ptrs: Optional[bytes] = None) -> None:
+        """Switch to the table of the layers' addresses (``ptrs`` when the
+        caller has them: 64 bits each, layer by layer in the header's order)."""
+        if ptrs is None:
+            ptrs = array("q", [0 if t is None else t.data_ptr()
+                               for blk in layers for t in _layer_tensors(blk)]).tobytes()
         if ptrs != self.ptrs:
             table = self.tables.get(ptrs)
             if table is None:
-                table = self.tables[ptrs] = torch.tensor(ptrs, dtype=torch.int64).to(self.device)
+                table = torch.frombuffer(bytearray(ptrs), dtype=torch.int64).to(self.device)
+                self.tables[ptrs] = table
             self.table = table
             self.ptrs = ptrs
 
-    def step(self, layers, x: torch.Tensor) -> torch.Tensor:
-        self.update(layers)
+    def step(self, layers, x: torch.Tensor, ptrs: Optional[bytes] = None) -> torch.Tensor:
+        self.update(layers, ptrs)
         out = torch.empty_like(x)
         with torch.cuda.device(x.device):
             N.check(N.lib().ssm_decode_layers(
@@ -365,16 +390,16 @@ class LayerChain:
                                                      _stream(self.device)))
 
 
-def layers_step(owner, layers, x: torch.Tensor) -> torch.Tensor:
+def layers_step(owner, layers, x: torch.Tensor, ptrs: Optional[bytes] = None) -> torch.Tensor:
     """x after Block.step of every layer in ``layers`` (one launch); the
     layers' caches advance in place.  ``owner`` keeps the LayerChain objects
-    (one per device, batch and dtype)."""
+    (one per device, batch and dtype); ``ptrs`` as in LayerChain.update."""
     chains = owner.__dict__.setdefault("_layer_chains", {})
     key = (x.device, x.shape[0], x.dtype)
     chain = chains.get(key)
     if chain is None:
         chain = chains[key] = LayerChain(layers, x)
-    return chain.step(layers, x)
+    return chain.step(layers, x, ptrs)
 
 
 _PICK_WS = {}

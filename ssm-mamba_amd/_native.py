@@ -9,6 +9,9 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+from contextlib import nullcontext
+
+import torch
 
 from ._build import LIB_PATH
 
@@ -174,6 +177,20 @@ def lib() -> ctypes.CDLL:
                 raise RuntimeError("ssm_mamba_amd: HIP library ABI version mismatch; rebuild it")
             _lib = l
     return _lib
+
+
+_HERE = nullcontext()
+
+
+def on(dev: torch.device):
+    """``torch.cuda.device(dev)`` for a tensor's device, and nothing where that
+    is the current one (with ``stream``: 4 us a launch less)."""
+    return _HERE if dev.index == torch._C._cuda_getDevice() else torch.cuda.device(dev)
+
+
+def stream(dev: torch.device) -> int:
+    """The current HIP stream of a tensor's device."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def profile_begin() -> None:

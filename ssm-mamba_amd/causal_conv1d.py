@@ -18,10 +18,6 @@ from . import _native as N
 _DTYPES = {torch.float32: N.SSM_F32, torch.bfloat16: N.SSM_BF16}
 
 
-def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
 def _check_x(x: torch.Tensor) -> None:
     if x.dim() != 3:
         raise RuntimeError("x must be a 3D tensor (batch, channels, seq_len)")
@@ -65,14 +61,14 @@ class CausalConv1dFn(torch.autograd.Function):
                 raise RuntimeError("lengths must be an int64 (batch,) tensor on x's device")
             lengths = lengths.contiguous()
         L = N.lib()
-        with torch.cuda.device(x.device):
+        with N.on(x.device):
             N.check(L.ssm_causal_conv1d_fwd(batch, dim, seqlen, width, _DTYPES[x.dtype],
                                             x.data_ptr(), xbs, w.data_ptr(),
                                             None if b is None else b.data_ptr(), int(silu),
                                             out.data_ptr(),
                                             None if lengths is None else lengths.data_ptr(),
                                             None if window is None else window.data_ptr(),
-                                            _stream(x.device)))
+                                            N.stream(x.device)))
         ctx.save_for_backward(x, w, b)
         ctx.silu = silu
         ctx.weight_shape = weight.shape
@@ -93,13 +89,13 @@ class CausalConv1dFn(torch.autograd.Function):
         L = N.lib()
         nbytes = L.ssm_causal_conv1d_bwd_workspace_bytes(batch, dim, width)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-        with torch.cuda.device(x.device):
+        with N.on(x.device):
             N.check(L.ssm_causal_conv1d_bwd(batch, dim, seqlen, width, _DTYPES[x.dtype],
                                             x.data_ptr(), w.data_ptr(),
                                             None if b is None else b.data_ptr(), dout.data_ptr(),
                                             int(ctx.silu), dx.data_ptr(), dw.data_ptr(),
                                             None if db is None else db.data_ptr(), ws.data_ptr(),
-                                            nbytes, _stream(x.device)))
+                                            nbytes, N.stream(x.device)))
         dw = dw.reshape(ctx.weight_shape).to(ctx.weight_dtype)
         if db is not None:
             db = db.to(ctx.bias_dtype)

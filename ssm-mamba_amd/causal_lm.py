@@ -82,11 +82,11 @@ def rms_norm_cm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tens
     x = x.contiguous()
     out = torch.empty_like(x)
     batch, ch, seqlen = x.shape
-    with torch.cuda.device(x.device):
+    with _N.on(x.device):
         _N.check(_N.lib().ssm_rms_norm_cm(batch, ch, seqlen, _DTYPES[x.dtype], x.data_ptr(),
                                           weight.contiguous().data_ptr(), float(eps),
                                           out.data_ptr(),
-                                          torch.cuda.current_stream(x.device).cuda_stream))
+                                          _N.stream(x.device)))
     return out
 
 
@@ -255,12 +255,12 @@ class Mamba(nn.Module):
         ws = torch.empty(lib.ssm_scan_fwd_workspace_bytes(batch, inner, seqlen, nstate),
                          dtype=torch.uint8, device=xc.device)
         ptr = lambda t: None if t is None else t.data_ptr()
-        with torch.cuda.device(xc.device):
+        with _N.on(xc.device):
             _N.check(lib.ssm_selective_scan_fwd_dt_proj(
                 batch, inner, seqlen, nstate, rank, _N.SSM_BF16, xc.data_ptr(), params.data_ptr(),
                 0, self.delta_proj.weight.data_ptr(), A.data_ptr(), ptr(D), ptr(dt_bias), ptr(h0),
                 ptr(lengths), 0, z.data_ptr(), zbs, 1, out.data_ptr(), None, last.data_ptr(),
-                ws.data_ptr(), ws.numel(), torch.cuda.current_stream(xc.device).cuda_stream))
+                ws.data_ptr(), ws.numel(), _N.stream(xc.device)))
         return out, last
 
     # ---- caches ---------------------------------------------------------

@@ -44,10 +44,6 @@ def _ptr(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
 
-def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
 def _aligned(t: torch.Tensor) -> bool:
     return t.data_ptr() % 16 == 0
 
@@ -60,10 +56,10 @@ def gemv(weight: torch.Tensor, x: torch.Tensor, norm_weight: Optional[torch.Tens
     batch, k = x.shape
     o = weight.shape[0]
     y = torch.empty(batch, o, device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
+    with N.on(x.device):
         N.check(N.lib().ssm_decode_gemv(batch, o, k, _DTYPES[x.dtype], weight.data_ptr(),
                                         x.data_ptr(), _ptr(norm_weight), float(eps), _ptr(bias),
-                                        _ptr(residual), y.data_ptr(), _stream(x.device)))
+                                        _ptr(residual), y.data_ptr(), N.stream(x.device)))
     return y
 
 
@@ -92,13 +88,13 @@ def in_proj_conv(weight: torch.Tensor, x: torch.Tensor, norm_weight: Optional[to
         if not nparts:
             raise RuntimeError(f"the x-projection cannot be folded at dim {dim}, params_dim {nout}")
         part = torch.empty(nparts, batch, (nout + 3) // 4 * 4, device=x.device, dtype=torch.float32)
-    with torch.cuda.device(x.device):
+    with N.on(x.device):
         N.check(N.lib().ssm_decode_in_proj_conv(batch, dim, k, width, _DTYPES[x.dtype],
                                                 weight.data_ptr(), x.data_ptr(), _ptr(norm_weight),
                                                 float(eps), _ptr(bias), conv_weight.data_ptr(),
                                                 _ptr(conv_bias), window.data_ptr(), xz.data_ptr(),
                                                 xc.data_ptr(), _ptr(x_proj_weight), nout,
-                                                _ptr(part), _stream(x.device)))
+                                                _ptr(part), N.stream(x.device)))
     return (xz, xc) if part is None else (xz, xc, part)
 
 
@@ -112,12 +108,12 @@ def ssm_step(params: torch.Tensor, rank: int, dt_proj_weight: torch.Tensor,
     nstate = state.shape[-1]
     blocks = params.shape[0] if params.dim() == 3 else 0
     y = torch.empty_like(xc)
-    with torch.cuda.device(xc.device):
+    with N.on(xc.device):
         N.check(N.lib().ssm_decode_ssm_step(batch, dim, nstate, rank, _DTYPES[xc.dtype],
                                             params.data_ptr(), blocks, dt_proj_weight.data_ptr(),
                                             _ptr(dt_bias), log_A.data_ptr(), _ptr(D),
                                             xc.data_ptr(), xz.data_ptr(), xz.stride(0),
-                                            state.data_ptr(), y.data_ptr(), _stream(xc.device)))
+                                            state.data_ptr(), y.data_ptr(), N.stream(xc.device)))
     return y
 
 
@@ -243,11 +239,11 @@ def rows_linear(weight: torch.Tensor, x: torch.Tensor, norm_weight: Optional[tor
     batch, k = x.shape
     o = weight.shape[0]
     y = torch.empty(batch, o, device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
+    with N.on(x.device):
         N.check(N.lib().ssm_decode_rows_linear(batch, o, k, _DTYPES[x.dtype], weight.data_ptr(),
                                                x.data_ptr(), _ptr(norm_weight), float(eps),
                                                _ptr(bias), _ptr(residual), y.data_ptr(),
-                                               _stream(x.device)))
+                                               N.stream(x.device)))
     return y
 
 
@@ -264,11 +260,11 @@ def rows_block_step(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tensor] = 
                      dtype=torch.uint8, device=x.device)
     tensors = _mixer_tensors(ssm, norm_weight)  # held until the launches are enqueued
     ptrs = (ctypes.c_void_p * _LAYER_NPTR)(*(_ptr(t) for t in tensors))
-    with torch.cuda.device(x.device):
+    with N.on(x.device):
         N.check(lib.ssm_decode_rows_block(batch, model_dim, dim, nstate, rank, ssm.conv_kernel,
                                           _DTYPES[x.dtype], ctypes.cast(ptrs, ctypes.c_void_p),
                                           x.data_ptr(), out.data_ptr(), float(eps), int(residual),
-                                          ws.data_ptr(), ws.numel(), _stream(x.device)))
+                                          ws.data_ptr(), ws.numel(), N.stream(x.device)))
     return out
 
 
@@ -374,20 +370,20 @@ class LayerChain:
     def step(self, layers, x: torch.Tensor, ptrs: Optional[bytes] = None) -> torch.Tensor:
         self.update(layers, ptrs)
         out = torch.empty_like(x)
-        with torch.cuda.device(x.device):
+        with N.on(x.device):
             N.check(N.lib().ssm_decode_layers(
                 self.batch, len(layers), self.model_dim, self.dim, _CHAIN_STATE, self.rank,
                 self.width, _DTYPES[x.dtype], self.table.data_ptr(), x.data_ptr(), out.data_ptr(),
-                self.eps, self.workspace.data_ptr(), self.workspace.numel(), _stream(x.device)))
+                self.eps, self.workspace.data_ptr(), self.workspace.numel(), N.stream(x.device)))
         return out
 
     def check(self) -> None:
         """Synchronise and raise if a grid barrier of an earlier launch timed
         out (the outputs since the last check are then invalid)."""
-        with torch.cuda.device(self.device):
+        with N.on(self.device):
             N.check(N.lib().ssm_decode_layers_status(self.workspace.data_ptr(),
                                                      self.workspace.numel(),
-                                                     _stream(self.device)))
+                                                     N.stream(self.device)))
 
 
 def layers_step(owner, layers, x: torch.Tensor, ptrs: Optional[bytes] = None) -> torch.Tensor:
@@ -430,12 +426,12 @@ def pick(probs: torch.Tensor, token: torch.Tensor, tokens: Optional[torch.Tensor
     need = int(N.lib().ssm_decode_pick_workspace(MAX_BATCH))
     if ws is None:
         ws = _PICK_WS[probs.device] = torch.zeros(need, dtype=torch.uint8, device=probs.device)
-    with torch.cuda.device(probs.device):
+    with N.on(probs.device):
         N.check(N.lib().ssm_decode_pick(
             batch, vocab, _DTYPES[probs.dtype], probs.data_ptr(), token.data_ptr(), _ptr(tokens),
             tokens.stride(0) if tokens is not None else 0,
             tokens.shape[1] if tokens is not None else 0, _ptr(pos), ws.data_ptr(), ws.numel(),
-            _stream(probs.device)))
+            N.stream(probs.device)))
 
 
 def layers_check(owner) -> None:

@@ -203,11 +203,21 @@ def supported(block, x: torch.Tensor) -> bool:
     """Whether token-major x through ``block`` takes the fused layer: float32 or
     bfloat16 on the GPU with every projection weight in x's dtype, no
     projection biases, a width the norm kernel takes, no autocast."""
-    ssm, w = block.ssm, block.norm.weight
+    w = block.norm.weight
     if torch.is_autocast_enabled() or not _lay.norm_tc_supported(x, w):
         return False
-    if ssm.input_proj.bias is not None or ssm.out_proj.bias is not None:
-        return False
-    return all(p.dtype == x.dtype and p.device == x.device
-               for p in (ssm.input_proj.weight, ssm.ssm_param_proj.weight, ssm.delta_proj.weight,
-                         ssm.out_proj.weight, ssm.conv.weight))
+    # read where nn.Module keeps them: a weight that is not a plain parameter
+    # (parametrized, computed by a hook) is not there and takes the other path
+    mods, dtype, dev = block.ssm._modules, x.dtype, x.device
+    for name in _PROJECTIONS:
+        params = mods[name]._parameters
+        p = params.get("weight")
+        if p is None or p.dtype != dtype or p.device != dev:
+            return False
+        if name in _NO_BIAS and params.get("bias") is not None:
+            return False
+    return True
+
+
+_PROJECTIONS = ("input_proj", "conv", "ssm_param_proj", "delta_proj", "out_proj")
+_NO_BIAS = ("input_proj", "out_proj")

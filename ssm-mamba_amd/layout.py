@@ -15,10 +15,6 @@ DTYPES = {torch.float32: N.SSM_F32, torch.bfloat16: N.SSM_BF16}
 _MAX_CHANNELS = {torch.float32: 1024, torch.bfloat16: 2048}
 
 
-def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
 def norm_tc_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether ``norm_tc`` takes token-major x (batch, seq_len, channels)."""
     if not (x.is_cuda and x.dim() == 3 and x.dtype in DTYPES and x.numel() > 0):
@@ -44,11 +40,11 @@ def norm_tc(x: torch.Tensor, weight: torch.Tensor, eps: float, token_major: bool
     h = torch.empty(batch, ch, seqlen, dtype=x.dtype, device=x.device)
     h_tm = torch.empty_like(x) if token_major else None
     rstd = torch.empty(batch, seqlen, dtype=torch.float32, device=x.device) if token_major else None
-    with torch.cuda.device(x.device):
+    with N.on(x.device):
         N.check(N.lib().ssm_rms_norm_tc_fwd(
             batch, seqlen, ch, DTYPES[x.dtype], x.data_ptr(), weight.data_ptr(), float(eps),
             h.data_ptr(), None if h_tm is None else h_tm.data_ptr(),
-            None if rstd is None else rstd.data_ptr(), _stream(x.device)))
+            None if rstd is None else rstd.data_ptr(), N.stream(x.device)))
     return h, h_tm, rstd, x
 
 
@@ -63,11 +59,11 @@ def norm_tc_backward(x: torch.Tensor, weight: torch.Tensor, rstd: torch.Tensor, 
     lib = N.lib()
     ws = torch.empty(lib.ssm_rms_norm_tc_bwd_workspace_bytes(batch, seqlen, ch), dtype=torch.uint8,
                      device=x.device)
-    with torch.cuda.device(x.device):
+    with N.on(x.device):
         N.check(lib.ssm_rms_norm_tc_bwd(
             batch, seqlen, ch, DTYPES[x.dtype], x.data_ptr(), weight.data_ptr(), rstd.data_ptr(),
             dh.data_ptr(), None if dres is None else dres.data_ptr(), dx.data_ptr(), dw.data_ptr(),
-            ws.data_ptr(), ws.numel(), _stream(x.device)))
+            ws.data_ptr(), ws.numel(), N.stream(x.device)))
     return dx, dw
 
 
@@ -82,10 +78,10 @@ def transposed(x: torch.Tensor) -> torch.Tensor:
     if x.stride(2) != 1 or x.stride(1) != cols or (batch > 1 and x.stride(0) < rows * cols):
         x = x.contiguous()
     out = torch.empty(batch, cols, rows, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with N.on(x.device):
         N.check(N.lib().ssm_transpose(batch, rows, cols, DTYPES[x.dtype], x.data_ptr(),
                                       0 if batch == 1 else x.stride(0), out.data_ptr(),
-                                      _stream(x.device)))
+                                      N.stream(x.device)))
     return out
 
 
@@ -97,7 +93,7 @@ def batch_sum(x: torch.Tensor, transpose: bool = False,
     x = x.contiguous()
     if out is None:
         out = torch.empty((cols, rows) if transpose else (rows, cols), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with N.on(x.device):
         N.check(N.lib().ssm_batch_sum(batch, rows, cols, DTYPES[x.dtype], x.data_ptr(),
-                                      int(transpose), out.data_ptr(), _stream(x.device)))
+                                      int(transpose), out.data_ptr(), N.stream(x.device)))
     return out

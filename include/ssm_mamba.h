@@ -270,6 +270,19 @@ int ssm_batch_sum(int64_t batch, int64_t rows, int64_t cols, int dtype, const vo
                   int transposed, void* out, void* stream);
 
 /*
+ * The scan's fp32 parameters from a layer's stored ones (modules/mamba.py:166):
+ * A (dim, nstate) = -exp(log_A), D32 (dim) = D and bias32 (dim) = bias, the
+ * stored ones of type dtype; D with D32 and bias with bias32 may be NULL.  The
+ * backward: dlog_A = dA * A, and dD and dbias, each rounded once to dtype (any
+ * pair NULL, a NULL dA with a NULL dlog_A).
+ */
+int ssm_scan_params_fwd(int64_t dim, int64_t nstate, int dtype, const void* log_A, const void* D,
+                        const void* bias, float* A, float* D32, float* bias32, void* stream);
+int ssm_scan_params_bwd(int64_t dim, int64_t nstate, int dtype, const float* A, const float* dA,
+                        const float* dD, const float* dbias, void* dlog_A, void* dD_out,
+                        void* dbias_out, void* stream);
+
+/*
  * Causal depthwise conv1d (+ SiLU) over channel-major rows: the prefill
  * convolution of the Mamba layer, nn.Conv1d(dim, dim, width, groups=dim,
  * padding=width-1)(x)[..., :seqlen] followed by F.silu

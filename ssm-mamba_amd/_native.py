@@ -148,6 +148,14 @@ SIGNATURES = {
     ]),
     "ssm_transpose": (_i32, [_i64, _i64, _i64, _i32, _p, _i64, _p, _p]),
     "ssm_batch_sum": (_i32, [_i64, _i64, _i64, _i32, _p, _i32, _p, _p]),
+    "ssm_scan_params_fwd": (_i32, [
+        _i64, _i64, _i32, _p, _p, _p,          # dim, nstate, dtype, log_A, D, bias
+        _p, _p, _p, _p,                        # A, D32, bias32, stream
+    ]),
+    "ssm_scan_params_bwd": (_i32, [
+        _i64, _i64, _i32, _p, _p, _p, _p,      # dim, nstate, dtype, A, dA, dD, dbias
+        _p, _p, _p, _p,                        # dlog_A, dD_out, dbias_out, stream
+    ]),
     "ssm_rms_norm_cm": (_i32, [
         _i64, _i64, _i64, _i32,                # batch, channels, seqlen, dtype
         _p, _p, ctypes.c_float, _p, _p,        # x, weight, eps, out, stream

@@ -337,9 +337,9 @@ class Mamba(nn.Module):
                               lengths=lengths if use_cache else None)
         if use_cache:
             self._conv_context = window
-        A, D, dt_bias = self._scan_params()
-        y, last = _lt.SsmFn.apply(xc, z, self.ssm_param_proj.weight, self.delta_proj.weight, A, D,
-                                  dt_bias, ssm_hiddens, lengths, "left")
+        y, last = _lt.SsmFn.apply(xc, z, self.ssm_param_proj.weight, self.delta_proj.weight,
+                                  self.log_A, self.D, self.delta_proj.bias, ssm_hiddens, lengths,
+                                  "left")
         if use_cache:
             self._ssm_hiddens = self._keep(self._ssm_hiddens, last.detach())
         return y, last

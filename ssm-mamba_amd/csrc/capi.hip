@@ -65,6 +65,9 @@ hipError_t launch_transpose(int bf16, const void* in, int64_t ibs, void* out, in
                             bool vec, hipStream_t st);
 hipError_t launch_batch_sum(int bf16, const void* in, void* out, int B, int R, int S, bool trans,
                             bool vec, hipStream_t st);
+hipError_t launch_scan_params(int bf16, bool bwd, const void* a_in, const float* A, const void* d_in,
+                              const void* b_in, void* a_out, void* d_out, void* b_out, int nA,
+                              int dim, hipStream_t st);
 int decode_rows_max_batch();
 hipError_t launch_decode_rows_linear(int bf16, const void* W, const void* x, const void* nw,
                                      float eps, const void* bias, const void* res, void* y, int B,
@@ -1073,6 +1076,39 @@ int ssm_batch_sum(int64_t batch, int64_t rows, int64_t cols, int dtype, const vo
                                           (int)cols, transposed != 0, vec,
                                           static_cast<hipStream_t>(stream)),
                     "batch_sum launch");
+}
+
+static int check_scan_params(int64_t dim, int64_t nstate, int dtype) {
+  if (dtype != SSM_F32 && dtype != SSM_BF16)
+    return fail(SSM_ERR_INVALID, "dtype must be SSM_F32 or SSM_BF16 (got %d)", dtype);
+  if (dim < 1 || nstate < 1) return fail(SSM_ERR_INVALID, "dim and nstate must be >= 1");
+  if (dim > INT_MAX / 2 / nstate) return fail(SSM_ERR_UNSUPPORTED, "scan_params sizes too large");
+  return SSM_OK;
+}
+
+int ssm_scan_params_fwd(int64_t dim, int64_t nstate, int dtype, const void* log_A, const void* D,
+                        const void* bias, float* A, float* D32, float* bias32, void* stream) {
+  g_err.clear();
+  if (int e = check_scan_params(dim, nstate, dtype)) return e;
+  if (!log_A || !A || !D != !D32 || !bias != !bias32)
+    return fail(SSM_ERR_INVALID, "log_A and A must be non-NULL, D with D32 and bias with bias32");
+  return hip_status(ssm::launch_scan_params(dtype == SSM_BF16, false, log_A, nullptr, D, bias, A, D32,
+                                            bias32, (int)(dim * nstate), (int)dim,
+                                            static_cast<hipStream_t>(stream)),
+                    "scan_params launch");
+}
+
+int ssm_scan_params_bwd(int64_t dim, int64_t nstate, int dtype, const float* A, const float* dA,
+                        const float* dD, const float* dbias, void* dlog_A, void* dD_out,
+                        void* dbias_out, void* stream) {
+  g_err.clear();
+  if (int e = check_scan_params(dim, nstate, dtype)) return e;
+  if (!A || !dA != !dlog_A || !dD != !dD_out || !dbias != !dbias_out)
+    return fail(SSM_ERR_INVALID, "A must be non-NULL, each gradient with its output");
+  return hip_status(ssm::launch_scan_params(dtype == SSM_BF16, true, dA, A, dD, dbias, dlog_A, dD_out,
+                                            dbias_out, (int)(dim * nstate), (int)dim,
+                                            static_cast<hipStream_t>(stream)),
+                    "scan_params backward launch");
 }
 
 size_t ssm_causal_conv1d_bwd_workspace_bytes(int64_t batch, int64_t dim, int64_t width) {

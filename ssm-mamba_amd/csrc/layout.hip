@@ -8,6 +8,7 @@
 //                           residual's gradient added, and the weight gradient
 //   transpose_kernel        (batch, R, S) -> (batch, S, R)
 //   batch_sum_kernel        sum over the batch, optionally transposed
+//   scan_params_kernel      the scan's fp32 parameters from the stored ones, and back
 //
 // All are memory-bound; each reads and writes every element once.  Measured at
 // (4, 2048, 1024) in bf16 (16.8 MB a tensor, 3.2 us at the copy rate): the norm
@@ -550,6 +551,33 @@ void launch_norm_bwd_c(const void* x, const void* w, const float* rstd, const vo
 #undef SSM_NORM_TC
 }
 
+// ---------------------------------------------------------------- scan parameters
+
+// A = -exp(log_A) and the fp32 copies of D and the step-size bias (kBwd: dlog_A
+// = dA * A and the gradients' casts).  A few 100 KB: what it costs is its
+// launch, so all three go in one, an element per thread.  As torch ops a
+// training step of a layer made 12 launches of 3.2 to 4.2 us for them (cast,
+// exp and negation forward, the casts again in the backward, negation, product
+// and three casts for the gradients): with two, the step at (4, 2048, 1024) bf16
+// went from 938 to 892 us.
+template <typename T, bool kBwd>
+__global__ __launch_bounds__(256) void scan_params_kernel(
+    const void* __restrict__ a_in, const float* __restrict__ A, const void* __restrict__ d_in,
+    const void* __restrict__ b_in, void* __restrict__ a_out, void* __restrict__ d_out,
+    void* __restrict__ b_out, const int nA, const int dim) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if constexpr (kBwd) {
+    if (a_out && i < nA)
+      Elem<T>::store1(static_cast<T*>(a_out) + i, static_cast<const float*>(a_in)[i] * A[i]);
+    if (d_out && i < dim) Elem<T>::store1(static_cast<T*>(d_out) + i, static_cast<const float*>(d_in)[i]);
+    if (b_out && i < dim) Elem<T>::store1(static_cast<T*>(b_out) + i, static_cast<const float*>(b_in)[i]);
+  } else {
+    if (i < nA) static_cast<float*>(a_out)[i] = -expf(Elem<T>::load1(static_cast<const T*>(a_in) + i));
+    if (d_out && i < dim) static_cast<float*>(d_out)[i] = Elem<T>::load1(static_cast<const T*>(d_in) + i);
+    if (b_out && i < dim) static_cast<float*>(b_out)[i] = Elem<T>::load1(static_cast<const T*>(b_in) + i);
+  }
+}
+
 }  // namespace
 
 // Channels the tile of 32 tokens holds in LDS: 128 KB at the largest.
@@ -636,6 +664,26 @@ hipError_t launch_batch_sum(int bf16, const void* in, void* out, int B, int R, i
     default: SSM_BS(__hip_bfloat16, true, true); break;
   }
 #undef SSM_BS
+  return hipGetLastError();
+}
+
+// nA, dim >= 1 (nA >= dim); bwd: a_in is dA, else log_A
+hipError_t launch_scan_params(int bf16, bool bwd, const void* a_in, const float* A, const void* d_in,
+                              const void* b_in, void* a_out, void* d_out, void* b_out, int nA,
+                              int dim, hipStream_t st) {
+  ProfScope prof("scan_params", st);
+  const dim3 grid((nA + 255) / 256);
+#define SSM_SP(T, b)                                                                            \
+  hipLaunchKernelGGL((scan_params_kernel<T, b>), grid, dim3(256), 0, st, a_in, A, d_in, b_in,   \
+                     a_out, d_out, b_out, nA, dim)
+  if (bf16) {
+    if (bwd) SSM_SP(__hip_bfloat16, true);
+    else SSM_SP(__hip_bfloat16, false);
+  } else {
+    if (bwd) SSM_SP(float, true);
+    else SSM_SP(float, false);
+  }
+#undef SSM_SP
   return hipGetLastError();
 }
 

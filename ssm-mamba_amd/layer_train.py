@@ -107,24 +107,26 @@ class SsmFn(torch.autograd.Function):
     read from params (``modules/mamba.py:141-182``)."""
 
     @staticmethod
-    def forward(ctx, xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, side):
-        rank, nstate = w_dt.shape[1], A.shape[1]
+    def forward(ctx, xc, z, w_x, w_dt, log_A, D, dt_bias, h_init, lengths, side):
+        rank, nstate = w_dt.shape[1], log_A.shape[1]
         params = _bmm(w_x, xc)
         delta = _bmm(w_dt, params[:, :rank])
-        f32 = lambda t: None if t is None else t.float().contiguous()
-        A32, D32, b32, h0 = f32(A), f32(D), f32(dt_bias), f32(h_init)
+        A32, D32, b32 = _lay.scan_params(log_A, D, dt_bias)
+        h0 = None if h_init is None else h_init.float().contiguous()
         y = torch.empty_like(xc)
         out, h = selective_scan.forward(
             xc, A32, params[:, rank:rank + nstate], params[:, rank + nstate:], D32, delta, b32, h0,
             lengths, side, z=z, out_ungated=y)
         ctx.set_materialize_grads(False)
-        ctx.save_for_backward(xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, params, delta, y, h)
+        ctx.save_for_backward(xc, z, w_x, w_dt, log_A, D, dt_bias, h_init, lengths, params, delta, y,
+                              h, A32, D32, b32)
         ctx.side = side
         return out, selective_scan.last_state(h)
 
     @staticmethod
-    def _op_by_op(xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, side):
-        rank, nstate = w_dt.shape[1], A.shape[1]
+    def _op_by_op(xc, z, w_x, w_dt, log_A, D, dt_bias, h_init, lengths, side):
+        rank, nstate = w_dt.shape[1], log_A.shape[1]
+        A = -torch.exp(log_A.float())
         params = _bmm(w_x, xc)
         delta = _bmm(w_dt, params[:, :rank])
         return selective_scan_fn(xc, delta, A, params[:, rank:rank + nstate],
@@ -134,20 +136,23 @@ class SsmFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, dlast):
-        xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, params, delta, y, h = ctx.saved_tensors
+        (xc, z, w_x, w_dt, log_A, D, dt_bias, h_init, lengths, params, delta, y, h, A32, D32,
+         b32) = ctx.saved_tensors
         if torch.is_grad_enabled():
             return _grads_op_by_op(ctx, SsmFn._op_by_op,
-                                   (xc, z, w_x, w_dt, A, D, dt_bias, h_init, lengths, ctx.side),
+                                   (xc, z, w_x, w_dt, log_A, D, dt_bias, h_init, lengths, ctx.side),
                                    (dout, dlast))
         need = ctx.needs_input_grad
-        rank, nstate = w_dt.shape[1], A.shape[1]
+        rank, nstate = w_dt.shape[1], log_A.shape[1]
         f32 = lambda t: None if t is None else t.float().contiguous()
         if dout is None:
             dout = torch.zeros_like(xc)
         du, dA, dB, dC, dD, ddelta, dbias, dh0, dz = selective_scan.backward(
-            xc, f32(A), params[:, rank:rank + nstate], params[:, rank + nstate:], f32(D), delta,
-            f32(dt_bias), h, f32(h_init), dout.contiguous(), f32(dlast), lengths, ctx.side, z=z,
+            xc, A32, params[:, rank:rank + nstate], params[:, rank + nstate:], D32, delta,
+            b32, h, f32(h_init), dout.contiguous(), f32(dlast), lengths, ctx.side, z=z,
             out_ungated=y)
+        dlog_A, dD, dbias = _lay.scan_params_backward(
+            A32, (log_A, D, dt_bias), [g if n else None for g, n in zip((dA, dD, dbias), need[4:7])])
         dw_dt = dw_x = None
         if need[3]:
             dw_dt = _lay.batch_sum(torch.bmm(ddelta, _lay.transposed(params[:, :rank])))
@@ -157,7 +162,8 @@ class SsmFn(torch.autograd.Function):
                 dw_x = _lay.batch_sum(torch.bmm(xc, _lay.transposed(dparams)), transpose=True)
             if need[0]:
                 du = _bmm(w_x.t(), dparams, du)
-        return (du if need[0] else None, dz, dw_x, dw_dt, dA, dD, dbias, dh0, None, None)
+        return (du if need[0] else None, dz, dw_x, dw_dt, dlog_A, dD, dbias, dh0, None,
+                None)
 
 
 class OutProjFn(torch.autograd.Function):

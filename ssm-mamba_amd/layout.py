@@ -5,7 +5,7 @@ and the channel-major layout the conv and scan kernels stream
 include/ssm_mamba.h).  No autograd here."""
 from __future__ import annotations
 
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -96,4 +96,59 @@ def batch_sum(x: torch.Tensor, transpose: bool = False,
     with N.on(x.device):
         N.check(N.lib().ssm_batch_sum(batch, rows, cols, DTYPES[x.dtype], x.data_ptr(),
                                       int(transpose), out.data_ptr(), N.stream(x.device)))
+    return out
+
+
+def _ptr(t: Optional[torch.Tensor]):
+    return None if t is None else t.data_ptr()
+
+
+def _one_type(log_A: torch.Tensor, *others: Optional[torch.Tensor]) -> bool:
+    """Whether the stored parameters (dim, nstate), (dim,), (dim,) are what the
+    scan_params kernels take."""
+    return (log_A.is_cuda and log_A.dtype in DTYPES and log_A.dim() == 2 and log_A.numel() > 0
+            and log_A.is_contiguous()
+            and all(t is None or (t.dtype == log_A.dtype and t.device == log_A.device
+                                  and t.is_contiguous() and tuple(t.shape) == log_A.shape[:1])
+                    for t in others))
+
+
+def scan_params(log_A: torch.Tensor, D: Optional[torch.Tensor],
+                bias: Optional[torch.Tensor]) -> Tuple[torch.Tensor, ...]:
+    """(A = -exp(log_A), D, bias) contiguous in float32: float32 D and bias are
+    the tensors given."""
+    if not _one_type(log_A, D, bias):
+        f32 = lambda t: None if t is None else t.float().contiguous()
+        return -torch.exp(log_A.float().contiguous()), f32(D), f32(bias)
+    dim, nstate = log_A.shape
+    cast = log_A.dtype != torch.float32
+    new = lambda t: torch.empty(t.shape, dtype=torch.float32, device=t.device)
+    A = new(log_A)
+    D32, b32 = ((None if t is None else new(t)) if cast else t for t in (D, bias))
+    with N.on(log_A.device):
+        N.check(N.lib().ssm_scan_params_fwd(
+            dim, nstate, DTYPES[log_A.dtype], log_A.data_ptr(), _ptr(D) if cast else None,
+            _ptr(bias) if cast else None, A.data_ptr(), _ptr(D32) if cast else None,
+            _ptr(b32) if cast else None, N.stream(log_A.device)))
+    return A, D32, b32
+
+
+def scan_params_backward(A: torch.Tensor, stored, grads):
+    """Gradients of the stored (log_A, D, bias) from those of ``scan_params``'s
+    results (float32, or None where none is wanted), in the stored types."""
+    dA, dD, db = grads
+    log_A, D, bias = stored
+    if not _one_type(log_A, D, bias):
+        to = lambda g, t: None if g is None else g.to(t.dtype)
+        return to(None if dA is None else dA * A, log_A), to(dD, D), to(db, bias)
+    cast = log_A.dtype != torch.float32
+    new = lambda g, t: None if g is None else torch.empty_like(t)
+    out = (new(dA, log_A), *((new(dD, D), new(db, bias)) if cast else (dD, db)))
+    if dA is not None or cast:
+        dim, nstate = log_A.shape
+        with N.on(A.device):
+            N.check(N.lib().ssm_scan_params_bwd(
+                dim, nstate, DTYPES[log_A.dtype], A.data_ptr(), _ptr(dA), _ptr(dD) if cast else None,
+                _ptr(db) if cast else None, _ptr(out[0]), _ptr(out[1]) if cast else None,
+                _ptr(out[2]) if cast else None, N.stream(A.device)))
     return out

@@ -144,3 +144,29 @@ def test_block_second_derivatives_and_frozen_parameters(cuda):
     blk(x0)[0].sum().backward()
     assert blk.ssm.input_proj.weight.grad is None and blk.norm.weight.grad is None
     assert all(p.grad is not None for n, p in blk.named_parameters() if p.requires_grad)
+
+
+# fewer and more elements than a workgroup, one state, no D, mixed stored types
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim,nstate,with_d,mixed", [(1, 1, True, False), (300, 1, True, False),
+                                                      (70, 16, False, False), (257, 64, True, True)])
+def test_scan_params(cuda, dtype, dim, nstate, with_d, mixed):
+    from ssm_mamba_amd import layout as LY
+    g = torch.Generator().manual_seed(dim)
+    log_A = torch.randn(dim, nstate, generator=g).to(dtype).to(cuda)
+    D = torch.randn(dim, generator=g).to(dtype).to(cuda) if with_d else None
+    bias = torch.randn(dim, generator=g).to(torch.float32 if mixed else dtype).to(cuda)
+    A, D32, b32 = LY.scan_params(log_A, D, bias)
+    ref = -torch.exp(log_A.double())
+    assert A.dtype == torch.float32
+    assert bool(((A.double() - ref).abs() <= 2.0 ** -22 * ref.abs()).all())
+    assert (D32 is None) == (D is None) and (D is None or torch.equal(D32, D.float()))
+    assert torch.equal(b32, bias.float())
+    grads = [torch.randn(t.shape, generator=g).to(cuda) if t is not None else None for t in (A, D32, b32)]
+    for want in ((1, 1, 1), (0, 1, 0), (1, 0, 0)):
+        use = [x if w else None for x, w in zip(grads, want)]
+        got = LY.scan_params_backward(A, (log_A, D, bias), use)
+        exp = [None if use[0] is None else use[0] * A, use[1], use[2]]
+        for o, e, t in zip(got, exp, (log_A, D, bias)):
+            assert (o is None) == (e is None)
+            assert o is None or (o.dtype == t.dtype and torch.equal(o, e.to(t.dtype)))

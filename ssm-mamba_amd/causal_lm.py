@@ -466,8 +466,11 @@ class Block(nn.Module):
         return y.transpose(1, 2).contiguous(), last
 
     def _fused(self, x: torch.Tensor) -> bool:
-        """Whether ``forward`` of token-major x runs on the fused layer kernels."""
-        return _dec.plain(self.norm, RMSNorm) and _lt.supported(self, x)
+        """Whether ``forward`` of token-major x runs on the fused layer kernels:
+        a subclass's own ``forward_cm`` keeps being called."""
+        return (type(self).forward_cm is Block.forward_cm
+                and type(self.ssm).forward_cm is Mamba.forward_cm
+                and _dec.plain(self.norm, RMSNorm) and _lt.supported(self, x))
 
     def forward_cm(self, x: torch.Tensor, lengths: Optional[torch.Tensor] = None,
                    ssm_hiddens: Optional[torch.Tensor] = None, use_cache: bool = False,

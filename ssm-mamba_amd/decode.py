@@ -151,7 +151,8 @@ def block_step_supported(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tenso
 def plain(module, cls) -> bool:
     """Whether calling ``module`` is exactly ``cls.forward``: no subclass and no
     hooks of its own, so a kernel may stand in for the call."""
-    return (type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks)
+    return (type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks
+            and not module._backward_hooks and not module._backward_pre_hooks)
 
 
 def rows_step_supported(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tensor]) -> bool:

@@ -33,6 +33,12 @@ def _bmm(w: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None) -
     return torch.bmm(w, x) if out is None else out.baddbmm_(w, x)
 
 
+def _product(w: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """w @ x of the op-by-op forms, in float32: its derivatives are batched
+    products with transposed right operands, which bfloat16 is kept out of."""
+    return torch.bmm(w.float().expand(x.shape[0], *w.shape), x.float()).type_as(x)
+
+
 def _grads_op_by_op(ctx, fn, inputs, grads):
     """Gradients of fn(*inputs) as differentiable torch ops (create_graph)."""
     with torch.enable_grad():
@@ -69,7 +75,7 @@ class NormInProjFn(torch.autograd.Function):
         h = (xf * torch.rsqrt(xf.pow(2).mean(1, keepdim=True) + eps)
              * (1.0 + norm_weight.float())[:, None]).type_as(x).contiguous()
         inner = w_in.shape[0] // 2
-        return _bmm(w_in[:inner], h), _bmm(w_in[inner:], h), x.view_as(x)
+        return _product(w_in[:inner], h), _product(w_in[inner:], h), x.view_as(x)
 
     @staticmethod
     def backward(ctx, dxs, dz, dres):
@@ -127,8 +133,8 @@ class SsmFn(torch.autograd.Function):
     def _op_by_op(xc, z, w_x, w_dt, log_A, D, dt_bias, h_init, lengths, side):
         rank, nstate = w_dt.shape[1], log_A.shape[1]
         A = -torch.exp(log_A.float())
-        params = _bmm(w_x, xc)
-        delta = _bmm(w_dt, params[:, :rank])
+        params = _product(w_x, xc)
+        delta = _product(w_dt, params[:, :rank])
         return selective_scan_fn(xc, delta, A, params[:, rank:rank + nstate],
                                  params[:, rank + nstate:], D, z=z, delta_bias=dt_bias,
                                  return_last_state=True, h_init=h_init, length=lengths,
@@ -177,7 +183,7 @@ class OutProjFn(torch.autograd.Function):
 
     @staticmethod
     def _op_by_op(y, w_out, residual):
-        out = _bmm(w_out, y).transpose(1, 2)
+        out = _product(w_out, y).transpose(1, 2)
         return (out if residual is None else residual + out,)
 
     @staticmethod

@@ -117,6 +117,23 @@ def test_block_gradients(cuda, dtype, batch, seqlen, model_dim, conv_bias):
         assert rel <= (2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -18), (k, rel)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_block_gradients_of_a_graph(cuda, dtype):
+    """With create_graph the gradients come from the op-by-op forms: the same
+    values, up to roundings of the layer's intermediate tensors."""
+    blk = _block(dtype, 64, False, seed=7)
+    g = torch.Generator().manual_seed(8)
+    x = torch.randn(2, 40, 64, generator=g).to(dtype).to(cuda).requires_grad_(True)
+    dout = torch.randn(2, 40, 64, generator=g).to(dtype).to(cuda)
+    ps = [x, *blk.parameters()]
+    for a, b in zip(torch.autograd.grad(blk(x)[0], ps, dout, create_graph=True),
+                    torch.autograd.grad(blk(x)[0], ps, dout)):
+        assert a.dtype == b.dtype
+        a = a.detach()
+        rel = float((a.double() - b.double()).norm() / b.double().norm())
+        assert rel <= (2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -18), rel
+
+
 def test_block_second_derivatives_and_frozen_parameters(cuda):
     """create_graph differentiates the op-by-op form; parameters and inputs
     that need no gradient get none."""
@@ -170,3 +187,33 @@ def test_scan_params(cuda, dtype, dim, nstate, with_d, mixed):
         for o, e, t in zip(got, exp, (log_A, D, bias)):
             assert (o is None) == (e is None)
             assert o is None or (o.dtype == t.dtype and torch.equal(o, e.to(t.dtype)))
+
+
+def test_norm_hooks_and_overridden_layers_keep_being_called(cuda):
+    """A layer whose norm has hooks, or whose class has a forward of its own,
+    does not take the fused kernels."""
+    from ssm_mamba_amd.causal_lm import Block, Mamba
+    x = torch.randn(1, 40, 64, generator=torch.Generator().manual_seed(5)).to(cuda)
+    blk = _block(torch.float32, 64, False, seed=6)
+    assert blk._fused(x)
+    seen = []
+    handle = blk.norm.register_full_backward_hook(lambda *a: seen.append("norm"))
+    blk(x.clone().requires_grad_(True))[0].sum().backward()
+    handle.remove()
+    assert seen == ["norm"] and blk._fused(x)
+
+    class OwnMixer(Mamba):
+        def forward_cm(self, *a, **k):
+            seen.append("mixer")
+            return super().forward_cm(*a, **k)
+
+    class OwnBlock(Block):
+        def forward_cm(self, *a, **k):
+            seen.append("block")
+            return super().forward_cm(*a, **k)
+
+    blk.ssm.__class__ = OwnMixer
+    blk(x)
+    blk.ssm.__class__, blk.__class__ = Mamba, OwnBlock
+    blk(x)
+    assert seen == ["norm", "mixer", "block"]

@@ -11,10 +11,16 @@
 //
 // Memory-bound: one workgroup streams one (b, c) row; each thread owns chunks
 // of 8 consecutive positions (one 16-byte load for bf16, two for fp32) plus
-// the previous chunk's last K-1 elements, which the cache serves.  The
-// backward recomputes pre over the K-1 positions past its chunk, writes dx,
-// and leaves per-row partial sums of dw / dbias that a second kernel adds
-// over the batch in a fixed order (deterministic, no atomics).
+// the K-1 elements before it, which the cache serves.  The backward recomputes
+// pre over the K-1 positions past its chunk, writes dx, and leaves per-row
+// partial sums of dw / dbias that a second kernel adds over the batch in a
+// fixed order (deterministic, no atomics).  All loads of a chunk go through
+// buffer ranges that end at the row, so none waits behind a bounds check, and
+// issue before the taps are waited for: one memory round trip a chunk.  Rows
+// that are not whole 16-byte pieces take the same chunks (ConvRow, store_chunk);
+// position by position, with K loads forward and K (K + 1) backward each, they
+// took 213 us forward and backward at (4, 2048, 2047) in bf16 and 344 at (1,
+// 2560, 8191), now 104 and 101, what a call costs its host.
 #include "ss_common.cuh"
 #include "ss_io.cuh"
 #include "ss_prof.h"
@@ -26,24 +32,6 @@ namespace {
 constexpr int kConvThreads = 256;
 constexpr int kConvChunk = 8;
 constexpr int kMaxWidth = 8;
-
-template <typename T>
-__device__ __forceinline__ void load8(const T* __restrict__ p, float* v);
-
-template <>
-__device__ __forceinline__ void load8<float>(const float* __restrict__ p, float* v) {
-  const float4 a = *reinterpret_cast<const float4*>(p);
-  const float4 b = *reinterpret_cast<const float4*>(p + 4);
-  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
-
-template <>
-__device__ __forceinline__ void load8<__hip_bfloat16>(const __hip_bfloat16* __restrict__ p, float* v) {
-  const uint4 x = *reinterpret_cast<const uint4*>(p);
-  v[0] = bf16_lo(x.x); v[1] = bf16_hi(x.x); v[2] = bf16_lo(x.y); v[3] = bf16_hi(x.y);
-  v[4] = bf16_lo(x.z); v[5] = bf16_hi(x.z); v[6] = bf16_lo(x.w); v[7] = bf16_hi(x.w);
-}
 
 template <typename T>
 __device__ __forceinline__ void store8(T* __restrict__ p, const float* v);
@@ -62,6 +50,138 @@ __device__ __forceinline__ void store8<__hip_bfloat16>(__hip_bfloat16* __restric
   x.z = pack_bf16x2(v[4], v[5]);
   x.w = pack_bf16x2(v[6], v[7]);
   *reinterpret_cast<uint4*>(p) = x;
+}
+
+// The elements a workgroup reads of a row for the positions [i0, i0 + kConvSpan):
+// from 8 before to 8 after, as one buffer range that ends with the row.  kVec:
+// rows of a multiple of 8 elements at 16-byte aligned addresses.  Otherwise any
+// element alignment (RowRange): fp32 at dword alignment, bf16 as the dwords that
+// hold the elements, shifted into place.
+constexpr int kConvSpan = kConvThreads * kConvChunk;
+
+template <typename T, bool kVec>
+struct ConvRow {
+  static constexpr bool kShift = !kVec && sizeof(T) == 2;
+  // dwords that hold N elements (an array of one where there are none)
+  template <int N> static constexpr int words() { return N ? N * (int)sizeof(T) / 4 + (kShift ? 1 : 0) : 1; }
+  __amdgpu_buffer_rsrc_t r;
+  uint32_t extra = 0;  // bytes from the (dword aligned) base to the first element: 0 or 2
+  int s, L;
+
+  __device__ __forceinline__ ConvRow(const T* row, int L_, int i0) : s(max(i0 - kConvChunk, 0)), L(L_) {
+    const uint64_t a = reinterpret_cast<uint64_t>(row + s);
+    const uint32_t bytes = (uint32_t)min(L - s, kConvSpan + 2 * kConvChunk) * (uint32_t)sizeof(T);
+    if constexpr (kShift) extra = __builtin_amdgcn_readfirstlane((uint32_t)a & 2u);
+    r = raw_rsrc(reinterpret_cast<void*>(kShift ? a & ~(uint64_t)3 : a),
+                 kShift ? (extra + bytes + 3u) & ~3u : bytes);
+  }
+  // N elements (4, 8, or none) from position t, a multiple of 4; zero outside
+  // the row, but past its end the next row's where it does not end with the range
+  template <int N> __device__ __forceinline__ void load(uint32_t* w, int t) const {
+    const int off = t >= 0 ? (t - s) * (int)sizeof(T) : (int)kOffDrop;
+    constexpr int W = words<N>();
+    if constexpr (N > 0) {
+#pragma unroll
+      for (int q = 0; q + 4 <= W; q += 4) {
+        const u32x4_v v = __builtin_amdgcn_raw_buffer_load_b128(r, off + 4 * q, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[q + i] = v[i];
+      }
+      if constexpr (W % 4 == 1) {
+        w[W - 1] = __builtin_amdgcn_raw_buffer_load_b32(r, off + 4 * (W - 1), 0, 0);
+      } else if constexpr (W % 4 == 2) {
+        const u32x2_v v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+        w[0] = v.x; w[1] = v.y;
+      } else if constexpr (W % 4 == 3) {
+        typedef unsigned int u32x3_v __attribute__((ext_vector_type(3)));
+        const u32x3_v v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
+        w[0] = v.x; w[1] = v.y; w[2] = v.z;
+      }
+    }
+  }
+  // their values; kEnd: zero at and past the row's end
+  template <int N, bool kEnd> __device__ __forceinline__ void decode(const uint32_t* w, int t, float* v) const {
+    if constexpr (N > 0) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        if constexpr (sizeof(T) == 4) {
+          v[i] = __uint_as_float(w[i]);
+        } else {
+          uint32_t p;
+          if constexpr (kShift) p = __builtin_amdgcn_alignbyte(w[i / 2 + 1], w[i / 2], extra);
+          else p = w[i / 2];
+          v[i] = i % 2 ? bf16_hi(p) : bf16_lo(p);
+        }
+        if constexpr (kEnd && !kVec) v[i] = t + i < L ? v[i] : 0.0f;
+      }
+    }
+  }
+};
+
+// Elements read on either side of a chunk.
+template <int K> constexpr int conv_halo() { return K == 1 ? 0 : K <= 5 ? 4 : 8; }
+
+// The chunk at t0 of a row into its output (positions below L).  Every thread
+// of the workgroup calls it.  kVec as above.  Otherwise 16 bytes a lane at dword
+// alignment too: in a bf16 row that starts between dwords each lane writes the
+// last element of the lane before and its own first seven; first and last lanes
+// and the row's end write element by element.
+template <typename T, bool kVec>
+__device__ __forceinline__ void store_chunk(T* __restrict__ row, int L, int i0, const float (&v)[kConvChunk]) {
+  const int t0 = i0 + threadIdx.x * kConvChunk;
+  if constexpr (kVec) {
+    if (t0 < L) store8<T>(row + t0, v);
+  } else {
+    const uint64_t a = reinterpret_cast<uint64_t>(row + i0);
+    const uint32_t extra = __builtin_amdgcn_readfirstlane((uint32_t)a & 2u);
+    const uint32_t n = (uint32_t)min(L - i0, kConvSpan);
+    const __amdgpu_buffer_rsrc_t r =
+        raw_rsrc(reinterpret_cast<void*>(a & ~(uint64_t)3), extra + n * (uint32_t)sizeof(T));
+    const int off = (int)extra + (t0 - i0) * (int)sizeof(T);
+    auto at = [&](bool ok, int o) { return ok ? o : (int)kOffDrop; };
+    if constexpr (sizeof(T) == 4) {
+      const bool whole = t0 + kConvChunk <= L;
+#pragma unroll
+      for (int q = 0; q < kConvChunk; q += 4) {
+        const u32x4_v d = {__float_as_uint(v[q]), __float_as_uint(v[q + 1]), __float_as_uint(v[q + 2]),
+                           __float_as_uint(v[q + 3])};
+        __builtin_amdgcn_raw_buffer_store_b128(d, r, at(whole, off + 4 * q), 0, 0);
+      }
+      if (!whole && t0 < L) {
+#pragma unroll
+        for (int j = 0; j < kConvChunk; ++j)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j]), r, at(t0 + j < L, off + 4 * j), 0, 0);
+      }
+    } else {
+      const int lane = threadIdx.x & 63;
+      const u32x4_v p = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                         pack_bf16x2(v[6], v[7])};
+      auto one = [&](int j, bool ok) {
+        const uint32_t w = p[j / 2];
+        __builtin_amdgcn_raw_buffer_store_b16((unsigned short)(j & 1 ? w >> 16 : w), r,
+                                              at(ok && t0 + j < L, off + 2 * j), 0, 0);
+      };
+      bool whole;
+      if (extra) {
+        const uint32_t before = __shfl_up(p[3], 1, 64);
+        const u32x4_v d = {__builtin_amdgcn_alignbyte(p[0], before, 2),
+                           __builtin_amdgcn_alignbyte(p[1], p[0], 2),
+                           __builtin_amdgcn_alignbyte(p[2], p[1], 2),
+                           __builtin_amdgcn_alignbyte(p[3], p[2], 2)};
+        whole = lane > 0 && t0 + kConvChunk - 1 <= L;
+        __builtin_amdgcn_raw_buffer_store_b128(d, r, at(whole, off - 2), 0, 0);
+        one(7, !(lane < 63 && t0 + 2 * kConvChunk - 1 <= L));
+      } else {
+        whole = t0 + kConvChunk <= L;
+        __builtin_amdgcn_raw_buffer_store_b128(p, r, at(whole, off), 0, 0);
+        one(7, !whole);
+      }
+      if (!whole && t0 < L) {
+#pragma unroll
+        for (int j = 0; j < kConvChunk - 1; ++j) one(j, true);
+      }
+    }
+  }
 }
 
 template <int K, typename T>
@@ -115,61 +235,26 @@ __global__ __launch_bounds__(kConvThreads) void causal_conv1d_fwd_kernel(
   float wk[K], bs;
   // the decode cache's row length, fetched now and used after the main loop
   const int64_t len_in = lengths ? lengths[row / (size_t)dim] : (int64_t)L;
-  if (kVec && L <= kConvThreads * kConvChunk) {
-    // one chunk per thread (L <= 2048): its row loads issue before the taps
-    // are waited for, so the workgroup pays one memory round trip
-    const int t0 = threadIdx.x * kConvChunk;
-    const int tc = min(t0, L - kConvChunk);
-    float v[2 * kConvChunk];
-    load8<T>(xr + tc, v + kConvChunk);
-    load8<T>(xr + max(tc - kConvChunk, 0), v);
-    load_taps<K>(w, bias, c, wk, bs);
-    if (tc == 0) {
-#pragma unroll
-      for (int i = 0; i < kConvChunk; ++i) v[i] = 0.0f;
-    }
-    float o[kConvChunk];
+  constexpr int H = conv_halo<K>();
+  using R = ConvRow<T, kVec>;
+  uint32_t w0[R::template words<kConvChunk>()], wp[R::template words<H>()];
+  for (int i0 = 0; i0 < L; i0 += kConvSpan) {
+    const R in(xr, L, i0);
+    const int t0 = i0 + threadIdx.x * kConvChunk;
+    in.template load<kConvChunk>(w0, t0);
+    in.template load<H>(wp, t0 - H);
+    if (i0 == 0) load_taps<K>(w, bias, c, wk, bs);
+    float v[H + kConvChunk], o[kConvChunk];
+    in.template decode<H, false>(wp, t0 - H, v);
+    in.template decode<kConvChunk, false>(w0, t0, v + H);
 #pragma unroll
     for (int i = 0; i < kConvChunk; ++i) {
       float acc = bs;
 #pragma unroll
-      for (int j = 0; j < K; ++j) acc = fmaf(wk[j], v[kConvChunk + i - (K - 1) + j], acc);
+      for (int j = 0; j < K; ++j) acc = fmaf(wk[j], v[H + i - (K - 1) + j], acc);
       o[i] = silu ? silu_f(acc) : acc;
     }
-    if (t0 < L) store8<T>(orow + t0, o);
-  } else if constexpr (kVec) {
-    load_taps<K>(w, bias, c, wk, bs);
-    for (int t0 = threadIdx.x * kConvChunk; t0 < L; t0 += kConvThreads * kConvChunk) {
-      float v[2 * kConvChunk];
-      load8<T>(xr + t0, v + kConvChunk);
-      // the previous chunk from a clamped address, zeroed at the row start
-      // (no load in a branch)
-      load8<T>(xr + max(t0 - kConvChunk, 0), v);
-      if (t0 == 0) {
-#pragma unroll
-        for (int i = 0; i < kConvChunk; ++i) v[i] = 0.0f;
-      }
-      float o[kConvChunk];
-#pragma unroll
-      for (int i = 0; i < kConvChunk; ++i) {
-        float acc = bs;
-#pragma unroll
-        for (int j = 0; j < K; ++j) acc = fmaf(wk[j], v[kConvChunk + i - (K - 1) + j], acc);
-        o[i] = silu ? silu_f(acc) : acc;
-      }
-      store8<T>(orow + t0, o);
-    }
-  } else {
-    load_taps<K>(w, bias, c, wk, bs);
-    for (int t = threadIdx.x; t < L; t += kConvThreads) {
-      float acc = bs;
-#pragma unroll
-      for (int j = 0; j < K; ++j) {
-        const int tt = t - (K - 1) + j;
-        if (tt >= 0) acc = fmaf(wk[j], Elem<T>::load1(xr + tt), acc);
-      }
-      Elem<T>::store1(orow + t, silu ? silu_f(acc) : acc);
-    }
+    store_chunk<T, kVec>(orow, L, i0, o);
   }
   // the decode cache last, off the main stream's path
   if (K > 1 && window && threadIdx.x < K - 1) {
@@ -194,84 +279,53 @@ __global__ __launch_bounds__(kConvThreads) void causal_conv1d_bwd_kernel(
   const T* __restrict__ gr = dout + row * (size_t)L;
   T* __restrict__ dxr = dx + row * (size_t)L;
   float wk[K], bs;
-  load_taps<K>(w, bias, c, wk, bs);
   float acc[K + 1];
 #pragma unroll
   for (int j = 0; j <= K; ++j) acc[j] = 0.0f;
 
   auto act_grad = [&](float pre) { return silu ? silu_grad_f(pre) : 1.0f; };
 
-  if constexpr (kVec) {
-    constexpr int E = kConvChunk;
-    for (int t0 = threadIdx.x * E; t0 < L; t0 += kConvThreads * E) {
-      // x over [t0-E, t0+2E), dout over [t0, t0+2E)
-      float xv[3 * E], dv[2 * E];
-      load8<T>(xr + t0, xv + E);
-      load8<T>(gr + t0, dv);
-      if (t0 > 0) {
-        load8<T>(xr + t0 - E, xv);
-      } else {
+  constexpr int E = kConvChunk, H = conv_halo<K>();
+  using R = ConvRow<T, kVec>;
+  uint32_t x0[R::template words<E>()], d0[R::template words<E>()];
+  uint32_t xp[R::template words<H>()], xn[R::template words<H>()], dn[R::template words<H>()];
+  for (int i0 = 0; i0 < L; i0 += kConvSpan) {
+    const R xin(xr, L, i0), din(gr, L, i0);
+    const int t0 = i0 + threadIdx.x * E;
+    // x over [t0-H, t0+E+H), dout over [t0, t0+E+H)
+    xin.template load<E>(x0, t0);
+    din.template load<E>(d0, t0);
+    xin.template load<H>(xp, t0 < L ? t0 - H : -1);  // (lanes past the row: all zero)
+    xin.template load<H>(xn, t0 + E);
+    din.template load<H>(dn, t0 + E);
+    if (i0 == 0) load_taps<K>(w, bias, c, wk, bs);
+    float xv[E + 2 * H], dv[E + H];
+    xin.template decode<H, false>(xp, t0 - H, xv);
+    xin.template decode<E, true>(x0, t0, xv + H);
+    xin.template decode<H, true>(xn, t0 + E, xv + H + E);
+    din.template decode<E, true>(d0, t0, dv);
+    din.template decode<H, true>(dn, t0 + E, dv + E);
+    // g at positions t0 + m, m < E + K - 1 (zero past the row end: dv = 0 there)
+    float g[E + K - 1];
 #pragma unroll
-        for (int i = 0; i < E; ++i) xv[i] = 0.0f;
-      }
-      if (t0 + E < L) {
-        load8<T>(xr + t0 + E, xv + 2 * E);
-        load8<T>(gr + t0 + E, dv + E);
-      } else {
+    for (int m = 0; m < E + K - 1; ++m) {
+      float pre = bs;
 #pragma unroll
-        for (int i = 0; i < E; ++i) xv[2 * E + i] = dv[E + i] = 0.0f;
-      }
-      // g at positions t0 + m, m < E + K - 1 (zero past the row end: dv = 0 there)
-      float g[E + K - 1];
-#pragma unroll
-      for (int m = 0; m < E + K - 1; ++m) {
-        float pre = bs;
-#pragma unroll
-        for (int j = 0; j < K; ++j) pre = fmaf(wk[j], xv[E + m - (K - 1) + j], pre);
-        g[m] = dv[m] * act_grad(pre);
-      }
-      float o[E];
-#pragma unroll
-      for (int i = 0; i < E; ++i) {
-        float s = 0.0f;
-#pragma unroll
-        for (int j = 0; j < K; ++j) s = fmaf(wk[j], g[i + (K - 1) - j], s);
-        o[i] = s;
-#pragma unroll
-        for (int j = 0; j < K; ++j) acc[j] = fmaf(g[i], xv[E + i - (K - 1) + j], acc[j]);
-        acc[K] += g[i];
-      }
-      store8<T>(dxr + t0, o);
+      for (int j = 0; j < K; ++j) pre = fmaf(wk[j], xv[H + m - (K - 1) + j], pre);
+      g[m] = dv[m] * act_grad(pre);
     }
-  } else {
-    for (int t = threadIdx.x; t < L; t += kConvThreads) {
-      float g[K];  // g at t + m, m < K
+    float o[E];
 #pragma unroll
-      for (int m = 0; m < K; ++m) {
-        const int tm = t + m;
-        float gm = 0.0f;
-        if (tm < L) {
-          float pre = bs;
-#pragma unroll
-          for (int j = 0; j < K; ++j) {
-            const int tt = tm - (K - 1) + j;
-            if (tt >= 0) pre = fmaf(wk[j], Elem<T>::load1(xr + tt), pre);
-          }
-          gm = Elem<T>::load1(gr + tm) * act_grad(pre);
-        }
-        g[m] = gm;
-      }
+    for (int i = 0; i < E; ++i) {
       float s = 0.0f;
 #pragma unroll
-      for (int j = 0; j < K; ++j) s = fmaf(wk[j], g[K - 1 - j], s);
-      Elem<T>::store1(dxr + t, s);
+      for (int j = 0; j < K; ++j) s = fmaf(wk[j], g[i + (K - 1) - j], s);
+      o[i] = s;
 #pragma unroll
-      for (int j = 0; j < K; ++j) {
-        const int tt = t - (K - 1) + j;
-        if (tt >= 0) acc[j] = fmaf(g[0], Elem<T>::load1(xr + tt), acc[j]);
-      }
-      acc[K] += g[0];
+      for (int j = 0; j < K; ++j) acc[j] = fmaf(g[i], xv[H + i - (K - 1) + j], acc[j]);
+      acc[K] += g[i];
     }
+    store_chunk<T, kVec>(dxr, L, i0, o);
   }
   block_sum<K>(acc, red);
   if (threadIdx.x == 0) {

@@ -238,13 +238,14 @@ int ssm_rms_norm_cm(int64_t batch, int64_t channels, int64_t seqlen, int dtype, 
  *   h_cm[b, c, t] = x[b, t, c] * rstd[b, t] * (1 + weight[c]),
  *   rstd[b, t] = rsqrt(mean_c x[b, t, c]^2 + eps)
  * with h_tm (batch, seqlen, channels; nullable) the same values token-major and
- * rstd (batch, seqlen; nullable) fp32, for the backward.  channels a multiple
- * of 16 bytes of elements, at most 2048 (bf16) or 1024 (fp32); x, weight and
- * h_tm 16-byte aligned.
+ * rstd (batch, seqlen; nullable) fp32, for the backward, and x_copy (as x;
+ * nullable) a copy of x, for a sum in place.  channels a multiple of 16 bytes
+ * of elements, at most 2048 (bf16) or 1024 (fp32); x, weight, h_tm and x_copy
+ * 16-byte aligned.
  */
 int ssm_rms_norm_tc_fwd(int64_t batch, int64_t seqlen, int64_t channels, int dtype, const void* x,
                         const void* weight, float eps, void* h_cm, void* h_tm, float* rstd,
-                        void* stream);
+                        void* x_copy, void* stream);
 
 /* Device workspace (bytes) for ssm_rms_norm_tc_bwd. */
 size_t ssm_rms_norm_tc_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t channels);

@@ -138,7 +138,7 @@ SIGNATURES = {
     ]),
     "ssm_rms_norm_tc_fwd": (_i32, [
         _i64, _i64, _i64, _i32,                # batch, seqlen, channels, dtype
-        _p, _p, ctypes.c_float, _p, _p, _p, _p,  # x, weight, eps, h_cm, h_tm, rstd, stream
+        _p, _p, ctypes.c_float, _p, _p, _p, _p, _p,  # x, weight, eps, h_cm, h_tm, rstd, x_copy, stream
     ]),
     "ssm_rms_norm_tc_bwd_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "ssm_rms_norm_tc_bwd": (_i32, [
@@ -162,7 +162,7 @@ SIGNATURES = {
     ]),
 }
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 
 def lib() -> ctypes.CDLL:

@@ -453,11 +453,13 @@ class Block(nn.Module):
             w_out = self.ssm.out_proj.weight
             if torch.is_grad_enabled():
                 xs, z, x = _lt.NormInProjFn.apply(hidden_states, self.norm.weight,
-                                                  self.ssm.input_proj.weight, self.norm.eps)
+                                                  self.ssm.input_proj.weight, self.norm.eps,
+                                                  not drop)
                 y, last = self.ssm._mix_train(xs, z, ssm_hiddens, lengths, use_cache)
                 out = _lt.OutProjFn.apply(y, w_out, None if drop else x)
             else:
-                h, _, _, x = _lay.norm_tc(hidden_states, self.norm.weight, self.norm.eps)
+                h, _, _, x = _lay.norm_tc(hidden_states, self.norm.weight, self.norm.eps,
+                                          copy=not drop)
                 y, last = self.ssm._mix_cm(h, ssm_hiddens, lengths, use_cache)
                 out = _lt.out_proj(y, w_out, None if drop else x)
             return (x + self.dropout(out) if drop else out), last

@@ -56,7 +56,7 @@ hipError_t launch_decode_layers(int bf16, const void* table, int nlayers, int B,
 int rms_norm_tc_max_channels(int bf16);
 int rms_norm_tc_part_rows(int B, int L);
 hipError_t launch_rms_norm_tc(int bf16, const void* x, const void* w, float eps, void* h_cm,
-                              void* h_tm, float* rstd, int B, int L, int C, bool vec,
+                              void* h_tm, float* rstd, void* x_copy, int B, int L, int C, bool vec,
                               hipStream_t st);
 hipError_t launch_rms_norm_tc_bwd(int bf16, const void* x, const void* w, const float* rstd,
                                   const void* dh, const void* dres, void* dx, void* dw, float* part,
@@ -277,7 +277,7 @@ extern "C" {
 
 const char* ssm_last_error(void) { return g_err.c_str(); }
 
-int ssm_abi_version(void) { return 10; }
+int ssm_abi_version(void) { return 11; }
 
 int ssm_profile_begin(void) {
   g_err.clear();
@@ -1004,13 +1004,13 @@ int check_rms_norm_tc(int64_t batch, int64_t seqlen, int64_t channels, int dtype
 
 int ssm_rms_norm_tc_fwd(int64_t batch, int64_t seqlen, int64_t channels, int dtype, const void* x,
                         const void* weight, float eps, void* h_cm, void* h_tm, float* rstd,
-                        void* stream) {
+                        void* x_copy, void* stream) {
   g_err.clear();
   if (!x || !weight || !h_cm) return fail(SSM_ERR_INVALID, "x, weight and h_cm must be non-NULL");
-  if (int rc = check_rms_norm_tc(batch, seqlen, channels, dtype, {x, weight, h_tm})) return rc;
+  if (int rc = check_rms_norm_tc(batch, seqlen, channels, dtype, {x, weight, h_tm, x_copy})) return rc;
   const bool vec = seqlen % elems16(dtype) == 0 && aligned16(h_cm);
   return hip_status(ssm::launch_rms_norm_tc(dtype == SSM_BF16, x, weight, eps, h_cm, h_tm, rstd,
-                                            (int)batch, (int)seqlen, (int)channels, vec,
+                                            x_copy, (int)batch, (int)seqlen, (int)channels, vec,
                                             static_cast<hipStream_t>(stream)),
                     "rms_norm_tc launch");
 }

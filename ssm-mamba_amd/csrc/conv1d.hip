@@ -18,9 +18,10 @@
 // buffer ranges that end at the row, so none waits behind a bounds check, and
 // issue before the taps are waited for: one memory round trip a chunk.  Rows
 // that are not whole 16-byte pieces take the same chunks (ConvRow, store_chunk);
-// position by position, with K loads forward and K (K + 1) backward each, they
-// took 213 us forward and backward at (4, 2048, 2047) in bf16 and 344 at (1,
-// 2560, 8191), now 104 and 101, what a call costs its host.
+// position by position, with K loads forward and K (K + 1) backward each, a
+// pass over (4, 2048, 2047) in bf16 with 4 taps took 61.5 us forward and 151.5
+// backward, now 18.3 and 31.0 (2048 positions: 15.8 and 27.1, 4.2 and 3.7 TB/s;
+// with the loads behind branches 18.3 and 30.4).
 #include "ss_common.cuh"
 #include "ss_io.cuh"
 #include "ss_prof.h"

@@ -56,18 +56,18 @@ def _grads_op_by_op(ctx, fn, inputs, grads):
 
 class NormInProjFn(torch.autograd.Function):
     """(xs, z, x) of token-major x: the two halves of W_in @ rmsnorm(x),
-    channel-major, and x itself for the residual, whose gradient then enters
-    the norm's backward."""
+    channel-major, and x itself (``copy``: a copy) for the residual, whose
+    gradient then enters the norm's backward."""
 
     @staticmethod
-    def forward(ctx, x, norm_weight, w_in, eps):
-        h, h_tm, rstd, xr = _lay.norm_tc(x, norm_weight, eps, token_major=True)
+    def forward(ctx, x, norm_weight, w_in, eps, copy):
+        h, h_tm, rstd, xr = _lay.norm_tc(x, norm_weight, eps, token_major=True, copy=copy)
         inner = w_in.shape[0] // 2
         xs, z = _bmm(w_in[:inner], h), _bmm(w_in[inner:], h)
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(x, norm_weight, w_in, h_tm, rstd)
         ctx.eps = eps
-        return xs, z, x.view_as(x)
+        return xs, z, xr if copy else x.view_as(x)
 
     @staticmethod
     def _op_by_op(x, norm_weight, w_in, eps):
@@ -104,7 +104,7 @@ class NormInProjFn(torch.autograd.Function):
             else:
                 xr = _lay.aligned(x)
                 dx, dnw = _lay.norm_tc_backward(xr, norm_weight, rstd, dh, dres)
-        return dx if need_x else None, dnw if need_nw else None, dw, None
+        return dx if need_x else None, dnw if need_nw else None, dw, None, None
 
 
 class SsmFn(torch.autograd.Function):
@@ -173,12 +173,14 @@ class SsmFn(torch.autograd.Function):
 
 
 class OutProjFn(torch.autograd.Function):
-    """Token-major W_out @ y (+ residual) of channel-major y."""
+    """Token-major W_out @ y of channel-major y, added to ``residual`` in place
+    when given."""
 
     @staticmethod
     def forward(ctx, y, w_out, residual):
         ctx.save_for_backward(y, w_out)
-        ctx.has_residual = residual is not None
+        if residual is not None:
+            ctx.mark_dirty(residual)
         return out_proj(y, w_out, residual)
 
     @staticmethod
@@ -200,15 +202,19 @@ class OutProjFn(torch.autograd.Function):
 
 
 def out_proj(y: torch.Tensor, w_out: torch.Tensor, residual: Optional[torch.Tensor]) -> torch.Tensor:
-    """(batch, seq_len, out) = y^T W_out^T (+ residual, added in the product) for
-    channel-major y.  The batched product takes W_out^T as a contiguous copy;
-    one batch row is a plain product and takes the views."""
+    """(batch, seq_len, out) = y^T W_out^T for channel-major y, in ``residual``
+    itself plus its values when given (out of place the product's library call
+    starts with a copy of it).  The batched product takes W_out^T as a
+    contiguous copy; one batch row is a plain product and takes the views."""
     if y.shape[0] == 1:
         a, b = y[0].t(), w_out.t()
-        return (torch.mm(a, b) if residual is None else torch.addmm(residual[0], a, b))[None]
+        if residual is None:
+            return torch.mm(a, b)[None]
+        residual[0].addmm_(a, b)
+        return residual
     wt = _lay.transposed(w_out[None]).expand(y.shape[0], w_out.shape[1], w_out.shape[0])
     return torch.bmm(y.transpose(1, 2), wt) if residual is None \
-        else torch.baddbmm(residual, y.transpose(1, 2), wt)
+        else residual.baddbmm_(y.transpose(1, 2), wt)
 
 
 def supported(block, x: torch.Tensor) -> bool:

@@ -31,21 +31,24 @@ def aligned(x: torch.Tensor) -> torch.Tensor:
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
-def norm_tc(x: torch.Tensor, weight: torch.Tensor, eps: float, token_major: bool = False):
+def norm_tc(x: torch.Tensor, weight: torch.Tensor, eps: float, token_major: bool = False,
+            copy: bool = False):
     """(h (batch, channels, seq_len), h token-major or None, 1 / rms (batch,
     seq_len) float32 or None, x as read) of RMSNorm(x) for token-major x;
-    ``token_major`` asks for the two that a backward needs."""
-    x = aligned(x)
+    ``token_major`` asks for the two that a backward needs, ``copy`` for an x
+    as read that is the caller's to write."""
+    given, x = x, aligned(x)
     batch, seqlen, ch = x.shape
     h = torch.empty(batch, ch, seqlen, dtype=x.dtype, device=x.device)
     h_tm = torch.empty_like(x) if token_major else None
     rstd = torch.empty(batch, seqlen, dtype=torch.float32, device=x.device) if token_major else None
+    x_copy = torch.empty_like(x) if copy and x is given else None
     with N.on(x.device):
         N.check(N.lib().ssm_rms_norm_tc_fwd(
             batch, seqlen, ch, DTYPES[x.dtype], x.data_ptr(), weight.data_ptr(), float(eps),
             h.data_ptr(), None if h_tm is None else h_tm.data_ptr(),
-            None if rstd is None else rstd.data_ptr(), N.stream(x.device)))
-    return h, h_tm, rstd, x
+            None if rstd is None else rstd.data_ptr(), _ptr(x_copy), N.stream(x.device)))
+    return h, h_tm, rstd, x if x_copy is None else x_copy
 
 
 def norm_tc_backward(x: torch.Tensor, weight: torch.Tensor, rstd: torch.Tensor, dh: torch.Tensor,

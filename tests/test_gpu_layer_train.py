@@ -217,3 +217,27 @@ def test_norm_hooks_and_overridden_layers_keep_being_called(cuda):
     blk.ssm.__class__, blk.__class__ = Mamba, OwnBlock
     blk(x)
     assert seen == ["norm", "mixer", "block"]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batch,seqlen,ch", [(1, 33, 64), (2, 37, 1000)])
+def test_residual_copy(cuda, dtype, batch, seqlen, ch):
+    """The norm's copy of x, which the layer's output is summed into: x's bits
+    in memory of its own, so a layer's input keeps its values."""
+    from ssm_mamba_amd import layout as LY
+    x = torch.randn(batch, seqlen, ch, generator=torch.Generator().manual_seed(ch)).to(dtype).to(cuda)
+    w = torch.zeros(ch, dtype=dtype, device=cuda)
+    h, _, _, xc = LY.norm_tc(x, w, 1e-6, copy=True)
+    assert torch.equal(xc, x) and xc.data_ptr() != x.data_ptr()
+    assert torch.equal(h, LY.norm_tc(x, w, 1e-6)[0])
+    strided = x.transpose(0, 1).contiguous().transpose(0, 1)  # read through a copy already
+    xc = LY.norm_tc(strided, w, 1e-6, copy=True)[3]
+    assert torch.equal(xc, x) and xc.data_ptr() != strided.data_ptr()
+    if ch != 64:
+        return
+    blk, keep = _block(dtype, ch, False, seed=9), x.clone()
+    with torch.no_grad():
+        out = blk(x)[0]
+    again = blk(x)[0]
+    assert torch.equal(x, keep) and torch.equal(blk(x.requires_grad_(True))[0], again)
+    assert float((out - again.detach()).norm() / out.norm()) <= 2.0 ** -7

@@ -8,7 +8,10 @@ over memory: the norm's chain of float32 elementwise kernels, the transpositions
 around the layer, the additions of gradients that meet (the residual's into the
 norm's backward, the scan's du into the x-projection's product), the zero-filled
 gradients of slices.  The weight gradients are batched products per batch row of
-contiguous operands, summed over the batch in float32 and rounded once.
+contiguous operands, summed over the batch in float32 and rounded once.  With
+one batch row there is nothing to sum, and plain products take the transposed
+views: nine of a step's launches less (1 x 186 x 136, bf16: 842 us a step before,
+822 now; 1 x 4096 x 1024: 844 and 819).
 
 ``supported`` says which layers and inputs take this path; every other one runs
 op by op (``Block.forward_cm``).  When a backward is itself being differentiated
@@ -31,6 +34,14 @@ def _bmm(w: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None) -
     contiguous (batch, k, n) x; added to ``out`` in place when given."""
     w = w.expand(x.shape[0], *w.shape)
     return torch.bmm(w, x) if out is None else out.baddbmm_(w, x)
+
+
+def _wgrad(g: torch.Tensor, x_tm: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Sum over the batch of g @ x_tm, for contiguous (batch, m, n) and (batch,
+    n, k); one batch row is the product itself, with no sum to launch."""
+    if g.shape[0] == 1:
+        return torch.mm(g[0], x_tm[0]) if out is None else torch.mm(g[0], x_tm[0], out=out)
+    return _lay.batch_sum(torch.bmm(g, x_tm), out=out)
 
 
 def _product(w: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
@@ -93,7 +104,7 @@ class NormInProjFn(torch.autograd.Function):
             if len(halves) < 2:
                 dw.zero_()
             for s, g in halves:
-                _lay.batch_sum(torch.bmm(g, h_tm), out=dw[s])
+                _wgrad(g, h_tm, out=dw[s])
         dx = dnw = None
         if need_x or need_nw:
             dh = None
@@ -160,12 +171,16 @@ class SsmFn(torch.autograd.Function):
         dlog_A, dD, dbias = _lay.scan_params_backward(
             A32, (log_A, D, dt_bias), [g if n else None for g, n in zip((dA, dD, dbias), need[4:7])])
         dw_dt = dw_x = None
+        one = xc.shape[0] == 1
         if need[3]:
-            dw_dt = _lay.batch_sum(torch.bmm(ddelta, _lay.transposed(params[:, :rank])))
+            # (one batch row: a plain product, which takes the transposed views)
+            dw_dt = torch.mm(ddelta[0], params[0, :rank].t()) if one \
+                else _wgrad(ddelta, _lay.transposed(params[:, :rank]))
         if need[0] or need[2]:
             dparams = torch.cat([_bmm(w_dt.t(), ddelta), dB, dC], dim=1)
             if need[2]:
-                dw_x = _lay.batch_sum(torch.bmm(xc, _lay.transposed(dparams)), transpose=True)
+                dw_x = torch.mm(dparams[0], xc[0].t()) if one \
+                    else _lay.batch_sum(torch.bmm(xc, _lay.transposed(dparams)), transpose=True)
             if need[0]:
                 du = _bmm(w_x.t(), dparams, du)
         return (du if need[0] else None, dz, dw_x, dw_dt, dlog_A, dD, dbias, dh0, None,
@@ -196,6 +211,10 @@ class OutProjFn(torch.autograd.Function):
             dy, dw, _ = _grads_op_by_op(ctx, OutProjFn._op_by_op, (y, w_out, None), (dout,))
             return dy, dw, dout if need[2] else None
         dout = dout.contiguous()
+        if y.shape[0] == 1:  # plain products, which take the transposed views
+            dt = dout[0].t()
+            dy = torch.mm(w_out.t(), dt)[None] if need[0] else None
+            return dy, torch.mm(dt, y[0].t()) if need[1] else None, dout if need[2] else None
         dy = _bmm(w_out.t(), _lay.transposed(dout)) if need[0] else None
         dw = _lay.batch_sum(torch.bmm(y, dout), transpose=True) if need[1] else None
         return dy, dw, dout if need[2] else None

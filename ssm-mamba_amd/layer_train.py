@@ -51,15 +51,19 @@ def _product(w: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
 
 
 def _grads_op_by_op(ctx, fn, inputs, grads):
-    """Gradients of fn(*inputs) as differentiable torch ops (create_graph)."""
+    """Gradients of fn(*inputs) as differentiable torch ops (create_graph).  The
+    function's every output takes a gradient when any of its inputs needs one;
+    the op-by-op form's only where an input it comes from does."""
+    res = [None] * len(ctx.needs_input_grad)
     with torch.enable_grad():
         outs = fn(*inputs)
-        pairs = [(o, g) for o, g in zip(outs, grads) if g is not None]
+        pairs = [(o, g) for o, g in zip(outs, grads) if g is not None and o.requires_grad]
         want = [i for i, t in enumerate(inputs)
                 if isinstance(t, torch.Tensor) and t.requires_grad and ctx.needs_input_grad[i]]
+        if not pairs or not want:
+            return tuple(res)
         got = torch.autograd.grad([o for o, _ in pairs], [inputs[i] for i in want],
                                   [g for _, g in pairs], create_graph=True, allow_unused=True)
-    res = [None] * len(ctx.needs_input_grad)
     for i, g in zip(want, got):
         res[i] = g
     return tuple(res)

@@ -241,3 +241,22 @@ def test_residual_copy(cuda, dtype, batch, seqlen, ch):
     again = blk(x)[0]
     assert torch.equal(x, keep) and torch.equal(blk(x.requires_grad_(True))[0], again)
     assert float((out - again.detach()).norm() / out.norm()) <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("frozen", [("norm", "ssm"), ("norm.weight", "ssm.input_proj.weight"),
+                                    ("ssm.input_proj.weight", "ssm.log_A", "ssm.out_proj.weight"), ()])
+def test_block_gradients_of_a_graph_on_data(cuda, frozen):
+    """create_graph for a layer whose input needs no gradient (the first layer,
+    a frozen embedding) and for subsets of frozen parameters."""
+    blk = _block(torch.float32, 64, False, seed=11)
+    for n, p in blk.named_parameters():
+        p.requires_grad_(not n.startswith(frozen) if frozen else True)
+    ps = [p for p in blk.parameters() if p.requires_grad]
+    g = torch.Generator().manual_seed(12)
+    x = torch.randn(2, 40, 64, generator=g).to(cuda)
+    dout, dlast = (torch.randn(s, generator=g).to(cuda) for s in ((2, 40, 64), (2, 128, 16)))
+    if not ps:
+        x.requires_grad_(True)
+        ps = [x]
+    for a, b in zip(*(torch.autograd.grad(blk(x), ps, [dout, dlast], create_graph=c) for c in (True, False))):
+        assert float((a.detach() - b).norm() / b.norm()) <= 2.0 ** -18

@@ -1,0 +1,45 @@
+"""Host logic of the fused training layer, on the CPU: the op-by-op gradients
+that create_graph takes, and which layers the fused kernels may stand in for."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from ssm_mamba_amd import layer_train as LT
+
+
+def _op_by_op(fn, inputs, grads, needs=None):
+    needs = needs or [isinstance(t, torch.Tensor) and t.requires_grad for t in inputs]
+    return LT._grads_op_by_op(SimpleNamespace(needs_input_grad=needs), fn, inputs, grads)
+
+
+@pytest.mark.parametrize("wants", [(True, True, True), (False, True, True), (False, False, True),
+                                   (True, False, False), (False, True, False), (False, False, False)])
+def test_norm_gradients_of_a_graph_with_parts_frozen(wants):
+    """All three outputs of NormInProjFn carry a gradient, whichever of its
+    inputs need one: the residual output of an input that needs none takes no
+    part.  Values and second derivatives against autograd in float64 (the form's
+    products are float32: 1e-5)."""
+    g = torch.Generator().manual_seed(1)
+    r = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64)
+    x, nw, w = (t.requires_grad_(k) for t, k in zip((r(2, 5, 8), r(8), r(12, 8)), wants))
+    dxs, dz, dres = r(2, 6, 5), r(2, 6, 5), r(2, 5, 8)
+    got = _op_by_op(LT.NormInProjFn._op_by_op, (x, nw, w, 1e-6), (dxs, dz, dres))
+    assert [t is not None for t in got[:3]] == list(wants)
+
+    def ref():
+        h = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * (1.0 + nw)
+        p = h @ w.t()
+        return (p * torch.cat([dxs, dz], 1).transpose(1, 2)).sum() + (x * dres).sum()
+
+    live = [t for t, k in zip((x, nw, w), wants) if k]
+    if not live:
+        return
+    want = torch.autograd.grad(ref(), live, create_graph=True)
+    got = [t for t in got if t is not None]
+    close = lambda a, b: bool((a.detach().double() - b.detach()).norm() <= 1e-5 * b.detach().norm())
+    assert all(close(a, b) for a, b in zip(got, want))
+    total = lambda gs: sum(t.double().pow(2).sum() for t in gs)
+    if wants[0] or sum(wants) > 1:  # otherwise linear in what is left
+        second = torch.autograd.grad(total(got), live)
+        assert all(close(a, b) for a, b in zip(second, torch.autograd.grad(total(want), live)))

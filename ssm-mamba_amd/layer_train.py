@@ -27,6 +27,7 @@ import torch
 from . import layout as _lay
 from . import selective_scan
 from .ops import selective_scan_fn
+from .utils.tensor_utils import ensure_contiguous
 
 
 def _bmm(w: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -134,6 +135,7 @@ class SsmFn(torch.autograd.Function):
         delta = _bmm(w_dt, params[:, :rank])
         A32, D32, b32 = _lay.scan_params(log_A, D, dt_bias)
         h0 = None if h_init is None else h_init.float().contiguous()
+        lengths = ensure_contiguous(lengths)
         y = torch.empty_like(xc)
         out, h = selective_scan.forward(
             xc, A32, params[:, rank:rank + nstate], params[:, rank + nstate:], D32, delta, b32, h0,

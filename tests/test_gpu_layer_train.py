@@ -260,3 +260,16 @@ def test_block_gradients_of_a_graph_on_data(cuda, frozen):
         ps = [x]
     for a, b in zip(*(torch.autograd.grad(blk(x), ps, [dout, dlast], create_graph=c) for c in (True, False))):
         assert float((a.detach() - b).norm() / b.norm()) <= 2.0 ** -18
+
+
+@pytest.mark.parametrize("strided", [lambda v: torch.stack([v, v], 1)[:, 0], lambda v: v[:1].expand(2)])
+def test_block_with_strided_lengths(cuda, strided):
+    """Lengths as a column of a tensor, or one expanded over the batch."""
+    blk = _block(torch.float32, 64, False, seed=13)
+    x = torch.randn(2, 40, 64, generator=torch.Generator().manual_seed(14)).to(cuda)
+    lengths = strided(torch.tensor([31, 40], device=cuda))
+    got, want = (blk(x, lengths=v, use_cache=True) for v in (lengths, lengths.contiguous()))
+    assert not lengths.is_contiguous() and all(torch.equal(a, b) for a, b in zip(got, want))
+    ps = list(blk.parameters())
+    for a, b in zip(*(torch.autograd.grad(list(o), ps, [torch.ones_like(t) for t in o]) for o in (got, want))):
+        assert torch.equal(a, b)

@@ -43,3 +43,29 @@ def test_norm_gradients_of_a_graph_with_parts_frozen(wants):
     if wants[0] or sum(wants) > 1:  # otherwise linear in what is left
         second = torch.autograd.grad(total(got), live)
         assert all(close(a, b) for a, b in zip(second, torch.autograd.grad(total(want), live)))
+
+
+@pytest.mark.parametrize("strided", [lambda v: torch.stack([v, v], 1)[:, 0], lambda v: v[:1].expand(2)])
+def test_lengths_reach_the_scan_contiguous(monkeypatch, strided):
+    """The scan's kernels take a dense lengths vector; a layer takes a column of
+    a tensor or one length expanded over the batch, forward and backward."""
+    seen = []
+
+    def forward(u, A, B, C, D, delta, bias, h0, length, side, **kw):
+        seen.append(length)
+        return torch.zeros_like(u), torch.zeros(2, 1, A.shape[1], A.shape[0])
+
+    def backward(u, A, B, C, D, delta, bias, h, h0, dout, dlast, length, side, **kw):
+        seen.append(length)
+        return [torch.zeros_like(t) for t in (u, A, B, C, D, delta, bias)] + [None, torch.zeros_like(u)]
+
+    monkeypatch.setattr(LT.selective_scan, "forward", forward)
+    monkeypatch.setattr(LT.selective_scan, "backward", backward)
+    monkeypatch.setattr(LT._lay, "batch_sum", lambda x, transpose=False: x.sum(0).t() if transpose else x.sum(0))
+    r = lambda *s: torch.randn(*s).requires_grad_(True)
+    lengths = strided(torch.tensor([3, 5]))
+    out, _ = LT.SsmFn.apply(r(2, 8, 5), r(2, 8, 5), r(6, 8), r(8, 2), r(8, 2), r(8), r(8), None,
+                            lengths, "left")
+    out.sum().backward()
+    assert len(seen) == 2
+    assert all(t.is_contiguous() and torch.equal(t, lengths) for t in seen)

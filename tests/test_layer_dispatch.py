@@ -61,7 +61,8 @@ def test_lengths_reach_the_scan_contiguous(monkeypatch, strided):
 
     monkeypatch.setattr(LT.selective_scan, "forward", forward)
     monkeypatch.setattr(LT.selective_scan, "backward", backward)
-    monkeypatch.setattr(LT._lay, "batch_sum", lambda x, transpose=False: x.sum(0).t() if transpose else x.sum(0))
+    monkeypatch.setattr(LT._lay, "batch_sum",
+                        lambda x, transpose=False, out=None: x.sum(0).t() if transpose else x.sum(0))
     r = lambda *s: torch.randn(*s).requires_grad_(True)
     lengths = strided(torch.tensor([3, 5]))
     out, _ = LT.SsmFn.apply(r(2, 8, 5), r(2, 8, 5), r(6, 8), r(8, 2), r(8, 2), r(8), r(8), None,

@@ -469,9 +469,9 @@ class Block(nn.Module):
 
     def _fused(self, x: torch.Tensor) -> bool:
         """Whether ``forward`` of token-major x runs on the fused layer kernels:
-        a subclass's own ``forward_cm`` keeps being called."""
-        return (type(self).forward_cm is Block.forward_cm
-                and type(self.ssm).forward_cm is Mamba.forward_cm
+        a ``forward_cm`` of a subclass, of the object itself or behind a wrapper
+        around the mixer keeps being called."""
+        return (_dec.own(self, Block, "forward_cm") and _dec.own(self.ssm, Mamba, "forward_cm")
                 and _dec.plain(self.norm, RMSNorm) and _lt.supported(self, x))
 
     def forward_cm(self, x: torch.Tensor, lengths: Optional[torch.Tensor] = None,

@@ -148,6 +148,13 @@ def block_step_supported(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tenso
     return _step_supported(gemv_supported, ssm, x, norm_weight)
 
 
+def own(obj, cls, name: str) -> bool:
+    """Whether ``obj.name`` is the method ``cls`` defines: not a subclass's, not
+    one set on the object, and not one a wrapper passes on (which has no such
+    attribute in its class)."""
+    return getattr(type(obj), name, None) is getattr(cls, name) and name not in vars(obj)
+
+
 def plain(module, cls) -> bool:
     """Whether calling ``module`` is exactly ``cls.forward``: no subclass and no
     hooks of its own, so a kernel may stand in for the call."""

@@ -253,7 +253,7 @@ def supported(block, x: torch.Tensor) -> bool:
     # (parametrized, computed by a hook) is not there and takes the other path
     mods, dtype, dev = block.ssm._modules, x.dtype, x.device
     for name in _PROJECTIONS:
-        params = mods[name]._parameters
+        params = getattr(mods.get(name), "_parameters", {})
         p = params.get("weight")
         if p is None or p.dtype != dtype or p.device != dev:
             return False

@@ -273,3 +273,18 @@ def test_block_with_strided_lengths(cuda, strided):
     ps = list(blk.parameters())
     for a, b in zip(*(torch.autograd.grad(list(o), ps, [torch.ones_like(t) for t in o]) for o in (got, want))):
         assert torch.equal(a, b)
+
+
+def test_wrapped_mixer_is_called(cuda):
+    """A mixer behind a wrapper that passes its attributes on runs op by op,
+    with and without autograd and in the decode step."""
+    from tests.test_layer_dispatch import _Delegate
+    blk = _block(torch.float32, 64, False, seed=15)
+    x = torch.randn(12, 40, 64, generator=torch.Generator().manual_seed(16)).to(cuda)
+    want = blk(x)[0].detach()
+    blk.ssm = _Delegate(blk.ssm)
+    assert float((blk(x)[0].detach() - want).norm() / want.norm()) <= 2.0 ** -18
+    with torch.no_grad():
+        got = blk(x, use_cache=True)[0]
+        step = blk.step(x[:, -1].contiguous())
+    assert float((got - want).norm() / want.norm()) <= 2.0 ** -18 and step.shape == (12, 64)

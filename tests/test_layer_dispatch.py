@@ -70,3 +70,48 @@ def test_lengths_reach_the_scan_contiguous(monkeypatch, strided):
     out.sum().backward()
     assert len(seen) == 2
     assert all(t.is_contiguous() and torch.equal(t, lengths) for t in seen)
+
+
+class _Delegate(torch.nn.Module):
+    """A wrapper that passes every attribute on, as torch.compile's does."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def __getattr__(self, name):
+        try:
+            return super().__getattr__(name)
+        except AttributeError:
+            return getattr(super().__getattr__("inner"), name)
+
+
+def _block(monkeypatch, **kw):
+    """A layer that takes the fused kernels, as far as its tensors go."""
+    from ssm_mamba_amd.causal_lm import Block
+    monkeypatch.setattr(LT._lay, "norm_tc_supported", lambda x, w: True)
+    return Block(model_dim=16, dropout_rate=0.0, **kw), torch.zeros(1, 4, 16)
+
+
+@pytest.mark.parametrize("wrap", [_Delegate, torch.compile])
+def test_wrapped_mixer(monkeypatch, wrap):
+    blk, x = _block(monkeypatch)
+    assert blk._fused(x)
+    blk.ssm = wrap(blk.ssm)
+    assert not blk._fused(x)
+
+
+def test_methods_set_on_the_object(monkeypatch):
+    for who in ("block", "mixer"):
+        blk, x = _block(monkeypatch)
+        obj = blk if who == "block" else blk.ssm
+        obj.forward_cm = lambda *a, **k: None
+        assert not blk._fused(x)
+
+
+def test_missing_projection(monkeypatch):
+    blk, x = _block(monkeypatch)
+    blk.ssm.conv = None
+    assert not blk._fused(x)
+    del blk.ssm.conv
+    assert not blk._fused(x)

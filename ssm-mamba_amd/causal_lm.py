@@ -574,8 +574,11 @@ class CausalLM(nn.Module):
                 use_cache: bool = False) -> torch.Tensor:
         """input_ids (batch, seq_len) -> logits (batch, seq_len, vocab)."""
         x = self.embedding(input_ids)
-        if torch.is_grad_enabled() and all(layer._fused(x) for layer in self.layers):
-            # training: each layer token-major in and out
+        if torch.is_grad_enabled() and all(_dec.own(layer, Block, "forward") and layer._fused(x)
+                                           for layer in self.layers):
+            # training: each layer token-major in and out (a model asks its
+            # layers for forward_cm alone: one with a forward of its own, or
+            # with forward_cm only, keeps being asked for that)
             for layer in self.layers:
                 x, _ = layer.forward(x, lengths=lengths, use_cache=use_cache)
             return self.lm_head(self.norm(x))

@@ -115,3 +115,41 @@ def test_missing_projection(monkeypatch):
     assert not blk._fused(x)
     del blk.ssm.conv
     assert not blk._fused(x)
+
+
+class _ChannelMajorOnly(torch.nn.Module):
+    def forward_cm(self, x, **kw):
+        return x + 1.0, None
+
+
+def test_model_asks_its_layers_for_forward_cm(monkeypatch):
+    """A layer in CausalLM.layers needs forward_cm and no more, and a forward of
+    a subclass or of the object is not what a model calls."""
+    from ssm_mamba_amd.causal_lm import Block, CausalLM, CausalLMConfig
+    monkeypatch.setattr(LT._lay, "norm_tc_supported", lambda x, w: True)
+    called = []
+
+    def forward_cm(self, x, **kw):
+        called.append("forward_cm")
+        return x, None
+
+    def forward(self, *a, **kw):
+        called.append("forward")
+
+    class OwnForward(Block):
+        pass
+
+    OwnForward.forward = forward
+    m = CausalLM(CausalLMConfig(vocab_size=11, model_dim=16, num_layers=2, dropout_rate=0.0))
+    ids = torch.randint(3, 11, (2, 5))
+    monkeypatch.setattr(Block, "forward", lambda self, x, **kw: (x, None))
+    assert m(ids).shape == (2, 5, 11)        # (plain layers: Block.forward)
+    monkeypatch.setattr(Block, "forward_cm", forward_cm)
+    m.layers[1].__class__ = OwnForward
+    m(ids)
+    m.layers[1].__class__ = Block
+    m.layers[1].forward = forward.__get__(m.layers[1])
+    m(ids)
+    assert called == ["forward_cm"] * 4
+    m.layers = torch.nn.ModuleList([_ChannelMajorOnly()])
+    assert m(ids).shape == (2, 5, 11)

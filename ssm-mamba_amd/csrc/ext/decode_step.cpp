@@ -40,7 +40,7 @@ namespace py = pybind11;
   X(_parameters) X(_buffers) X(_modules) X(_forward_hooks) X(_forward_pre_hooks) X(norm) X(ssm) \
   X(weight) X(bias) X(eps) X(input_proj) X(conv) X(ssm_param_proj) X(delta_proj) X(out_proj)     \
   X(log_A) X(D) X(_conv_context) X(_ssm_hiddens) X(inner_dim) X(state_dim) X(delta_rank)         \
-  X(conv_kernel)
+  X(conv_kernel) X(forward)
 
 struct Names {
 #define SSM_DECL(n) PyObject* n = PyUnicode_InternFromString(#n);
@@ -89,7 +89,9 @@ struct Module {
     }
     return true;
   }
-  bool no_hooks() const {
+  // a call is the class's forward: none set on the object, no hooks of its own
+  bool plain_call() const {
+    if (PyDict_GetItem(dicts[0], names().forward)) return false;
     for (PyObject* n : {names()._forward_hooks, names()._forward_pre_hooks}) {
       PyObject* h = PyDict_GetItem(dicts[0], n);
       if (!h || PyObject_Size(h) != 0) return false;
@@ -143,7 +145,7 @@ struct Step {  // the token batch
 struct Layer {
   int64_t dim, nstate, rank, width, nout;
   double eps;
-  bool norm_plain;                // no hooks on the norm
+  bool norm_plain;                // calling the norm is its class's forward
   void* row[SSM_LAYER_NPTR];
 
   bool put(const Step& s, int slot, PyObject* o, std::initializer_list<int64_t> shape, bool optional) {
@@ -184,7 +186,7 @@ struct Layer {
     PyObject* ep = norm.get(n.eps);
     if (!ep || !PyFloat_CheckExact(ep)) return false;
     eps = PyFloat_AS_DOUBLE(ep);
-    norm_plain = norm.no_hooks();
+    norm_plain = norm.plain_call();
     if (!ssm.integer(n.inner_dim, dim) || !ssm.integer(n.state_dim, nstate) ||
         !ssm.integer(n.delta_rank, rank) || !ssm.integer(n.conv_kernel, width))
       return false;

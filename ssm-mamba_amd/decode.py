@@ -16,6 +16,7 @@ from array import array
 from typing import Optional
 
 import torch
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _ext as _E
 from . import _native as N
@@ -156,9 +157,11 @@ def own(obj, cls, name: str) -> bool:
 
 
 def plain(module, cls) -> bool:
-    """Whether calling ``module`` is exactly ``cls.forward``: no subclass and no
-    hooks of its own, so a kernel may stand in for the call."""
-    return (type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks
+    """Whether calling ``module`` is exactly ``cls.forward``: no subclass, no
+    forward set on the object, no hooks of its own and none on all modules, so
+    a kernel may stand in for the call."""
+    return (type(module) is cls and "forward" not in vars(module) and not _has_any_global_hook()
+            and not module._forward_hooks and not module._forward_pre_hooks
             and not module._backward_hooks and not module._backward_pre_hooks)
 
 
@@ -210,8 +213,8 @@ def plain_block_step(block, x: torch.Tensor, classes) -> Optional[torch.Tensor]:
     None leaves the call to the checks above."""
     if not ENABLED or not x.is_cuda:
         return None
-    return _E.module("decode_step").block_step(block, x, classes, FOLD_XPROJ,
-                                               not torch.is_autocast_enabled())
+    rows = not (torch.is_autocast_enabled() or _has_any_global_hook())
+    return _E.module("decode_step").block_step(block, x, classes, FOLD_XPROJ, rows)
 
 
 def plain_layer_rows(layers, x: torch.Tensor, classes) -> Optional[bytes]:

@@ -146,3 +146,37 @@ def test_hooked_norm_and_autocast(cuda):
         m.layers[0].norm.register_forward_hook(lambda *a: None)
         assert _native(m, x) is None
         assert _native(m, x[:2]) is None  # the caches hold 16 rows
+
+
+def test_norm_with_a_forward_of_its_own(cuda):
+    """Past 8 rows a forward set on the norm, or a hook on all modules, keeps
+    being called by the layer's step and by the model's head."""
+    seen = []
+
+    def check(m, x, calls):
+        with torch.no_grad():
+            _caches(m, 16, torch.float32)
+            want = [m.layers[0].step(x), m._head(x)]
+            undo = calls()
+            seen.clear()
+            assert _native(m, x) is None
+            _caches(m, 16, torch.float32)
+            got = [m.layers[0].step(x), m._head(x)]
+            undo()
+        assert len(seen) >= 2
+        assert all(float((a - b).norm() / b.norm()) <= 2.0 ** -18 for a, b in zip(got, want))
+
+    m = _model(cuda, torch.float32, 16)
+    x = torch.randn(16, 64, device=cuda)
+
+    def on_the_object():
+        norms = (m.layers[0].norm, m.norm)
+        for n in norms:
+            n.forward = lambda v, f=n.forward, **kw: (seen.append(n), f(v, **kw))[1]
+        return lambda: [delattr(n, "forward") for n in norms]
+
+    def on_all_modules():
+        return nn.modules.module.register_module_forward_hook(lambda mod, *a: seen.append(mod)).remove
+
+    check(m, x, on_the_object)
+    check(m, x, on_all_modules)

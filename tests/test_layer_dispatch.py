@@ -153,3 +153,33 @@ def test_model_asks_its_layers_for_forward_cm(monkeypatch):
     assert called == ["forward_cm"] * 4
     m.layers = torch.nn.ModuleList([_ChannelMajorOnly()])
     assert m(ids).shape == (2, 5, 11)
+
+
+def _global(register):
+    return lambda m: getattr(torch.nn.modules.module, register)(lambda *a: None)
+
+
+@pytest.mark.parametrize("change", [
+    _global("register_module_forward_hook"), _global("register_module_forward_pre_hook"),
+    _global("register_module_full_backward_hook"),
+    lambda m: m.register_forward_hook(lambda *a: None),
+    lambda m: m.register_forward_pre_hook(lambda *a: None),
+    lambda m: m.register_full_backward_hook(lambda *a: None),
+    lambda m: setattr(m, "forward", type(m).forward.__get__(m)),
+    lambda m: setattr(m, "__class__", type("Own", (type(m),), {})),
+])
+def test_plain_module_calls(change):
+    """A kernel may stand in for a module's call only where the call is its
+    class's forward and nothing else."""
+    from ssm_mamba_amd import decode as DEC
+    from ssm_mamba_amd.causal_lm import RMSNorm
+    for m in (RMSNorm(8), torch.nn.Linear(8, 8)):
+        cls = type(m)
+        assert DEC.plain(m, cls)
+        handle = change(m)
+        try:
+            assert not DEC.plain(m, cls)
+        finally:
+            if handle is not None:
+                handle.remove()
+    assert DEC.plain(RMSNorm(8), RMSNorm)

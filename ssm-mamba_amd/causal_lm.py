@@ -497,7 +497,7 @@ class Block(nn.Module):
             # norm, mixer and residual in the four fused decode kernels
             return _dec.block_step(self.ssm, hidden_states, self.norm.weight, self.norm.eps,
                                    residual=True)
-        if (_dec.plain(self.norm, RMSNorm)
+        if (_dec.plain(self.norm, RMSNorm) and _dec.own(self.ssm, Mamba, "step")
                 and _dec.rows_step_supported(self.ssm, hidden_states, self.norm.weight)):
             # the same for 9 to 64 rows, on the matrix cores
             return _dec.rows_block_step(self.ssm, hidden_states, self.norm.weight, self.norm.eps,

@@ -40,7 +40,7 @@ namespace py = pybind11;
   X(_parameters) X(_buffers) X(_modules) X(_forward_hooks) X(_forward_pre_hooks) X(norm) X(ssm) \
   X(weight) X(bias) X(eps) X(input_proj) X(conv) X(ssm_param_proj) X(delta_proj) X(out_proj)     \
   X(log_A) X(D) X(_conv_context) X(_ssm_hiddens) X(inner_dim) X(state_dim) X(delta_rank)         \
-  X(conv_kernel) X(forward)
+  X(conv_kernel) X(forward) X(step)
 
 struct Names {
 #define SSM_DECL(n) PyObject* n = PyUnicode_InternFromString(#n);
@@ -145,7 +145,7 @@ struct Step {  // the token batch
 struct Layer {
   int64_t dim, nstate, rank, width, nout;
   double eps;
-  bool norm_plain;                // calling the norm is its class's forward
+  bool calls_plain;               // norm() and ssm.step() are their classes' own
   void* row[SSM_LAYER_NPTR];
 
   bool put(const Step& s, int slot, PyObject* o, std::initializer_list<int64_t> shape, bool optional) {
@@ -186,7 +186,7 @@ struct Layer {
     PyObject* ep = norm.get(n.eps);
     if (!ep || !PyFloat_CheckExact(ep)) return false;
     eps = PyFloat_AS_DOUBLE(ep);
-    norm_plain = norm.plain_call();
+    calls_plain = norm.plain_call() && !PyDict_GetItem(ssm.dicts[0], n.step);
     if (!ssm.integer(n.inner_dim, dim) || !ssm.integer(n.state_dim, nstate) ||
         !ssm.integer(n.delta_rank, rank) || !ssm.integer(n.conv_kernel, width))
       return false;
@@ -248,7 +248,7 @@ py::object block_step(const py::object& block, const py::object& xo, const py::t
   Layer l;
   if (!s.open(xo.ptr(), 1, rows ? 64 : 8) || !l.open(s, block.ptr(), Classes(classes)))
     return py::none();
-  if (s.batch > 8 && !l.norm_plain) return py::none();
+  if (s.batch > 8 && !l.calls_plain) return py::none();
   const at::Tensor& x = *s.x;
   c10::hip::HIPGuard guard(x.get_device());
   void* const st = stream_of(x);

@@ -180,3 +180,32 @@ def test_norm_with_a_forward_of_its_own(cuda):
 
     check(m, x, on_the_object)
     check(m, x, on_all_modules)
+
+
+def test_mixer_with_a_step_of_its_own(cuda):
+    """Past 8 rows a layer's step calls the mixer's step where a subclass or the
+    object has one."""
+    from ssm_mamba_amd.causal_lm import Mamba
+
+    class Own(Mamba):
+        def step(self, x):
+            return super().step(x) + 1.0
+
+    m = _model(cuda, torch.float32, 16)
+    x = torch.randn(16, 64, device=cuda)
+    ssm = m.layers[0].ssm
+
+    def run():
+        _caches(m, 16, torch.float32)
+        return m.layers[0].step(x)
+
+    with torch.no_grad():
+        want = run() + 1.0
+        ssm.__class__ = Own
+        got = [run()]
+        ssm.__class__ = Mamba
+        ssm.step = lambda v, f=ssm.step: f(v) + 1.0
+        got.append(run())
+        assert _native(m, x) is None
+    for a in got:
+        assert float((a - want).norm() / want.norm()) <= 2.0 ** -18

@@ -77,7 +77,8 @@ class NormInProjFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, norm_weight, w_in, eps, copy):
-        h, h_tm, rstd, xr = _lay.norm_tc(x, norm_weight, eps, token_major=True, copy=copy)
+        h, h_tm, rstd, xr = _lay.norm_tc(x, norm_weight, eps, copy=copy,
+                                         token_major=any(ctx.needs_input_grad))
         inner = w_in.shape[0] // 2
         xs, z = _bmm(w_in[:inner], h), _bmm(w_in[inner:], h)
         ctx.set_materialize_grads(False)
@@ -136,10 +137,14 @@ class SsmFn(torch.autograd.Function):
         A32, D32, b32 = _lay.scan_params(log_A, D, dt_bias)
         h0 = None if h_init is None else h_init.float().contiguous()
         lengths = ensure_contiguous(lengths)
-        y = torch.empty_like(xc)
+        # (no gradient wanted, as in a frozen layer: no states and no ungated output)
+        grad = any(ctx.needs_input_grad)
+        y = torch.empty_like(xc) if grad else None
         out, h = selective_scan.forward(
             xc, A32, params[:, rank:rank + nstate], params[:, rank + nstate:], D32, delta, b32, h0,
-            lengths, side, z=z, out_ungated=y)
+            lengths, side, z=z, save_chunks=grad, out_ungated=y)
+        if not grad:
+            return out, h
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(xc, z, w_x, w_dt, log_A, D, dt_bias, h_init, lengths, params, delta, y,
                               h, A32, D32, b32)

@@ -288,3 +288,25 @@ def test_wrapped_mixer_is_called(cuda):
         got = blk(x, use_cache=True)[0]
         step = blk.step(x[:, -1].contiguous())
     assert float((got - want).norm() / want.norm()) <= 2.0 ** -18 and step.shape == (12, 64)
+
+
+def test_frozen_layer_saves_nothing(cuda):
+    """With gradients enabled and none wanted, a layer's scan saves no states
+    (seqlen / 16 of them) and the results are the same."""
+    blk = _block(torch.float32, 64, False, seed=17)
+    x = torch.randn(2, 4096, 64, generator=torch.Generator().manual_seed(18)).to(cuda)
+    peak = []
+    for wanted in (True, False):
+        blk.requires_grad_(wanted)
+        out = [t.detach().clone() for t in blk(x, use_cache=True)]
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        base = torch.cuda.memory_allocated()
+        res = blk(x)
+        peak.append((out, torch.cuda.max_memory_allocated() - base))
+        assert res[0].requires_grad == wanted
+        del res
+    (a, most), (b, least) = peak
+    assert all(float((u - v).norm() / v.norm()) <= 2.0 ** -20 for u, v in zip(a, b))
+    # the states, the ungated output and the token-major norm
+    assert most - least >= 2 * 256 * 16 * 128 * 4 // 2

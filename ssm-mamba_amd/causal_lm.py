@@ -32,6 +32,7 @@ sequences (``models/causal_lm.py:98-133``), including its EOS handling.
 from __future__ import annotations
 
 import math
+from contextlib import nullcontext
 from dataclasses import dataclass
 from typing import Literal, Optional
 
@@ -51,20 +52,32 @@ _DTYPES = {torch.float32: _N.SSM_F32, torch.bfloat16: _N.SSM_BF16}
 __all__ = ["RMSNorm", "Mamba", "Block", "CausalLMConfig", "CausalLM", "GreedyDecoder"]
 
 
-def _proj_cm(weight: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor] = None):
-    """``weight @ x`` for channel-major x (batch, in, L) -> (batch, out, L):
+def _proj_cm(weight: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor] = None,
+             residual: Optional[torch.Tensor] = None):
+    """``weight @ x`` for channel-major x (batch, in, L) -> (batch, out, L), plus
+    bias (out,) or, in its place, residual (of the result's shape):
     one strided-batched GEMM with the weight broadcast over the batch (batch
     stride 0), contiguous result.  (``torch.matmul`` would fold a weight that
     requires grad through transposed copies of x and of the result.)  A view
     whose per-batch (in, L) matrices are contiguous, such as a channel slice
     of a larger activation, is passed as it is: the GEMM takes its batch
-    stride."""
+    stride.  With autograd in bfloat16 the product is one of its own
+    (``layer_train.ProductFn`` says why)."""
     if not (x.stride(2) == 1 and x.stride(1) == x.shape[2]):
         x = x.contiguous()
+    addend = residual if bias is None else bias[None, :, None]
+    if torch.is_grad_enabled():
+        cast = x.is_cuda and torch.is_autocast_enabled()
+        if cast:  # autocast's own casts, made here: it does not reach into a function
+            dtype = torch.get_autocast_dtype("cuda")
+            weight, x, addend = (None if t is None else t.to(dtype) for t in (weight, x, addend))
+        if x.dtype == weight.dtype == torch.bfloat16:
+            with torch.autocast("cuda", enabled=False) if cast else nullcontext():
+                return _lt.ProductFn.apply(weight, x, addend)
     w = weight.expand(x.shape[0], weight.shape[0], weight.shape[1])
-    if bias is None:
+    if addend is None:
         return torch.bmm(w, x)
-    return torch.baddbmm(bias[None, :, None].expand(x.shape[0], weight.shape[0], x.shape[2]), w, x)
+    return torch.baddbmm(addend.expand(x.shape[0], weight.shape[0], x.shape[2]), w, x)
 
 
 def _channel_major(x: torch.Tensor) -> torch.Tensor:
@@ -318,11 +331,11 @@ class Mamba(nn.Module):
         the last SSM state."""
         y, last = self._mix_cm(x, ssm_hiddens, lengths, use_cache)
         if residual is not None and self.out_proj.bias is None:
-            w = self.out_proj.weight.expand(y.shape[0], *self.out_proj.weight.shape)
+            w = self.out_proj.weight
             if residual_inplace:
-                out = residual.baddbmm_(w, y)       # the stream is updated in place
+                out = residual.baddbmm_(w.expand(y.shape[0], *w.shape), y)  # the stream itself
             else:
-                out = torch.baddbmm(residual, w, y)
+                out = _proj_cm(w, y, residual=residual)
         else:
             out = _proj_cm(self.out_proj.weight, y, self.out_proj.bias)
             if residual is not None:

@@ -2,6 +2,8 @@
 layouts and its backward against float64, the transposition and the batch sum
 bit for bit, and a Block's outputs and gradients against the op-by-op
 path (which tests/test_gpu_lm.py checks against float64)."""
+import copy
+
 import pytest
 import torch
 
@@ -310,3 +312,29 @@ def test_frozen_layer_saves_nothing(cuda):
     assert all(float((u - v).norm() / v.norm()) <= 2.0 ** -20 for u, v in zip(a, b))
     # the states, the ungated output and the token-major norm
     assert most - least >= 2 * 256 * 16 * 128 * 4 // 2
+
+
+@pytest.mark.parametrize("autocast", [False, True])
+@pytest.mark.parametrize("batch", [1, 2])
+def test_bf16_layer_op_by_op_makes_no_transposed_products(cuda, batch, autocast):
+    """A layer with projection biases, or under autocast, trains op by op: no
+    bfloat16 batched product with a transposed right operand either way, and
+    gradients against the float32 layer's (which float64 checks elsewhere)."""
+    from ssm_mamba_amd.causal_lm import Block
+    from tests.test_layer_dispatch import _NoTransposedRight
+    torch.manual_seed(19)
+    blk = Block(model_dim=64, dropout_rate=0.0, bias=True).cuda()
+    x = torch.randn(batch, 40, 64, device=cuda)
+    low = blk if autocast else copy.deepcopy(blk).bfloat16()
+    xl = x if autocast else x.bfloat16()
+    assert not low._fused(xl)
+    with _NoTransposedRight() as seen:
+        with torch.autocast("cuda", torch.bfloat16, enabled=autocast):
+            out = low(xl)[0]
+        got = torch.autograd.grad(out.float().pow(2).sum(), list(low.parameters()))
+    assert seen.count
+    want = torch.autograd.grad(blk(x)[0].pow(2).sum(), list(blk.parameters()))
+    for (n, p), a, b in zip(low.named_parameters(), got, want):
+        assert a.dtype == p.dtype
+        # a chain of a dozen bfloat16 roundings, each of 2^-9 relative
+        assert float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -5, n

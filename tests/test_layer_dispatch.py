@@ -4,6 +4,7 @@ from types import SimpleNamespace
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from ssm_mamba_amd import layer_train as LT
 
@@ -183,3 +184,47 @@ def test_plain_module_calls(change):
             if handle is not None:
                 handle.remove()
     assert DEC.plain(RMSNorm(8), RMSNorm)
+
+
+class _NoTransposedRight(TorchDispatchMode):
+    """Counts batched products and refuses a bfloat16 one whose right operand
+    is a transposed view."""
+    count = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        name = func.overloadpacket.__name__.rstrip("_")
+        if name in ("bmm", "baddbmm"):
+            right = args[1 if name == "bmm" else 2]
+            self.count += 1
+            bad = right.shape[2] > 1 and right.stride(2) != 1
+            assert not (bad and right.dtype == torch.bfloat16), (name, right.shape, right.stride())
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("add", [None, "bias", "residual"])
+def test_products_of_a_bf16_layer_op_by_op(batch, add):
+    """Forward, backward and the backward of create_graph make no bfloat16
+    batched product with a transposed right operand; values against float64,
+    within one rounding of each batch row's product and of their sum."""
+    from ssm_mamba_amd.causal_lm import _proj_cm
+    g = torch.Generator().manual_seed(batch)
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16().requires_grad_(True)
+    w, xs, dout = r(6, 8), r(batch, 12, 7), r(batch, 6, 7).detach()
+    a = {None: None, "bias": r(6), "residual": r(batch, 6, 7)}[add]
+    live = [t for t in (w, xs, a) if t is not None]
+    kw = {} if a is None else {add: a}
+    with _NoTransposedRight() as seen:
+        for graph in (False, True):
+            out = _proj_cm(w, xs[:, :8], **kw)
+            got = torch.autograd.grad(out, live, dout, create_graph=graph)
+            if graph:
+                torch.autograd.grad(sum(t.float().pow(2).sum() for t in got), live, allow_unused=True)
+    assert seen.count
+    w64, x64, a64 = (None if t is None else t.detach().double().requires_grad_(True) for t in (w, xs, a))
+    ref = w64 @ x64[:, :8]
+    if a64 is not None:
+        ref = ref + (a64[None, :, None] if add == "bias" else a64)
+    want = torch.autograd.grad(ref, [t for t in (w64, x64, a64) if t is not None], dout.double())
+    for p, q in ((out, ref), *zip(got, want)):
+        assert float((p.double() - q).detach().norm()) <= 2.0 ** -7 * float(q.detach().norm())

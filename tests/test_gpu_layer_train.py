@@ -1,11 +1,14 @@
 """The fused layer of a training step and its kernels: the norm between the
 layouts and its backward against float64, the transposition and the batch sum
-bit for bit, and a Block's outputs and gradients against the op-by-op
-path (which tests/test_gpu_lm.py checks against float64)."""
+bit for bit, and a layer's and a model's outputs and gradients against float64
+and, over more forms of the call, against the op-by-op path."""
 import copy
 
 import pytest
 import torch
+
+from helpers import lm_state64
+from oracle import lm_ref as LR
 
 pytestmark = pytest.mark.gpu
 
@@ -69,10 +72,10 @@ def test_transpose_and_batch_sum(cuda, dtype, batch, rows, cols):
     assert torch.equal(LY.batch_sum(x, transpose=True), ref.t())
 
 
-def _block(dtype, model_dim, conv_bias, seed):
+def _block(dtype, model_dim, conv_bias, seed, nstate=16):
     from ssm_mamba_amd.causal_lm import Block
     torch.manual_seed(seed)
-    blk = Block(model_dim=model_dim, dropout_rate=0.0, conv_bias=conv_bias)
+    blk = Block(model_dim=model_dim, dropout_rate=0.0, conv_bias=conv_bias, state_dim=nstate)
     with torch.no_grad():
         blk.norm.weight.normal_(0.0, 0.3)
         blk.ssm.D.normal_(1.0, 0.1)
@@ -338,3 +341,130 @@ def test_bf16_layer_op_by_op_makes_no_transposed_products(cuda, batch, autocast)
         assert a.dtype == p.dtype
         # a chain of a dozen bfloat16 roundings, each of 2^-9 relative
         assert float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -5, n
+
+
+def _ref64(p, x, nstate, h0, lengths, use_cache, scale):
+    """The layer in float64: (out, last state, conv window)."""
+    y, last, ctx = LR.mamba_forward(p, LR.rms_norm(x, p["norm.weight"]), nstate,
+                                    p["ssm.delta_proj.weight"].shape[1], h0=h0, lengths=lengths,
+                                    use_cache=use_cache)
+    return x + (y if scale is None else y * scale), last, ctx
+
+
+def _with_mask(blk, scale, dev):
+    """Dropout with a given mask in place of a drawn one."""
+    if scale is not None:
+        blk.dropout.p = 0.25
+        blk.dropout.forward = lambda v, s=scale.to(dev): v * s.to(v.dtype)
+
+
+def _mask(shape, g):
+    return (torch.rand(shape, generator=g) >= 0.25).double() / 0.75
+
+
+# one and several batch rows, odd and whole rows; 8 to 64 states; without a first
+# state the last state's gradient still counts; the caches of a prefill; dropout
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batch,seqlen,model_dim,nstate,h0,pads,use_cache,drop", [
+    (2, 37, 64, 16, False, True, True, False),
+    (1, 100, 72, 32, True, False, False, True),
+    (3, 64, 40, 64, False, False, True, True),
+    (2, 130, 64, 8, True, True, False, True),
+])
+def test_layer_against_float64(cuda, dtype, batch, seqlen, model_dim, nstate, h0, pads, use_cache, drop):
+    """Outputs, caches and every gradient of the fused layer.  float32: norm-wise
+    2^-16, the float32 sums over up to 128 channels and 130 steps and their
+    exponentials.  bfloat16: no further from float64 than the op-by-op layer by
+    more than half (they round as many tensors, at other places) and one
+    rounding."""
+    blk = _block(dtype, model_dim, True, seed=nstate, nstate=nstate)
+    g = torch.Generator().manual_seed(seqlen)
+    r = lambda *s: torch.randn(*s, generator=g)
+    x, dout, dlast = r(batch, seqlen, model_dim).to(dtype), r(batch, seqlen, model_dim).to(dtype), \
+        r(batch, 2 * model_dim, nstate)
+    first = 0.1 * r(batch, 2 * model_dim, nstate) if h0 else None
+    lengths = torch.randint(5, seqlen + 1, (batch,), generator=g) if pads else None
+    scale = _mask((batch, seqlen, model_dim), g) if drop else None
+    _with_mask(blk, scale, cuda)
+    names = ["x"] + (["h0"] if h0 else []) + [n for n, _ in blk.named_parameters()]
+
+    def run(fused):
+        from ssm_mamba_amd import layer_train as LT
+        keep = LT.supported
+        s = blk.dropout.forward if drop else None
+        if not fused:
+            LT.supported = lambda *a: False
+            if drop:  # the op-by-op layer drops channel-major
+                blk.dropout.forward = lambda v: s(v.transpose(1, 2)).transpose(1, 2)
+        try:
+            leaves = [t.detach().to(cuda).requires_grad_(True) for t in (x, first) if t is not None]
+            xg, hg = leaves[0], leaves[1] if h0 else None
+            assert blk._fused(xg) == fused
+            out, last = blk(xg, lengths=None if lengths is None else lengths.to(cuda),
+                            ssm_hiddens=hg, use_cache=use_cache)
+            grads = torch.autograd.grad([out, last], [*leaves, *blk.parameters()],
+                                        [dout.to(cuda), dlast.to(cuda)])
+        finally:
+            LT.supported = keep
+            if drop:
+                blk.dropout.forward = s
+        res = dict(zip(names, grads), out=out, last=last)
+        if use_cache:
+            res["window"] = blk.ssm._conv_context
+            assert torch.equal(blk.ssm._ssm_hiddens, last)
+        return res
+
+    p = {n: t.detach().double().cpu().requires_grad_(True) for n, t in blk.named_parameters()}
+    x64 = x.double().requires_grad_(True)
+    f64 = first.double().requires_grad_(True) if h0 else None
+    out, last, ctx = _ref64(p, x64, nstate, f64, lengths, use_cache, scale)
+    grads = torch.autograd.grad([out, last], [t for t in (x64, f64) if t is not None] + list(p.values()),
+                                [dout.double(), dlast.double()])
+    want = dict(zip(names, grads), out=out.detach(), last=last.detach())
+    if use_cache:
+        want["window"] = ctx.detach()
+    err = lambda got: {k: float((got[k].detach().double().cpu() - w).norm() / w.norm())
+                       for k, w in want.items()}
+    got = err(run(True))
+    if dtype == torch.float32:
+        assert max(got.values()) <= 2.0 ** -16, got
+    else:
+        ops = err(run(False))
+        for k in got:
+            assert got[k] <= 1.5 * ops[k] + 2.0 ** -9, (k, got[k], ops[k])
+
+
+@pytest.mark.parametrize("pads", [False, True])
+def test_model_training_step_against_float64(cuda, pads):
+    """CausalLM.forward with gradients in its default form (no projection
+    biases, dropout on): logits and every parameter's gradient."""
+    from ssm_mamba_amd.causal_lm import CausalLM, CausalLMConfig
+    torch.manual_seed(21)
+    m = CausalLM(CausalLMConfig(vocab_size=31, model_dim=64, num_layers=3)).cuda().train()
+    with torch.no_grad():
+        for n, t in m.named_parameters():
+            if n.endswith("norm.weight"):
+                t.normal_(0.0, 0.3)
+    g = torch.Generator().manual_seed(22)
+    ids = torch.randint(3, 31, (2, 45), generator=g)
+    lengths = torch.tensor([45, 30]) if pads else None
+    r = torch.randn(2, 45, 31, generator=g)
+    masks = [_mask((2, 45, 64), g) for _ in m.layers]
+    for layer, s in zip(m.layers, masks):
+        _with_mask(layer, s, cuda)
+        assert layer._fused(m.embedding(ids.to(cuda)))
+    sd = lm_state64(m)
+    for v in sd.values():
+        v.requires_grad_(True)
+    x = sd["embedding.weight"][ids]
+    for i, s in enumerate(masks):
+        p = LR.layer_params(sd, i)
+        x = _ref64(p, x, 16, None, lengths, False, s)[0]
+    want = LR.rms_norm(x, sd["norm.weight"]) @ sd["lm_head.weight"].t()
+    names = [n for n, _ in m.named_parameters()]
+    grads = torch.autograd.grad(want, [sd[n] for n in names], r.double())
+    got = m(ids.to(cuda), None if lengths is None else lengths.to(cuda))
+    mine = torch.autograd.grad(got, list(m.parameters()), r.to(cuda))
+    for n, a, b in zip(["logits", *names], [got, *mine], [want, *grads]):
+        rel = float((a.detach().double().cpu() - b.detach()).norm() / b.detach().norm())
+        assert rel <= 2.0 ** -16, (n, rel)

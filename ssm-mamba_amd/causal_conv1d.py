@@ -111,7 +111,8 @@ def causal_conv1d_fn(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     (channels,); ``activation`` is "silu" or None.  ``window`` (batch,
     channels, width - 1), if given, receives the decode cache of a prefill:
     the width - 1 inputs ending at position lengths[b] - 1 (seq_len - 1
-    without lengths), zero before the row start (``modules/mamba.py:113-135``)."""
+    without lengths), zero before the row start (``modules/mamba.py:113-135``).
+    Differentiable once, as ``selective_scan_fn`` is."""
     if activation not in (None, "silu"):
         raise RuntimeError("activation must be 'silu' or None")
     return CausalConv1dFn.apply(x, weight, bias, activation == "silu", lengths, window)

@@ -82,7 +82,7 @@ def _proj_cm(weight: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor]
 
 def _channel_major(x: torch.Tensor) -> torch.Tensor:
     """x.transpose(1, 2).contiguous() (its own inverse: also channel-major to
-    token-major); without autograd on the GPU one tiled kernel (6.8 us for 16.8
+    token-major); without autograd on the GPU one tiled kernel (5.4 us for 16.8
     MB, against 42 us for torch's strided copy)."""
     if torch.is_grad_enabled() or x.dim() != 3:
         return x.transpose(1, 2).contiguous()

@@ -17,7 +17,7 @@
 // Measured at d_model 1024, batch 32, bf16: in-projection 7.8 us, x- and
 // out-projection 7.2 each, state update 5.9, 28 us in all (43 at batch 64);
 // the same step op by op (29 launches) took 99 us of kernels and 274 us a
-// call, host-bound, against 61 now.
+// call, host-bound, against 30 now.
 //
 // Split: a workgroup owns kMT * 16 weight rows and every batch row; its waves
 // split K in groups of kU MFMA steps (whole 256-byte pieces of a weight row),

@@ -14,7 +14,7 @@
 // (4, 2048, 1024) in bf16 (16.8 MB a tensor, 3.2 us at the copy rate): the norm
 // 9.5 us (11.0 with a copy of x for the layer's sum, in place of a device copy
 // of 6.5; 13.6 with the token-major result too), its backward 19 + 4 us, a
-// transposition 6.8 us, a batch sum of four 2048 x 1024 matrices 4 us.  They
+// transposition 5.4 to 5.7 us, a batch sum of four 2048 x 1024 matrices 4 us.  They
 // replace strided copies of 42 us on either side of a layer and, in a training
 // step, about 25 elementwise and reduction kernels of the norm (290 us).
 //

@@ -676,7 +676,8 @@ __global__ __launch_bounds__(kThreads) void scan_bwd_kernel(
 // Role-split backward for up to 64 states, the counterpart of the forward's
 // role split.  A workgroup of 12 waves covers one batch row b x 64 channels
 // and walks its segment's 16-step tiles from the end:
-//   consumer waves 0..7   lane = channel, wave w = states 2w and 2w+1: take
+//   consumer waves 0..7   lane = channel, wave w = states 2w and 2w+1 (and
+//                         16 g + 2w, + 1 for g < kSG past 16 states): take
 //                         the state the forward saved before the tile,
 //                         recompute the tile's 16 states and decays, run the
 //                         reverse recurrence, leave the per-position sums
@@ -690,7 +691,8 @@ __global__ __launch_bounds__(kThreads) void scan_bwd_kernel(
 //                         slices of each sum added in a fixed order, du,
 //                         ddelta, the dD and dbias accumulators).
 // One barrier per tile; the staging buffers and the slices alternate between
-// two LDS buffers by tile parity (159,744 bytes in all).  The arithmetic and
+// two LDS buffers by tile parity (159,744 bytes in all; past 16 states see kSG
+// below).  The arithmetic and
 // its order are those of scan_bwd_kernel, and the outputs agree bit for bit
 // with that kernel's except dbias (the compiler contracts a multiply and an
 // add of its accumulator differently), dB/dC (the channel sums run in another
@@ -721,9 +723,12 @@ struct BwsRows {  // one tile's raw loads of a producer lane, as loaded
 // consumers run the recompute of their first pair meanwhile.  A pair's A,
 // adjoint carry and dA then live in LDS between its turns and the pairs run
 // in a loop: held in registers over unrolled pairs, four of them spilled 155
-// registers at the 168 three waves a SIMD allow.  Measured against
-// scan_bwd_kernel at (4, 1024, 1000) x 64 states, bf16: 272 -> 197 us, its
-// segment summaries 102 -> 45 us; at (8, 2048, 512) x 32 states 206 -> 193 us.
+// registers at the 168 three waves a SIMD allow (2 or 3 as it is).  Measured
+// against scan_bwd_kernel at (4, 1024, 1000) x 64 states, bf16: 272 -> 184 to 197
+// us, its segment summaries 102 -> 45 us; at (8, 2048, 512) x 32 states 206 ->
+// 193 us.  At 64 states its VALU instructions take 140 us of the 184 at full
+// issue; LDS is active a quarter of the time, with 0.3% bank conflicts, and
+// waves wait 43% of theirs (35% at 16 states, with one barrier per tile).
 template <typename T, int kSG, bool kHasZ, bool kAligned>
 __global__ __launch_bounds__(kWsThreads) void scan_bwd_ws_kernel(
     const ScanDims p, const T* __restrict__ u, const T* __restrict__ dl,
@@ -1499,9 +1504,10 @@ __global__ __launch_bounds__(kThreads) void scan_bwd_segsum_kernel(
 // steps (blockIdx.z = k: global sub-segment k + sub_k, so the sub-segments
 // of segments 1 .. nseg-1), with the forward's role split so that staging
 // overlaps the recurrence:
-//   consumer waves 0..7   lane = channel, wave w = states 2w and 2w+1: from
-//                         gamma = 0 after the sub-segment's last step, down
-//                         to its first, G_t = gamma_t + dout_t C_t and
+//   consumer waves 0..7   lane = channel, wave w = states 2w and 2w+1 (and
+//                         16 g + 2w, + 1 for g < kSG): from gamma = 0 after
+//                         the sub-segment's last step, down to its first,
+//                         G_t = gamma_t + dout_t C_t and
 //                         gamma_{t-1} = a_t G_t, reading delta, the effective
 //                         dout and (C_2w, C_2w+1) from LDS;
 //   producer waves 8..11  lane -> (channel row, 4-step column): stage the

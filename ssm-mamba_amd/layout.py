@@ -90,8 +90,8 @@ def transposed(x: torch.Tensor) -> torch.Tensor:
 
 def batch_sum(x: torch.Tensor, transpose: bool = False,
               out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x.sum(0), or its transpose, for contiguous x (batch, rows, cols), added
-    in float32 and rounded once; into ``out`` (contiguous) when given."""
+    """x.sum(0), or its transpose, for contiguous x (batch, rows, cols), its
+    elements added in float32 and the sum rounded once; into ``out`` (contiguous) when given."""
     batch, rows, cols = x.shape
     x = x.contiguous()
     if out is None:

@@ -118,7 +118,9 @@ def selective_scan_fn(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: 
                       h_init: Optional[torch.Tensor] = None, length: Optional[torch.Tensor] = None,
                       padding_side: str = "left"):
     """Functional selective scan: out = (D*u + sum_n C*h) * silu(z), returned
-    alone or with the last state (batch, channels, state_dim)."""
+    alone or with the last state (batch, channels, state_dim).  Differentiable
+    once: with create_graph its gradients are constants to the next
+    differentiation."""
     out, last = _SelectiveScanExtFn.apply(u, delta, A, B, C, D, z, delta_bias, h_init, length,
                                           delta_softplus, padding_side)
     return (out, last) if return_last_state else out

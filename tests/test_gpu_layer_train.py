@@ -140,8 +140,11 @@ def test_block_gradients_of_a_graph(cuda, dtype):
 
 
 def test_block_second_derivatives_and_frozen_parameters(cuda):
-    """create_graph differentiates the op-by-op form; parameters and inputs
-    that need no gradient get none."""
+    """create_graph differentiates the op-by-op form: the second derivatives of
+    the op-by-op layer, whose terms through the scan's and the conv's own
+    gradients are left out on both paths (float64 checks of the norm's and the
+    products' second derivatives: tests/test_layer_dispatch.py).  Parameters and
+    inputs that need no gradient get none."""
     from ssm_mamba_amd import layer_train as LT
     blk = _block(torch.float32, 64, False, seed=3)
     x0 = torch.randn(2, 40, 64, generator=torch.Generator().manual_seed(4)).to(cuda)

@@ -125,8 +125,9 @@ def gemv_supported(weight: torch.Tensor, x: torch.Tensor, *others) -> bool:
 def rows_supported(weight: torch.Tensor, x: torch.Tensor, *others) -> bool:
     """Whether ``rows_linear`` takes the product: the GEMV kernels' conditions,
     for the batches past theirs (autocast keeps the op-by-op path and its
-    casts)."""
-    return not torch.is_autocast_enabled() and _linear_supported(MAX_BATCH + 1, MAX_ROWS, weight, x, *others)
+    casts, tensors with semantics of their own torch's operators)."""
+    return (not torch.is_autocast_enabled() and all(plain_tensor(t) for t in (weight, *others))
+            and _linear_supported(MAX_BATCH + 1, MAX_ROWS, weight, x, *others))
 
 
 def _linear_supported(lo: int, hi: int, weight: torch.Tensor, x: torch.Tensor, *others) -> bool:
@@ -147,6 +148,12 @@ def _linear_supported(lo: int, hi: int, weight: torch.Tensor, x: torch.Tensor, *
 def block_step_supported(ssm, x: torch.Tensor, norm_weight: Optional[torch.Tensor]) -> bool:
     """Whether the fused kernels can run Mamba ``ssm`` on the token batch x."""
     return _step_supported(gemv_supported, ssm, x, norm_weight)
+
+
+def plain_tensor(t: Optional[torch.Tensor]) -> bool:
+    """Whether ``t`` (None: yes) is a tensor and no subclass, whose operators
+    (a quantized or sharded weight's) its address says nothing of."""
+    return t is None or type(t) in (torch.nn.Parameter, torch.Tensor)
 
 
 def own(obj, cls, name: str) -> bool:

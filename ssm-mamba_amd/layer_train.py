@@ -26,6 +26,7 @@ from typing import Optional
 
 import torch
 
+from . import decode as _dec
 from . import layout as _lay
 from . import selective_scan
 from .ops import selective_scan_fn
@@ -289,10 +290,10 @@ def out_proj(y: torch.Tensor, w_out: torch.Tensor, residual: Optional[torch.Tens
 
 def supported(block, x: torch.Tensor) -> bool:
     """Whether token-major x through ``block`` takes the fused layer: float32 or
-    bfloat16 on the GPU with every projection weight in x's dtype, no
-    projection biases, a width the norm kernel takes, no autocast."""
+    bfloat16 on the GPU with every projection weight a plain tensor in x's
+    dtype, no projection biases, a width the norm kernel takes, no autocast."""
     w = block.norm.weight
-    if torch.is_autocast_enabled() or not _lay.norm_tc_supported(x, w):
+    if torch.is_autocast_enabled() or not _dec.plain_tensor(w) or not _lay.norm_tc_supported(x, w):
         return False
     # read where nn.Module keeps them: a weight that is not a plain parameter
     # (parametrized, computed by a hook) is not there and takes the other path
@@ -300,7 +301,7 @@ def supported(block, x: torch.Tensor) -> bool:
     for name in _PROJECTIONS:
         params = getattr(mods.get(name), "_parameters", {})
         p = params.get("weight")
-        if p is None or p.dtype != dtype or p.device != dev:
+        if p is None or p.dtype != dtype or p.device != dev or not _dec.plain_tensor(p):
             return False
         if name in _NO_BIAS and params.get("bias") is not None:
             return False

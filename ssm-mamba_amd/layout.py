@@ -10,6 +10,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _native as N
+from .decode import plain_tensor
 
 DTYPES = {torch.float32: N.SSM_F32, torch.bfloat16: N.SSM_BF16}
 _MAX_CHANNELS = {torch.float32: 1024, torch.bfloat16: 2048}
@@ -110,7 +111,7 @@ def _one_type(log_A: torch.Tensor, *others: Optional[torch.Tensor]) -> bool:
     """Whether the stored parameters (dim, nstate), (dim,), (dim,) are what the
     scan_params kernels take."""
     return (log_A.is_cuda and log_A.dtype in DTYPES and log_A.dim() == 2 and log_A.numel() > 0
-            and log_A.is_contiguous()
+            and log_A.is_contiguous() and all(map(plain_tensor, (log_A, *others)))
             and all(t is None or (t.dtype == log_A.dtype and t.device == log_A.device
                                   and t.is_contiguous() and tuple(t.shape) == log_A.shape[:1])
                     for t in others))

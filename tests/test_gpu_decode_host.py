@@ -209,3 +209,19 @@ def test_mixer_with_a_step_of_its_own(cuda):
         assert _native(m, x) is None
     for a in got:
         assert float((a - want).norm() / want.norm()) <= 2.0 ** -18
+
+
+def test_weight_with_operators_of_its_own(cuda):
+    """Past 8 rows a projection or head whose weight is a tensor subclass without
+    memory of its own takes torch's operators."""
+    from tests.test_layer_dispatch import _wrap_weight
+    m = _model(cuda, torch.float32, 16, tie_embeddings=False)
+    x = torch.randn(16, 64, device=cuda)
+    with torch.no_grad():
+        want = [m.layers[0].step(x), m._head(x), m.layers[0](x[:, None].expand(16, 40, 64))[0]]
+        _caches(m, 16, torch.float32)
+        _wrap_weight(m.lm_head)
+        _wrap_weight(m.layers[0].ssm.out_proj)
+        got = [m.layers[0].step(x), m._head(x), m.layers[0](x[:, None].expand(16, 40, 64))[0]]
+    for a, b in zip(got, want):
+        assert float((a - b).norm() / b.norm()) <= 2.0 ** -18

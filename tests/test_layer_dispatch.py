@@ -5,6 +5,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
+from torch.utils._pytree import tree_map
 
 from ssm_mamba_amd import layer_train as LT
 
@@ -228,3 +229,34 @@ def test_products_of_a_bf16_layer_op_by_op(batch, add):
     want = torch.autograd.grad(ref, [t for t in (w64, x64, a64) if t is not None], dout.double())
     for p, q in ((out, ref), *zip(got, want)):
         assert float((p.double() - q).detach().norm()) <= 2.0 ** -7 * float(q.detach().norm())
+
+
+class _Wrapped(torch.Tensor):
+    """A weight that holds another tensor and no memory of its own, as a
+    quantized or sharded one does."""
+
+    @staticmethod
+    def __new__(cls, held):
+        return torch.Tensor._make_wrapper_subclass(cls, held.shape, dtype=held.dtype, device=held.device)
+
+    def __init__(self, held):
+        self.held = held
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        held = lambda t: t.held if isinstance(t, _Wrapped) else t
+        if func is torch.ops.aten.detach.default:
+            return _Wrapped(args[0].held)
+        return func(*tree_map(held, args), **tree_map(held, kwargs or {}))
+
+
+def _wrap_weight(module):
+    module.weight = torch.nn.Parameter(_Wrapped(module.weight.detach()), requires_grad=False)
+
+
+@pytest.mark.parametrize("part", ["norm", "ssm.out_proj", "ssm.ssm_param_proj", "ssm.conv"])
+def test_weights_with_operators_of_their_own(monkeypatch, part):
+    blk, x = _block(monkeypatch)
+    assert blk._fused(x)
+    _wrap_weight(blk.get_submodule(part))
+    assert not blk._fused(x)
